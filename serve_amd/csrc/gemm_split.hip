@@ -1,10 +1,13 @@
 // C[M, N] = A[M, K] * W[N, K]^T for five and more rows of float32 (the 32-bit path) on the bf16 matrix
 // cores, with no operand rounded: every float is the sum of three bf16 numbers,
-//     x = x0 + x1 + x2,   x0 = x cut to its upper 16 bits, x1 = x - x0 cut likewise, x2 = x - x0 - x1,
-// exactly (24 significant bits are three times eight; both differences are exact, so x2 has no bits below its upper
-// 16).  A product of two floats is then nine products of bf16 numbers, each exact in float32, of which the six
-// x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0 are taken: what is left out is below 2^-23 of the product at worst and
-// 2^-26 of it on the average, less than the rounding of one float32 addition.  Sums are float32, in two levels.
+//     x = x0 + x1 + x2,   x0 = x rounded to the nearest bf16 number, x1 = x - x0 rounded likewise, x2 = x - x0 - x1,
+// exactly (both differences are exact; with x in [1, 2) x1 is at most 2^-8, x2 at most 2^-17 and a multiple of 2^-23, six
+// bits).  A product of two floats is then nine products of bf16 numbers, each exact in float32, of which the six
+// x0 w0, x0 w1, x1 w0, x1 w1, x0 w2, x2 w0 are taken: x1 w2 + x2 w1 + x2 w2 is what is left out, at most 2^-24 of the
+// product (at 1.0038986 squared; no more than one rounding) and 2^-28 of it on the average of the mantissas, of either sign.
+// (Planes cut instead of rounded all have the number's sign and are twice and four times as large: 2^-21 at worst, 2^-24.6 on
+// the average, always towards zero.)  Sums are float32, in two levels.  What remains with a sign: the matrix cores cut an
+// addend two bits behind the last place of the sum, 2^-26 of a stage's sum where all six products go to one accumulator.
 //
 // Why: the float32 matrix instruction runs at a sixteenth of the bf16 rate; six bf16 instructions for the same terms
 // are 2.7 times as fast where both are at their peak.
@@ -23,7 +26,11 @@ union Frag8 {
 
 #define SP_BN 128                  // rows of W a workgroup owns
 #define SP_WPITCH (SP_BN + 8)      // 16-byte units between the two halves of a stage's columns of W in LDS
-#define SP_FLUSH 16                // stages of 16 columns summed in one accumulator before they join the total
+// Stages of 16 columns summed in one accumulator before they join the total, out of `n`.  Long inner sizes take more, which
+// balances the roundings of the two sums: distance to 64 bits (rms) with 16 / 24 / 32 of them, operands of one sign, K 14336
+// 1.02e-7 / 0.90e-7 / 0.85e-7 of the result, of either sign 3.0e-7 / 3.4e-7 / 3.8e-7 (the float32 instruction: 0.95e-7, 4.2e-7).
+__device__ __forceinline__ int flush_after(int n) { return n >= 1280 ? 32 : n >= 640 ? 24 : 16; }
+#define SP_ROWS_FLUSH 32           // the same in the kernel of few rows, in stages of 64 or 128 columns
 
 typedef __attribute__((address_space(1))) const void* gptr_t;
 // All but the newest n of this wave's loads have landed and its LDS operations are done; then the workgroup's barrier
@@ -41,27 +48,27 @@ typedef __attribute__((address_space(1))) const void* gptr_t;
 #define SGB_DS_READ 0x100
 #define SGB_DS_WRITE 0x200
 
+// Two floats as bf16 numbers, rounded to the nearest (ties to even), side by side, and the first and second of such a pair.
+// (The instruction by name: where one of the pair is used again the compiler converts it once more.)
+__device__ __forceinline__ uint32_t round2(float lo, float hi) {
+  uint32_t u;
+  asm("v_cvt_pk_bf16_f32 %0, %1, %2" : "=v"(u) : "v"(lo), "v"(hi));
+  return u;
+}
+__device__ __forceinline__ float first_of(uint32_t u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float second_of(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
+
 // Eight floats into the three planes (eight bf16 numbers each, in order).
 __device__ __forceinline__ void split8(const f32x4_t& a, const f32x4_t& b, u32x4_t (&p)[3]) {
   const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-  uint32_t q[3][8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const uint32_t u0 = __float_as_uint(x[i]);
-    const float r1 = x[i] - __uint_as_float(u0 & 0xffff0000u);
-    const uint32_t u1 = __float_as_uint(r1);
-    const float r2 = r1 - __uint_as_float(u1 & 0xffff0000u);
-    q[0][i] = u0;
-    q[1][i] = u1;
-    q[2][i] = __float_as_uint(r2);
-  }
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    // (the upper halves of two words side by side)
-    p[k].x = __builtin_amdgcn_perm(q[k][1], q[k][0], 0x07060302u);
-    p[k].y = __builtin_amdgcn_perm(q[k][3], q[k][2], 0x07060302u);
-    p[k].z = __builtin_amdgcn_perm(q[k][5], q[k][4], 0x07060302u);
-    p[k].w = __builtin_amdgcn_perm(q[k][7], q[k][6], 0x07060302u);
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t u0 = round2(x[2 * i], x[2 * i + 1]);
+    const float r0 = x[2 * i] - first_of(u0), r1 = x[2 * i + 1] - second_of(u0);
+    const uint32_t u1 = round2(r0, r1);
+    p[0][i] = u0;
+    p[1][i] = u1;
+    p[2][i] = round2(r0 - first_of(u1), r1 - second_of(u1));
   }
 }
 
@@ -161,9 +168,10 @@ __device__ __forceinline__ void read_stage(Frag8 (&a)[TI][3], Frag8 (&w)[2][3], 
 //
 // What bounds it: the matrix cores (24 instructions of 32 cycles a wave and stage, beside 12 16-byte LDS reads and a split
 // of eight floats).  Measured, the float32 matrix instruction on 128 x 128 tiles / this kernel with split_rows_kernel, in
-// us: 1,050 rows, K 2048, 3,072 rows of W 192 / 112, 16,384 rows 736 / 413; K 8192, 2,048 rows of W 719 / 221 (five parts);
-// 2,048 rows, K 2048, 16,384 rows of W 1106 / 706 (195 TFLOP/s).  Distance to 64 bits (rms, operands of size one): K 2048
-// 3.7e-7 / 2.3e-7 of the result's size, K 8192 7.5e-7 / 5.0e-7, K 14336 1.0e-6 / 7.2e-7.
+// us: 1,050 rows, K 2048, 3,072 rows of W 192 / 110, 16,384 rows 736 / 418; K 8192, 2,048 rows of W 719 / 229 (five parts);
+// 2,048 rows, K 2048, 16,384 rows of W 1106 / 712 (193 TFLOP/s).  Distance to 64 bits (rms, of the result's size): normal
+// operands, K 2048 4.1e-7 / 2.5e-7, K 8192 4.1e-7 / 2.7e-7, K 14336 4.2e-7 / 3.4e-7; operands in 1 .. 2, 1.7e-7 / 0.8e-7,
+// 1.05e-7 / 0.92e-7 and 0.95e-7 / 0.90e-7; all operands the same number (60 pairs of them), K 2048 4.1e-6 / 0.5e-6.
 template <int TI>
 __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* __restrict__ P, const float* __restrict__ A,
                                                                 const float* __restrict__ W, float* __restrict__ C, int M,
@@ -269,8 +277,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
     fetch_a(s_begin + 2, As + 12 * BM);
     stash_w(Ws, rw0[0]);
     SP_STAGE_END(2 * NA);
+    const int flush = flush_after(s_end - s_begin);
     for (int s = s_begin; s < s_end;) {
-      const int stop = min(s + SP_FLUSH, s_end);
+      const int stop = min(s + flush, s_end);
       for (; s < stop; s += 4) {
         stage(s, Slot<0>(), rw0[1], &rw0);
         stage(s + 1, Slot<1>(), rw1[0], nullptr);
@@ -325,16 +334,16 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
 // and 4-7, 8-11, 16-19, 28-31, and rows of 256 bytes and more then touch every bank once.
 // gridDim.z parts of K, each with sums [M, N] of its own.
 //
-// Measured, the float32 matrix instruction / this kernel in us (weights not in a cache): K 2048, 16,384 rows of W 43 / 31 at
-// 24 rows of A, 65 / 40 at 64, 121 / 61 at 128; 3,072 rows of W in four parts 20 / 10, 2,048 in eight 8.7 / 8.7; K 8192, 2,048
-// rows in eight parts 24 / 18; 128,256 rows 315 / 216 at 24, 489 / 307 at 64, 965 / 489 at 128.  A step at 24 rows reads
-// its 134 MB at 4.3 TB/s; from 64 rows on the splits of A, which every workgroup makes again, weigh as much.  Distance to
-// 64 bits (rms, of the result's size), K 2048, 8192 and 14336: 2.9e-7, 3.9e-7 and 3.9e-7 before, 1.2e-7, 2.0e-7 and 2.7e-7 at
-// 24 rows, 1.5e-7, 2.8e-7 and 3.7e-7 at 100; K in eight parts 1.0e-7, 1.3e-7 and 1.5e-7.
-// From five rows, with K in parts: 12.3, 10.3 and 24.6 us with the kernel of few rows of csrc/gemm.hip over 3,072 and 2,048
-// rows of W at K 2048 and 2,048 at K 8192, 9.8, 8.6 and 18.1 with this one; up to four rows they are level.  Up to 128 rows,
-// which is what a stage has room for: at 128 the tiles above take 25, 18, 88 (16,384 rows of W) and 51 us where this takes
-// 21, 16, 61 and 36, and only over 128,256 rows of W 402 for 489.
+// Measured, the float32 matrix instruction / this kernel in us (weights not in a cache): K 2048, 16,384 rows of W 43 / 32 at
+// 24 rows of A, 65 / 41 at 64, 121 / 67 at 128; 3,072 rows of W in four parts 20 / 10, 2,048 in eight 8.7 / 8.3; K 8192, 2,048
+// rows in eight parts 24 / 19; 128,256 rows 315 / 219 at 24, 489 / 332 at 64, 965 / 550 at 128.  A step at 24 rows reads
+// its 134 MB at 4.2 TB/s; from 64 rows on the splits of A, which every workgroup makes again, weigh as much.  Distance to
+// 64 bits (rms, of the result's size), normal operands: K 2048 2.9e-7 / 1.1e-7 at 24 rows and 1.35e-7 at 100, K 8192 3.9e-7 /
+// 1.4e-7 at 64 and 100; operands in 1 .. 2: 0.97e-7 / 0.48e-7 and 0.68e-7, 0.88e-7 / 0.56e-7.
+// From five rows, with K in parts: level with the kernel of few rows of csrc/gemm.hip over 3,072 and 2,048 rows of W at K 2048
+// (9.3 and 8.2 us there, 9.9 and 8.1 here), 21.3 / 18.6 over 2,048 at K 8192.  Up to 128 rows, which is what a stage has room
+// for: at 128 the tiles above take 20, 87 (16,384 rows of W) and 51 us where this takes 17, 67 and 38, and only over
+// 128,256 rows of W 366 for 550.
 // ---------------------------------------------------------------------------------------------
 template <int MT, int NT>
 __device__ __forceinline__ void read_rows(Frag8 (&w)[2], Frag8 (&a)[MT][2], uint32_t w0, uint32_t w1, uint32_t a0, uint32_t a1) {
@@ -415,48 +424,65 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   const uint32_t a1 = base + (32 * NT + r) * ROWB + (((seg0 + 1) ^ (r & 15)) << 4);
 
   // the large products x0 w0 and the small ones in sums of their own: a rounding of the large sum an instruction, not six
-  floatx16_t acc[MT], low[MT];
+  // (the large ones in two levels; with four tiles of A there are no registers for it, and the launch keeps K short)
+  constexpr int TOTALS = MT <= 3 ? MT : 0;
+  floatx16_t acc[MT], low[MT], total[TOTALS ? TOTALS : 1];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[mt][e] = low[mt][e] = 0.f;
+#pragma unroll
+  for (int mt = 0; mt < TOTALS; ++mt)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) total[mt][e] = 0.f;
 
   if (n > 0) {
 #pragma unroll
     for (int i = 0; i < NB - 1; ++i) fetch(i);
-    for (int s = 0; s < n; ++s) {
-      // stage s has landed: behind it come those of NB - 2 stages; everybody has read the one before, whose place is free
-      SP_STAGE_END(ND * (NB - 2));
-      fetch(s + NB - 1);
-      const uint32_t off = (uint32_t)((s % NB) * STAGE);
-      Frag8 wf[2], af[MT][2];
-      read_rows<MT, NT>(wf, af, w0 + off, w1 + off, a0 + off, a1 + off);
-      const int k = (s_begin + s) * COLS + kc * 16 + h * 8;
-      if ((s_begin + s + 1) * COLS > K) {                    // the last columns: beyond K the operand of A is zero
-        const u32x4_t zero4 = {0u, 0u, 0u, 0u};
+    for (int s = 0; s < n;) {
+      const int stop = min(s + SP_ROWS_FLUSH, n);
+      for (; s < stop; ++s) {
+        // stage s has landed: behind it come those of NB - 2 stages; everybody has read the one before, whose place is free
+        SP_STAGE_END(ND * (NB - 2));
+        fetch(s + NB - 1);
+        const uint32_t off = (uint32_t)((s % NB) * STAGE);
+        Frag8 wf[2], af[MT][2];
+        read_rows<MT, NT>(wf, af, w0 + off, w1 + off, a0 + off, a1 + off);
+        const int k = (s_begin + s) * COLS + kc * 16 + h * 8;
+        if ((s_begin + s + 1) * COLS > K) {                    // the last columns: beyond K the operand of A is zero
+          const u32x4_t zero4 = {0u, 0u, 0u, 0u};
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) {
+            if (k >= K) af[mt][0].u = zero4;
+            if (k + 4 >= K) af[mt][1].u = zero4;
+          }
+        }
+        constexpr int PA[5] = {2, 1, 0, 1, 0}, PW[5] = {0, 1, 2, 0, 1};
+        u32x4_t q[3];
+        Frag8 w[3], a[MT][3];
+        split8(wf[0].f, wf[1].f, q);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) w[p].u = q[p];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          if (k >= K) af[mt][0].u = zero4;
-          if (k + 4 >= K) af[mt][1].u = zero4;
+          split8(af[mt][0].f, af[mt][1].f, q);
+#pragma unroll
+          for (int p = 0; p < 3; ++p) a[mt][p].u = q[p];
+          acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[0].v, a[mt][0].v, acc[mt], 0, 0, 0);
+#pragma unroll
+          for (int p = 0; p < 5; ++p)
+            low[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[PW[p]].v, a[mt][PA[p]].v, low[mt], 0, 0, 0);
         }
       }
-      constexpr int PA[5] = {2, 1, 0, 1, 0}, PW[5] = {0, 1, 2, 0, 1};
-      u32x4_t q[3];
-      Frag8 w[3], a[MT][3];
-      split8(wf[0].f, wf[1].f, q);
 #pragma unroll
-      for (int p = 0; p < 3; ++p) w[p].u = q[p];
+      for (int mt = 0; mt < TOTALS; ++mt) {
+        total[mt] += acc[mt];
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        split8(af[mt][0].f, af[mt][1].f, q);
-#pragma unroll
-        for (int p = 0; p < 3; ++p) a[mt][p].u = q[p];
-        acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[0].v, a[mt][0].v, acc[mt], 0, 0, 0);
-#pragma unroll
-        for (int p = 0; p < 5; ++p)
-          low[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[PW[p]].v, a[mt][PA[p]].v, low[mt], 0, 0, 0);
+        for (int e = 0; e < 16; ++e) acc[mt][e] = 0.f;
       }
     }
+#pragma unroll
+    for (int mt = 0; mt < TOTALS; ++mt) acc[mt] = total[mt];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[mt] += low[mt];
     SP_STAGE_END(0);                                         // (loads beyond the last stage; everybody has read it)
@@ -529,6 +555,11 @@ static int launch_f32_wide(const void* A, const void* W, void* C, int M, int N, 
 }
 
 static int few_rows(const void* A, const void* W, void* C, int M, int N, int K, int parts, size_t part_stride, hipStream_t stream) {
+  // (four tiles of A have no registers for sums in two levels: over a long inner size twice two of them)
+  if (M > 96 && K / parts > 4096) {
+    const int rc = few_rows(A, W, C, 64, N, K, parts, part_stride, stream);
+    return rc != 0 ? rc : few_rows((const float*)A + (size_t)64 * K, W, (float*)C + (size_t)64 * N, M - 64, N, K, parts, part_stride, stream);
+  }
   // 64 rows of W a workgroup, or 32 where those would leave half of the chip idle (up to 64 rows of A: LDS)
   if (M <= 64 && (long long)((N + 63) / 64) * parts <= compute_units() / 2) {
     if (M <= 32) return launch_f32_wide<1, 1, 3>(A, W, C, M, N, K, parts, part_stride, stream);

@@ -163,9 +163,9 @@ def gemm_nt(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor
     if out.dtype == torch.float32:
         if gemm_f32_split_available(a, w):
             return gemm_f32_split(a, w, out)
-        # (5 to 8 rows of a narrow matrix leave most of the chip without a workgroup there: 12.0 us with the kernel of few
-        # rows, 14.5 with this one, over 3,072 rows of W at K 2048, 24.5 and 38.8 over 2,048 at K 8192, but 39 and 32 over
-        # 16,384 at K 2048)
+        # (5 to 8 rows of a narrow matrix leave most of the chip without a workgroup there: 9.7 us with the kernel of few
+        # rows, 15.4 with this one, over 3,072 rows of W at K 2048, 21.6 and 45.2 over 2,048 at K 8192; level over 16,384 at
+        # K 2048, 32)
         if gemm_f32_mid_available(a, w) and (M > ROWS_KERNEL_MAX_ROWS or N >= 32 * compute_units()):
             gemm_f32_mid_parts(a, w, out.unsqueeze(0))
             return out
@@ -186,7 +186,8 @@ def gemm_f32_split_available(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 
 def gemm_f32_split(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
-    """out = a @ w^T in float32 through exact splits of the operands into bf16 numbers; out fp32 [M, N], or [parts, M, N]
+    """out = a @ w^T in float32 through exact splits of the operands into bf16 numbers (a product of two floats to 2^-24 of
+    it); out fp32 [M, N], or [parts, M, N]
     (1 to 8): the inner dimension cut into parts over the grid, whose sums the consumer adds in order."""
     _dev(a, w, out)
     M, K = a.shape
@@ -224,7 +225,7 @@ def _f32_split_plan(M: int, N: int, K: int, parts: int):
     whole = _f32_tiles_cost(tiles, N, K, parts)
     if not tail or tiles == 1 or (tiles - 1) * -(-N // 128) * parts < compute_units():
         return whole, 0
-    cut = _f32_tiles_cost(tiles - 1, N, K, parts) + 5.0 + N * K * 4 / 4.3e6 * (1.0, 1.25, 1.6, 1.9)[(tail - 1) // 32]
+    cut = _f32_tiles_cost(tiles - 1, N, K, parts) + 5.0 + N * K * 4 / 4.3e6 * (1.0, 1.3, 1.7, 2.1)[(tail - 1) // 32]
     return (cut, tail) if cut < 0.97 * whole else (whole, 0)
 
 
@@ -389,7 +390,7 @@ def paged_attention_tiled_f32(q: torch.Tensor, q_row_stride: int, out: torch.Ten
                               scale: float, window: Optional[int], num_splits: int = 1,
                               sinks: Optional[torch.Tensor] = None, chunk: Optional[int] = None) -> torch.Tensor:
     """float32 attention: 64 rows (tokens x the query heads of a KV head) a workgroup share the keys
-    and values of their KV head through LDS (fp32 arithmetic on the vector ALU).  `num_splits` > 1
+    and values of their KV head through LDS (the matrix cores' float32 instruction).  `num_splits` > 1
     cuts the key range of every tile into that many parts across workgroups, merged by a second kernel
     (for few rows over long contexts, where there are few tiles; the segments then begin at token 0).
     The tables may describe a run of the step's segments only: `num_tokens` then counts the tokens up

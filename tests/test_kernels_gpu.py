@@ -182,6 +182,55 @@ def test_gemm_f32_by_split_operands_with_the_end_cut_off(monkeypatch, M, N, K, p
         assert torch.equal(end, out[:, M - M % 128:])
 
 
+@pytest.mark.parametrize("M", [24, 70, 100, 300])
+def test_gemm_f32_by_split_operands_loses_no_more_than_a_rounding(M):
+    """One product a result: random mantissas, and those at which the terms left out weigh most with planes rounded to the
+    nearest (1.0038986) and with planes cut (1 + 2^-7 - 2^-23).  And no drift: operands of one sign."""
+    from serve_amd import ops
+    N, K = 70, 4
+    g = torch.Generator().manual_seed(22)
+    x, y = 1 + torch.rand((M,), generator=g), 1 + torch.rand((N,), generator=g)
+    worst = torch.tensor([0x3f807fc0, 0x3f807fff, 0x3f804040, 0x3fffffff], dtype=torch.int32).view(torch.float32)
+    x[:4], y[:4], y[4:8] = worst, worst, worst.flip(0)
+    a, w = torch.zeros((M, K)), torch.zeros((N, K))
+    a[:, 1], w[:, 1] = x, y
+    a, w = a.to(DEV), w.to(DEV)
+    out = torch.empty((M, N), dtype=torch.float32, device=DEV)
+    ops.gemm_nt(a, w, out)
+    want = a.double() @ w.double().T
+    err = (out.double() - want) / want
+    # what is left out is at most 2^-24 of the product, and the sum is rounded once, 2^-24.  Where all six products go to one
+    # sum (the tiles), the matrix cores cut the sum of the small ones two bits behind the last place of the largest: 2^-25 at
+    # most, 2^-26 on the average, always the same way
+    one_sum = 2.0 ** -25 if M > ops.F32_MID_MAX_ROWS else 0.0
+    assert err.abs().max() <= 2.0 ** -24 + 2.0 ** -24 + one_sum + 2.0 ** -30, err.abs().max().log2()
+    # (1,680 results and more, each off by some 2^-25.5 of either sign)
+    assert err.mean().abs() <= one_sum / 1.5 + 2.0 ** -28, err.mean()
+
+
+@pytest.mark.parametrize("M,N,K", [(24, 1024, 2048), (64, 512, 8192), (100, 512, 8192), (300, 512, 2048), (300, 256, 14336)])
+@pytest.mark.parametrize("signs", [True, False])
+def test_gemm_f32_by_split_operands_is_as_close_as_sums_in_two_levels(M, N, K, signs):
+    """The distance to 64 bits is no larger than that of float32 sums rounded at every column, of which every 512 columns
+    join a second sum (the order of the product on the matrix cores' float32 instruction), for operands of either sign and of
+    one."""
+    from serve_amd import ops
+    a, w = rnd((M, K), torch.float32, 25), rnd((N, K), torch.float32, 26)
+    if not signs:
+        a, w = 1 + a.abs().remainder(1.0), 1 + w.abs().remainder(1.0)
+    out = torch.empty((M, N), dtype=torch.float32, device=DEV)
+    ops.gemm_nt(a, w, out)
+    want = a.double() @ w.double().T
+    total = torch.zeros((M, N), dtype=torch.float32, device=DEV)
+    for k0 in range(0, K, 512):
+        sums = torch.zeros((M, N), dtype=torch.float32, device=DEV)
+        for k in range(k0, k0 + 512):
+            sums = torch.addcmul(sums.double(), a[:, k: k + 1].double(), w[:, k].double()).float()
+        total += sums
+    rms = lambda x: (x.double() - want).pow(2).mean().sqrt().item()   # noqa: E731
+    assert rms(out) <= rms(total), (rms(out), rms(total))
+
+
 @pytest.mark.parametrize("M,N,K", [(24, 2048, 2048), (100, 1024, 8192), (300, 2048, 2048), (300, 512, 8192)])
 def test_gemm_f32_by_split_operands_is_as_close_as_float32(M, N, K):
     """The distance to 64 bits is no larger than that of one float32 sum a result in steps of two columns (what the matrix
