@@ -9,6 +9,9 @@
 // the average, always towards zero.)  Sums are float32, in two levels.  What remains with a sign: the matrix cores cut an
 // addend two bits behind the last place of the sum, 2^-26 of a stage's sum where all six products go to one accumulator.
 //
+// Range: bf16 has the exponents of float32 but no bits below 2^-133, and what the matrix instruction does with numbers
+// below 2^-126 is not relied on.  So results that such numbers can have reached are computed again, see redo_limit.
+//
 // Why: the float32 matrix instruction runs at a sixteenth of the bf16 rate; six bf16 instructions for the same terms
 // are 2.7 times as fast where both are at their peak.
 #include "common.h"
@@ -72,13 +75,22 @@ __device__ __forceinline__ void split8(const f32x4_t& a, const f32x4_t& b, u32x4
   }
 }
 
+// The largest size among m and eight floats (NaN aside).
+__device__ __forceinline__ void max8(float& m, const f32x4_t& a, const f32x4_t& b) {
+  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a.x), "v"(a.y));
+  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(a.z), "v"(a.w));
+  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(b.x), "v"(b.y));
+  asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(m) : "v"(b.z), "v"(b.w));
+}
+
 // The rows of A as planes, in the order the product reads them: 16-byte unit ((stage * 3 + plane) * 2 + half) * Mp + row
-// holds columns 16 stage + 8 half .. + 7 of a row.  Columns beyond K and rows beyond M are zeros.
-__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ A, u32x4_t* __restrict__ P, int M, int Mp,
-                                                        int K, int halves) {
+// holds columns 16 stage + 8 half .. + 7 of a row.  Columns beyond K and rows beyond M are zeros.  A workgroup takes 32
+// rows (Mp is a multiple of them) by 64 columns and leaves their largest size in `most` [rows / 32][columns / 64].
+__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ A, u32x4_t* __restrict__ P,
+                                                        float* __restrict__ most, int M, int Mp, int K) {
+  __shared__ float sizes[4];
   const int k8 = blockIdx.y * 8 + (threadIdx.x & 7);
   const int row = blockIdx.x * 32 + (threadIdx.x >> 3);
-  if (k8 >= halves || row >= Mp) return;
   const f32x4_t zero4 = {0.f, 0.f, 0.f, 0.f};
   f32x4_t a = zero4, b = zero4;
   const int k = k8 * 8;
@@ -91,28 +103,72 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
   split8(a, b, q);
 #pragma unroll
   for (int i = 0; i < 3; ++i) P[((size_t)((k8 >> 1) * 3 + i) * 2 + (k8 & 1)) * Mp + row] = q[i];
+  float m = 0.f;
+  max8(m, a, b);
+  m = wave_max(m);
+  if ((threadIdx.x & 63) == 0) sizes[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    most[(size_t)blockIdx.x * gridDim.y + blockIdx.y] = fmaxf(fmaxf(sizes[0], sizes[1]), fmaxf(sizes[2], sizes[3]));
 }
 
-// A result that is computed again, term by term in float32: one that is not finite (with an infinite operand the planes'
-// products are not those of the floats: infinity times a zero plane), and one below 2^-64 (the matrix instruction takes
-// planes below 2^-126 as zeros: beside factors up to 2^36 that is nothing to a larger result).  A result of exactly zero
-// stays: rows of zeros are ordinary, sums of which no term reaches 2^-126 are not.
-__device__ __forceinline__ bool to_redo(float v) {
-  const uint32_t u = __float_as_uint(v) & 0x7fffffffu;
-  return u >= 0x7f800000u || u - 1u < (63u << 23) - 1u;
+// Results that are computed again, term by term in 64 bits, if need be.
+// * One that is not finite: with an infinite operand, or one that rounds to infinity, the planes' products are not those of
+//   the floats (infinity times a zero plane).
+// * One that numbers below 2^-126 may have reached.  Taking every plane and every product of planes below that as zero
+//   would change a sum of K products by less than 3 K 2^-126 (|a| + |w|) + 6 K 2^-126, with the largest |a| and |w| of the
+//   workgroup's rows.  That is nothing (2^-26 of it) to a result above redo_limit.  The others, the zeros among them, are
+//   computed again if the operands of the workgroup's rows are small enough for it: no plane of a number of 2^-103 and
+//   more is below 2^-126, and products of planes that are make 2^-29 of the numbers' product where that is 2^-94 and more.
+//   Results of rows of zeros, and small ones of ordinary operands, so stay as they are.
+__device__ __forceinline__ float redo_limit(float most_a, float most_w, int K) {
+  if (most_a == 0.f || most_w == 0.f) return -1.f;                   // (all results are zeros, or not finite)
+  const float limit = (float)K * 0x1p-97f * (1.f + most_a + most_w);
+  return limit == limit ? limit : INFINITY;
 }
 
-// C[m, n], just stored by this lane, once more if need be.
-__device__ __noinline__ void redo(const float* A, const float* W, float* C, int m, int n, int N, int K, int k_begin, int k_end) {
+// The bits, twice, less one, of the smallest number but zero in rows row0 .. row0 + rows - 1 (below `end`) of X, columns
+// k_begin .. k_end - 1; all ones if there is none.  For a whole wave.
+__device__ __forceinline__ uint32_t least_key(const float* X, int row0, int rows, int end, int K, int k_begin, int k_end) {
+  const int lane = threadIdx.x & 63;
+  uint32_t key = 0xffffffffu;
+  for (int r = row0; r < row0 + rows; r += 16)
+    for (int k = k_begin + lane * 4; k < k_end; k += 256) {
+      f32x4_t v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const f32x4_t*>(X + (size_t)min(r + i, end - 1) * K + k);
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) key = min(key, (__float_as_uint(v[i][e]) << 1) - 1u);
+    }
+  for (int o = 32; o > 0; o >>= 1) key = min(key, (uint32_t)__shfl_xor((int)key, o, SA_WAVE));
+  return key;
+}
+
+// Whether numbers below 2^-126 can have come up in the products of these rows of A and W.  For a whole wave.
+__device__ __forceinline__ bool small_operands(const float* A, int m0, int ms, int M, const float* W, int n0, int ns, int N, int K,
+                                           int k_begin, int k_end) {
+  const uint32_t ka = least_key(A, m0, ms, M, K, k_begin, k_end), kw = least_key(W, n0, ns, N, K, k_begin, k_end);
+  if (ka == 0xffffffffu || kw == 0xffffffffu) return false;          // (nothing but zeros)
+  const float a = __uint_as_float((ka + 1u) >> 1), w = __uint_as_float((kw + 1u) >> 1);
+  return a < 0x1p-103f || w < 0x1p-103f || a * w < 0x1p-94f;
+}
+
+// C[m, n], just stored by this lane, once more if it is not finite or at most `limit`.
+__device__ __noinline__ void redo(const float* A, const float* W, float* C, int m, int n, int N, int K, int k_begin, int k_end,
+                                  float limit) {
   float* cp = C + (size_t)m * N + n;
-  if (!to_redo(*cp)) return;
-  float sum = 0.f;
+  const float size = fabsf(*cp);
+  if (size > limit && size < INFINITY) return;
+  double sum = 0.0;
   for (int k = k_begin; k < k_end; k += 4) {
     const f32x4_t a = *reinterpret_cast<const f32x4_t*>(A + (size_t)m * K + k);
     const f32x4_t w = *reinterpret_cast<const f32x4_t*>(W + (size_t)n * K + k);
-    sum = fmaf(a.w, w.w, fmaf(a.z, w.z, fmaf(a.y, w.y, fmaf(a.x, w.x, sum))));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sum = fma((double)a[e], (double)w[e], sum);
   }
-  *cp = sum;
+  *cp = (float)sum;
 }
 
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
@@ -173,9 +229,10 @@ __device__ __forceinline__ void read_stage(Frag8 (&a)[TI][3], Frag8 (&w)[2][3], 
 // operands, K 2048 4.1e-7 / 2.5e-7, K 8192 4.1e-7 / 2.7e-7, K 14336 4.2e-7 / 3.4e-7; operands in 1 .. 2, 1.7e-7 / 0.8e-7,
 // 1.05e-7 / 0.92e-7 and 0.95e-7 / 0.90e-7; all operands the same number (60 pairs of them), K 2048 4.1e-6 / 0.5e-6.
 template <int TI>
-__global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* __restrict__ P, const float* __restrict__ A,
-                                                                const float* __restrict__ W, float* __restrict__ C, int M,
-                                                                int Mp, int N, int K, int mtiles, size_t part_stride) {
+__global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* __restrict__ P, const float* __restrict__ most,
+                                                                const float* __restrict__ A, const float* __restrict__ W,
+                                                                float* __restrict__ C, int M, int Mp, int N, int K,
+                                                                int mtiles, size_t part_stride) {
   constexpr int BM = 64 * TI;
   constexpr int NA = (6 * BM + 255) / 256;         // kilobytes of A's planes a wave fetches a stage
   __shared__ u32x4_t As[4 * 6 * BM], Ws[2 * 6 * SP_WPITCH];
@@ -197,6 +254,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
   const int s_begin = 4 * (int)((long long)blockIdx.z * quads / gridDim.z);
   const int s_end = 4 * (int)((long long)(blockIdx.z + 1) * quads / gridDim.z);
   C += blockIdx.z * part_stride;
+
+  // the largest sizes among this workgroup's rows of A and (this thread's share, as they come by) of W
+  float most_a = 0.f, most_w = 0.f;
+  for (int i = tid, nq = (s_end - s_begin) >> 2; i < BM / 32 * nq; i += 256)
+    most_a = fmaxf(most_a, most[(size_t)(m0 / 32 + i / nq) * quads + (s_begin >> 2) + i % nq]);
 
   f32x4_t rw0[2][2], rw1[2][2];
   const float* wrow = W + (size_t)min(n0 + (tid >> 1), N - 1) * K;
@@ -222,6 +284,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
   auto stash_w = [&](u32x4_t* ws, f32x4_t (&rw)[2]) __attribute__((always_inline)) {
     u32x4_t q[3];
     split8(rw[0], rw[1], q);
+    max8(most_w, rw[0], rw[1]);
 #pragma unroll
     for (int i = 0; i < 3; ++i) ws[(i * 2 + (tid & 1)) * SP_WPITCH + (tid >> 1)] = q[i];
   };
@@ -298,7 +361,17 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
     SP_STAGE_END(0);                  // (loads into LDS beyond the last stage)
   }
 
-  bool bad = false;
+  float* sizes = reinterpret_cast<float*>(As);
+  most_a = wave_max(most_a);
+  most_w = wave_max(most_w);
+  if (lane == 0) {
+    sizes[wave] = most_a;
+    sizes[4 + wave] = most_w;
+  }
+  __syncthreads();
+  const float limit = redo_limit(fmaxf(fmaxf(sizes[0], sizes[1]), fmaxf(sizes[2], sizes[3])),
+                                 fmaxf(fmaxf(sizes[4], sizes[5]), fmaxf(sizes[6], sizes[7])), K);
+  bool small = false, odd = false;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -310,17 +383,21 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
         const float v = total[i][j][e];
         if (m < M && n < N) {
           C[(size_t)m * N + n] = v;
-          bad |= to_redo(v);
+          small |= fabsf(v) <= limit;
+          odd |= !(fabsf(v) < INFINITY);
         }
       }
     }
-  if (!bad) return;
+  const bool any_small = __any(small);
+  if (!any_small && !__any(odd)) return;
   const int k_begin = s_begin * 16, k_end = min(K, s_end * 16);
+  const float below = any_small && small_operands(A, m0 + wm * 32 * TI, 32 * TI, M, W, n0 + wn * 64, 64, N, K, k_begin, k_end) ? limit : -1.f;
+  if (!odd && !(small && below >= 0.f)) return;
   for (int x = 0; x < TI * 32; ++x) {
     const int m = m0 + wm * 32 * TI + (x >> 5) * 32 + 8 * ((x & 15) >> 2) + 4 * h + (x & 3);
     const int n = n0 + wn * 64 + ((x >> 4) & 1) * 32 + r32;
     if (m >= M || n >= N) continue;
-    redo(A, W, C, m, n, N, K, k_begin, k_end);
+    redo(A, W, C, m, n, N, K, k_begin, k_end, below);
   }
 }
 
@@ -423,6 +500,7 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   const uint32_t a0 = base + (32 * NT + r) * ROWB + ((seg0 ^ (r & 15)) << 4);
   const uint32_t a1 = base + (32 * NT + r) * ROWB + (((seg0 + 1) ^ (r & 15)) << 4);
 
+  float most_a = 0.f, most_w = 0.f;                          // the largest sizes of what this wave reads
   // the large products x0 w0 and the small ones in sums of their own: a rounding of the large sum an instruction, not six
   // (the large ones in two levels; with four tiles of A there are no registers for it, and the launch keeps K short)
   constexpr int TOTALS = MT <= 3 ? MT : 0;
@@ -461,11 +539,13 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
         u32x4_t q[3];
         Frag8 w[3], a[MT][3];
         split8(wf[0].f, wf[1].f, q);
+        max8(most_w, wf[0].f, wf[1].f);
 #pragma unroll
         for (int p = 0; p < 3; ++p) w[p].u = q[p];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
           split8(af[mt][0].f, af[mt][1].f, q);
+          max8(most_a, af[mt][0].f, af[mt][1].f);
 #pragma unroll
           for (int p = 0; p < 3; ++p) a[mt][p].u = q[p];
           acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[0].v, a[mt][0].v, acc[mt], 0, 0, 0);
@@ -488,6 +568,13 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
     SP_STAGE_END(0);                                         // (loads beyond the last stage; everybody has read it)
   }
 
+  __shared__ float sizes[16];
+  most_a = wave_max(most_a);
+  most_w = wave_max(most_w);
+  if (lane == 0) {
+    sizes[wave] = most_a;
+    sizes[8 + wave] = most_w;
+  }
   float* sums = reinterpret_cast<float*>(ring);              // [KH - 1][NT][MT][16][64]
   if (kc > 0) {
 #pragma unroll
@@ -497,7 +584,13 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   }
   __syncthreads();
   if (kc > 0) return;
-  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    most_a = fmaxf(most_a, sizes[i]);
+    most_w = fmaxf(most_w, sizes[8 + i]);
+  }
+  const float limit = redo_limit(most_a, most_w, K);
+  bool small = false, odd = false;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int m = mt * 32 + r;
@@ -516,7 +609,10 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
       if (m >= M) continue;
       float* cp = C + (size_t)m * N + cn;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) bad |= cn + c < N && to_redo(v[c]);
+      for (int c = 0; c < 4; ++c) {
+        small |= cn + c < N && fabsf(v[c]) <= limit;
+        odd |= cn + c < N && !(fabsf(v[c]) < INFINITY);
+      }
       if (cn + 3 < N && (((uintptr_t)cp) & 15) == 0) {
         *reinterpret_cast<f32x4_t*>(cp) = (f32x4_t){v[0], v[1], v[2], v[3]};
       } else {
@@ -526,11 +622,14 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
       }
     }
   }
-  if (!bad) return;
+  const bool any_small = __any(small);
+  if (!any_small && !__any(odd)) return;
+  const int k_begin = s_begin * COLS, k_end = min(K, (s_begin + n) * COLS);
+  const float below = any_small && small_operands(A, 0, 32 * MT, M, W, n0 + wt * 32, 32, N, K, k_begin, k_end) ? limit : -1.f;
+  if (!odd && !(small && below >= 0.f)) return;
   for (int x = 0; x < MT * 16; ++x) {
     const int m = (x >> 4) * 32 + r, cn = n0 + wt * 32 + ((x & 15) >> 2) * 8 + h * 4 + (x & 3);
-    if (m < M && cn < N)
-      redo(A, W, C, m, cn, N, K, s_begin * COLS, min(K, (s_begin + n) * COLS));
+    if (m < M && cn < N) redo(A, W, C, m, cn, N, K, k_begin, k_end, below);
   }
 }
 
@@ -590,8 +689,11 @@ static int plane_rows(int M, int K) {
   return (int)(run < 128 ? 128 : run < all ? run : all);
 }
 
+// ... and behind them the largest sizes of their pieces of 32 rows by 64 columns.
+static long long plane_bytes(int M, int K) { return ((long long)K + 63) / 64 * 64 * 6 * plane_rows(M, K); }
+
 extern "C" long long sa_gemm_f32_split_bytes(int M, int K) {
-  return M > 0 && K > 0 ? ((long long)K + 63) / 64 * 64 * 6 * plane_rows(M, K) : 0;
+  return M > 0 && K > 0 ? plane_bytes(M, K) + ((long long)K + 63) / 64 * (plane_rows(M, K) / 32) * 4 : 0;
 }
 
 // C fp32 [parts, M, N] (1 to 8 parts of K, which the consumer adds in order); `planes`: sa_gemm_f32_split_bytes of
@@ -603,27 +705,27 @@ extern "C" int sa_gemm_f32_split(const void* A, const void* W, void* C, void* pl
   if (K <= 0 || (K & 3) || parts < 1 || parts > 8 || ((((uintptr_t)A | (uintptr_t)W | (uintptr_t)planes) & 15) != 0) ||
       tail < 0 || tail > 128 || tail >= M)
     return SA_ERR_ARG;
-  const int halves = (K + 63) / 64 * 8;
+  const int quads = (K + 63) / 64;
   const int run = plane_rows(M, K);
+  float* most = (float*)((char*)planes + plane_bytes(M, K));
   const long long ntiles = ((long long)N + SP_BN - 1) / SP_BN;
-  if ((run / 64) * ntiles > 0x7fffffffLL || (halves + 7) / 8 > 65535) return SA_ERR_ARG;
+  if ((run / 64) * ntiles > 0x7fffffffLL || quads > 65535) return SA_ERR_ARG;
   const int tiled = M - tail;
   for (long long row0 = 0; row0 < tiled; row0 += run) {
     const int rows = (int)(tiled - row0 < run ? tiled - row0 : run);
     const int Mp = (rows + 127) / 128 * 128;
     const float* a = (const float*)A + (size_t)row0 * K;
     float* c = (float*)C + (size_t)row0 * N;
-    hipLaunchKernelGGL(split_rows_kernel, dim3(Mp / 32, (halves + 7) / 8), dim3(256), 0, stream, a, (u32x4_t*)planes, rows, Mp,
-                       K, halves);
+    hipLaunchKernelGGL(split_rows_kernel, dim3(Mp / 32, quads), dim3(256), 0, stream, a, (u32x4_t*)planes, most, rows, Mp, K);
     SA_LAUNCH_CHECK();
     // tiles of 128 rows, or of 64 where those would leave compute units without one
     const long long mt128 = (rows + 127) / 128, mt64 = (rows + 63) / 64;
     if (mt128 * ntiles * parts >= compute_units())
       hipLaunchKernelGGL((gemm_f32_split_kernel<2>), dim3(mt128 * ntiles, 1, parts), dim3(256), 0, stream,
-                         (const u32x4_t*)planes, a, (const float*)W, c, rows, Mp, N, K, (int)mt128, (size_t)M * N);
+                         (const u32x4_t*)planes, most, a, (const float*)W, c, rows, Mp, N, K, (int)mt128, (size_t)M * N);
     else
       hipLaunchKernelGGL((gemm_f32_split_kernel<1>), dim3(mt64 * ntiles, 1, parts), dim3(256), 0, stream,
-                         (const u32x4_t*)planes, a, (const float*)W, c, rows, Mp, N, K, (int)mt64, (size_t)M * N);
+                         (const u32x4_t*)planes, most, a, (const float*)W, c, rows, Mp, N, K, (int)mt64, (size_t)M * N);
     SA_LAUNCH_CHECK();
   }
   if (tail == 0) return 0;

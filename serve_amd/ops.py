@@ -187,7 +187,7 @@ def gemm_f32_split_available(a: torch.Tensor, w: torch.Tensor) -> bool:
 
 def gemm_f32_split(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     """out = a @ w^T in float32 through exact splits of the operands into bf16 numbers (a product of two floats to 2^-24 of
-    it); out fp32 [M, N], or [parts, M, N]
+    it, over the whole range of float32); out fp32 [M, N], or [parts, M, N]
     (1 to 8): the inner dimension cut into parts over the grid, whose sums the consumer adds in order."""
     _dev(a, w, out)
     M, K = a.shape

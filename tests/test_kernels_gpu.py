@@ -208,6 +208,29 @@ def test_gemm_f32_by_split_operands_loses_no_more_than_a_rounding(M):
     assert err.mean().abs() <= one_sum / 1.5 + 2.0 ** -28, err.mean()
 
 
+@pytest.mark.parametrize("M,N,K,parts", [(24, 70, 516, 1), (100, 33, 260, 2), (130, 129, 516, 1), (300, 70, 1028, 3)])
+@pytest.mark.parametrize("ea,ew", [(-127, 100), (-149, 120), (-120, 100), (-112, 60), (-108, 60), (-103, 60), (-100, 120), (60, -112),
+                                   (-60, -60), (-64, -62), (-40, -75)])
+def test_gemm_f32_by_split_operands_over_the_range_of_floats(M, N, K, parts, ea, ew):
+    """Very small operands beside very large ones, products below 2^-126 whose sum is not, in all rows and in a few beside
+    ordinary ones; rows of zeros stay zeros."""
+    from serve_amd import ops
+    run = ops.gemm_f32_mid_parts if M <= ops.F32_MID_MAX_ROWS else ops.gemm_f32_split
+    a, w = rnd((M, K), torch.float32, 23), rnd((N, K), torch.float32, 24)
+    small, large = (a.double() * 2.0 ** ea).float(), (w.double() * 2.0 ** ew).float()
+    some, other = a.clone(), w.clone()
+    some[3], other[5] = small[3], large[5]
+    for a, w in ((small, large), (some, other)):
+        a[1], w[2] = 0, 0
+        out = torch.full((parts, M, N), float("nan"), dtype=torch.float32, device=DEV)
+        run(a, w, out)
+        want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+        got = out.double().sum(0)
+        # as above; results below the smallest normal number are rounded to multiples of 2^-149, part by part
+        assert ((got - want).abs() <= size * (2.0 ** -23 + (6 * (K // 16 + 1) + 16) * 2.0 ** -24) + parts * 2.0 ** -149).all()
+        assert (got[1] == 0).all() and (got[:, 2] == 0).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(24, 1024, 2048), (64, 512, 8192), (100, 512, 8192), (300, 512, 2048), (300, 256, 14336)])
 @pytest.mark.parametrize("signs", [True, False])
 def test_gemm_f32_by_split_operands_is_as_close_as_sums_in_two_levels(M, N, K, signs):
