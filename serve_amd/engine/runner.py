@@ -35,10 +35,21 @@ MIXED_MAX_PORTIONS = 32
 MIXED_MAX_TOKENS = 4096
 # steps of few tokens with prompt portions among them (short prompts, the ends of longer ones) are captured too, padded to
 # one of these token counts and a power of two of segments.  Launched kernel by kernel they are bound by the host: at the
-# 1B shape 17 tokens take 1.61 ms against 0.98 ms of kernels, replayed 1.12 ms.  Beyond 128 tokens the kernels take
-# longer than their launches.
-SMALL_TOKEN_PADS = (16, 32, 64, 96, 128)
-SMALL_MAX_SEGMENTS = 32
+# 1B shape 17 tokens take 1.61 ms against 0.98 ms of kernels, replayed 1.12 ms.
+# Only where the padding does not cost more than the launches: the kernels of a captured step are chosen for the bounds of
+# its shape, so that every segment counts as a portion of all the tokens over the longest context (single tokens of
+# decoding requests lose their own attention kernel, and key ranges are cut into fewer parts).  Kernel by kernel / replayed,
+# ms, in bfloat16: one portion of 3 to 60 tokens over 100 to 4,000 keys 1.54 .. 1.75 / 0.94 .. 1.25 at the 1B shape, 0.57 ..
+# 0.74 / 0.55 .. 0.67 with two layers of width 4,096; 8 decoding requests and a portion of 20, 1B shape: 1.97 / 1.30 over
+# 1,000 keys, 2.0 / 1.8 over 4,000 and 2.0 / 2.5 over 8,000, width 4,096: 0.70 / 0.67, 0.75 / 0.92 over 4,000; padded to 96
+# or 128 tokens 1.6 / 1.6 .. 1.8, with 8 decoding requests 1.8 / 2.1 and 2.1 / 2.8 over 8,000.  With recurrent layers
+# many segments lose (width 4,096, 16 portions of 4 tokens 1.27 / 1.32).  In float32 the kernels take as long as their launches
+# (20 tokens 2.03 / 2.00, 100 tokens 3.3 / 4.5; 8 decoding requests over 4,000 keys and a portion of 20 2.6 / 5.5).
+SMALL_TOKEN_PADS = (16, 32, 64)
+SMALL_FEW_SEGMENTS = 4              # up to so many segments: contexts of up to SMALL_CONTEXT_OF_FEW keys
+SMALL_CONTEXT_OF_FEW = 2048
+SMALL_MAX_SEGMENTS = 32             # more, in models without per-request state: of up to SMALL_CONTEXT_OF_MANY
+SMALL_CONTEXT_OF_MANY = 1024
 
 
 class _GraphEntry:
@@ -135,6 +146,7 @@ class ModelRunner:
         self.sampled = torch.zeros(max(ASYNC_GRAPH_BATCHES[-1], MIXED_DECODE_PADS[-1] + MIXED_MAX_PORTIONS,
                                        cfg.max_requests), dtype=torch.int32, device=rt.device)
         self._row_of = {}
+        self._has_state = any(s is not None for s in sreq)
         self._use_graphs = bool(cfg.use_graphs) and model.graph_safe()
         # steps launched ahead of the host need parts that never read back from the device
         self._launch_ahead = model.graph_safe()
@@ -316,8 +328,11 @@ class ModelRunner:
         (tokens, segments, pages of a block table's row, bucket of the longest context).  What is missing of the
         tokens are inert segments: single tokens, and the last takes the rest; so a padded step has at least one of
         them.  As many logit rows as segments."""
-        if not self._use_graphs or not 0 < len(segments) <= SMALL_MAX_SEGMENTS:
+        if not self._use_graphs or self.rt.dtype != torch.bfloat16 or not 0 < len(segments) <= SMALL_MAX_SEGMENTS:
             return None
+        most_keys = SMALL_CONTEXT_OF_FEW
+        if len(segments) > SMALL_FEW_SEGMENTS:
+            most_keys = 0 if self._has_state else SMALL_CONTEXT_OF_MANY
         tokens = sum(len(s.tokens) for s in segments)
         if tokens > SMALL_TOKEN_PADS[-1] or any(s.req_id is INERT or s.req_id not in self.cache for s in segments):
             return None
@@ -340,7 +355,7 @@ class ModelRunner:
         while bucket < longest:
             bucket *= 2
         limit = self.cfg.max_pages_per_request * self.cfg.page_size
-        if longest > limit:                      # (beyond the context limit: an error below; the inert portion must fit, too)
+        if longest > limit or longest > most_keys:   # (beyond the context limit: an error below; the inert portion must fit, too)
             return None
         bucket = min(bucket, limit)
         # (many shapes, each used now and then: they take free places among the kept graphs, not those of decode steps)

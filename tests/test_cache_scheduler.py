@@ -446,3 +446,34 @@ def test_stop_tokens_keep_the_host_in_step():
     assert not sched.async_decode
     out = sched.run([GenerationRequest(1, [4, 5], 6)])
     assert out[0].generated == alone([4, 5], 3) and runner.handles == []
+
+
+def test_which_small_steps_are_padded_and_replayed():
+    """Decoding requests beside a portion, follow-ups over long contexts, many segments of a model with recurrent layers and
+    float32 steps run kernel by kernel where a shape's bounds would take their kernels away; the padded shapes of the others."""
+    from types import SimpleNamespace as NS
+
+    import torch
+
+    from serve_amd.engine import runner as rn
+
+    class Cache(dict):
+        tokens_of = dict.__getitem__
+
+    def shape(portions, dtype=None, state=False, graphs=(), limit=4096):
+        r = NS(_use_graphs=True, _has_state=state, rt=NS(dtype=dtype or torch.bfloat16), _graphs={k: None for k in graphs},
+               cache=Cache({i: c for i, (c, _, _) in enumerate(portions)}),
+               cfg=NS(max_pages_per_request=limit // 16, page_size=16, max_graphs=64))
+        got = rn.ModelRunner._small_shape(r, [Segment(i, [1] * n, w) for i, (_, n, w) in enumerate(portions)])
+        return got and got[:2] + got[3:]
+    one = [0]
+    assert shape([(0, 17, [16])]) == (32, 2, 256) and shape([(0, 64, [63])]) == (64, 1, 256)
+    assert shape([(0, 65, [64])]) is None and shape([(0, 17, [16])], torch.float32) is None
+    assert shape([(1000, 20, [19])]) == (32, 2, 1024) and shape([(2038, 10, [9])]) == (16, 2, 2048)
+    assert shape([(2039, 10, [9])]) is None
+    assert shape([(900, 1, one)] * 3 + [(0, 20, [19])], state=True) == (32, 8, 1024)
+    assert shape([(2048, 1, one)] * 3 + [(0, 20, [19])]) is None
+    assert shape([(900, 1, one)] * 8 + [(0, 20, [19])]) == (64, 16, 1024)
+    assert shape([(1024, 1, one)] * 8 + [(0, 20, [19])]) is None
+    assert shape([(900, 1, one)] * 8 + [(0, 20, [19])], state=True) is None
+    assert shape([(0, 4, [3])] * 5, state=True) is None

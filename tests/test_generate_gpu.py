@@ -226,7 +226,8 @@ def test_small_steps_with_prompt_portions_replayed_from_graphs(tmp_path, dtype):
         for k in toks:
             eng.runner.release(k)
     small = [e for k, e in eng.runner._graphs.items() if k[0] == "small"]
-    assert len(small) == 5 and all(e.graph is not None for e in small)
+    # (in float32 such steps run kernel by kernel, and so do those of more than 64 tokens)
+    assert len(small) == (3 if dtype == "bfloat16" else 0) and all(e.graph is not None for e in small)
 
 
 @pytest.mark.parametrize("live", [44, 64, 100])
