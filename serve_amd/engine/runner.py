@@ -50,6 +50,7 @@ SMALL_FEW_SEGMENTS = 4              # up to so many segments: contexts of up to 
 SMALL_CONTEXT_OF_FEW = 2048
 SMALL_MAX_SEGMENTS = 32             # more, in models without per-request state: of up to SMALL_CONTEXT_OF_MANY
 SMALL_CONTEXT_OF_MANY = 1024
+SMALL_USES_FOR_A_PLACE = 3          # of a shape without a graph while all places of small steps are taken
 
 
 class _GraphEntry:
@@ -138,6 +139,7 @@ class ModelRunner:
         # captured decode steps by (padded batch, bucket of contexts), least recently used first; at most
         # cfg.max_graphs of them are kept
         self._graphs = OrderedDict()
+        self._small_uses = OrderedDict()    # small shapes that have no place among them: how often they were asked for
         self._graph_pool = None
         # the fp32 logits of every graph-replayed step: one buffer for all graphs (they never run side
         # by side), made at the first such step
@@ -202,20 +204,48 @@ class ModelRunner:
     # -- steps replayed from HIP graphs ---------------------------------------------------------------
     def _graph_entry(self, key, make):
         """The entry of a captured shape, made by `make()` if it is new; the most recently used
-        entries are kept, up to cfg.max_graphs."""
+        entries are kept, up to cfg.max_graphs: those of small steps up to their share, and they make room first."""
         entry = self._graphs.get(key)
         if entry is not None:
             self._graphs.move_to_end(key)
             return entry
+        if key[0] == "small":
+            self._small_uses.pop(key, None)
+            while len(self._small_keys()) >= self._small_share():
+                self._drop_graph(self._small_keys()[0])
         while len(self._graphs) >= max(1, int(self.cfg.max_graphs)):
-            # the least recently used shape goes: its graph, index buffers and pinned staging memory
-            # (a copy out of that memory may still run: wait for it)
-            _, old = self._graphs.popitem(last=False)
-            old.copied.synchronize()
-            torch.cuda.current_stream().synchronize()
-            old.graph = None
+            self._drop_graph((self._small_keys() or list(self._graphs))[0])
         entry = self._graphs[key] = make()
         return entry
+
+    def _drop_graph(self, key) -> None:
+        """Give back a shape's graph, index buffers and pinned staging memory (a copy out of that memory may still run: wait
+        for it)."""
+        old = self._graphs.pop(key)
+        old.copied.synchronize()
+        torch.cuda.current_stream().synchronize()
+        old.graph = None
+
+    def _small_keys(self) -> List[tuple]:
+        """The kept shapes of small steps, the least recently used first."""
+        return [k for k in self._graphs if k[0] == "small"]
+
+    def _small_share(self) -> int:
+        return max(1, int(self.cfg.max_graphs) // 4)
+
+    def _small_place(self, key) -> bool:
+        """Whether a small shape that has no graph may have one.  There are many such shapes, each used now and then: up
+        to a quarter of the kept graphs, in places that nothing else holds, and one that has none in the place of the least
+        recently used one once it has been asked for SMALL_USES_FOR_A_PLACE times (so that rare shapes do not take turns)."""
+        held = len(self._small_keys())
+        if held < self._small_share() and len(self._graphs) < int(self.cfg.max_graphs):
+            return True
+        if held == 0:
+            return False
+        uses = self._small_uses[key] = self._small_uses.pop(key, 0) + 1
+        if len(self._small_uses) > 4 * self._small_share():
+            self._small_uses.popitem(last=False)
+        return uses >= SMALL_USES_FOR_A_PLACE
 
     def _run_then_capture(self, entry, run):
         """Run a shape's step kernel by kernel; from its second run on (every library is loaded and
@@ -358,8 +388,8 @@ class ModelRunner:
         if longest > limit or longest > most_keys:   # (beyond the context limit: an error below; the inert portion must fit, too)
             return None
         bucket = min(bucket, limit)
-        # (many shapes, each used now and then: they take free places among the kept graphs, not those of decode steps)
-        if ("small", t_pad, b_pad, bucket) not in self._graphs and len(self._graphs) >= int(self.cfg.max_graphs):
+        key = ("small", t_pad, b_pad, bucket)
+        if key not in self._graphs and not self._small_place(key):
             return None
         return t_pad, b_pad, -(-bucket // self.cfg.page_size), bucket
 

@@ -463,7 +463,7 @@ def test_which_small_steps_are_padded_and_replayed():
     def shape(portions, dtype=None, state=False, graphs=(), limit=4096):
         r = NS(_use_graphs=True, _has_state=state, rt=NS(dtype=dtype or torch.bfloat16), _graphs={k: None for k in graphs},
                cache=Cache({i: c for i, (c, _, _) in enumerate(portions)}),
-               cfg=NS(max_pages_per_request=limit // 16, page_size=16, max_graphs=64))
+               cfg=NS(max_pages_per_request=limit // 16, page_size=16, max_graphs=64), _small_place=lambda key: True)
         got = rn.ModelRunner._small_shape(r, [Segment(i, [1] * n, w) for i, (_, n, w) in enumerate(portions)])
         return got and got[:2] + got[3:]
     one = [0]

@@ -595,3 +595,59 @@ def test_small_steps_of_every_design_padded_captured_and_replayed(name):
         # a close call may take another expert, which the middle one of the rows' distances does not see
         off = ((got - want).norm(dim=-1) / want.norm(dim=-1)).median().item()
         assert off < 0.05, f"{name}: step {i}: {off:.3f}"
+
+
+def test_graphs_of_small_steps_keep_to_their_share(tmp_path):
+    """Of eight kept graphs two are of small steps: further small shapes run kernel by kernel and take the place of the least
+    recently used one once they come often; decode shapes push out small ones and never each other while there are any."""
+    from serve_amd.config.engine import EngineConfig
+    from serve_amd.engine.batch import Segment
+    from serve_amd.engine.engine import Engine
+    folder = util.make_folder(tmp_path, "A")
+    eng = Engine.from_folder(folder, EngineConfig(dtype="bfloat16", page_size=4, num_pages=512, max_context=64, max_requests=64,
+                                                  max_graphs=8))
+    tokens = util.random_tokens(random.Random(9), 64, 256)
+    want = util.plain_logits(folder, tokens)
+    graphs = eng.runner._graphs
+
+    def prompts(*lengths):
+        ids = list(range(len(lengths)))
+        for i in ids:
+            assert eng.runner.admit(i)
+        got = eng.step([Segment(i, tokens[:n], [n - 1]) for i, n in zip(ids, lengths)]).cpu().double()
+        util.assert_close(got, torch.stack([want[n - 1] for n in lengths]), "bfloat16", f"{lengths}")
+        for i in ids:
+            eng.runner.release(i)
+
+    def decode(count):
+        for i in range(count):
+            assert eng.runner.admit(i)
+        got = eng.step([Segment(i, tokens[:1], [0]) for i in range(count)]).cpu().double()
+        util.assert_close(got, want[:1].expand(count, -1), "bfloat16", f"{count} single tokens")
+        for i in range(count):
+            eng.runner.release(i)
+    small = lambda: [k[1:3] for k in graphs if k[0] == "small"]        # noqa: E731
+    for _ in range(3):
+        prompts(7)
+        prompts(20)
+    assert small() == [(16, 2), (32, 2)]
+    for uses in (1, 2, 3):                       # a third shape: a place at its third use
+        assert small() == [(16, 2), (32, 2)]
+        prompts(40)
+    assert small() == [(32, 2), (64, 2)]
+    prompts(5, 6, 7)                             # a fourth, once: kernel by kernel
+    prompts(20)
+    assert small() == [(64, 2), (32, 2)] and graphs[("small", 32, 2, 64)].graph is not None
+    counts = (1, 2, 3, 5, 9, 17, 33, 49)
+    for n in counts[:6]:
+        decode(n)
+    assert len(small()) == 2 and len(graphs) == 8
+    kept = [k for k in graphs if k[0] != "small"]
+    decode(counts[6])                            # a seventh decode shape takes the place of a small one
+    assert len(small()) == 1 and all(k in graphs for k in kept) and len(graphs) == 8
+    prompts(40)                                  # (the shape that lost its place takes no other's)
+    assert len(small()) == 1 and all(k in graphs for k in kept)
+    kept = [k for k in graphs if k[0] != "small"]
+    for n in counts[:7]:
+        decode(n)
+    assert [k for k in graphs if k[0] != "small"] == kept and len(small()) == 1
