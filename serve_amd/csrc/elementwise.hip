@@ -132,8 +132,10 @@ __device__ __forceinline__ void store4(bf16_t* p, float4 v) {
 // of 2,048 with four parts 3.22 / 2.59, of 4,096 4.12 / 3.12; 64 rows of 4,096 in bf16 4.18 / 3.02 (a fifth of a microsecond of it
 // through the sums over a wave, see common.h);
 // 2,048 rows of 2,048 in bf16 9.6 / 8.2, of 4,096 18.9 / 16.7 (5.0 TB/s).
+// (Four groups and more are workgroups of 256 threads, and may so have more than 128 registers: eight groups of two parts
+// with float32 weights take 138.)
 template <typename TA, typename TD, typename TW, int PMAX, int NK>
-__global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(float* __restrict__ x, const TD* __restrict__ delta,
+__global__ __launch_bounds__(NK <= 2 ? 1024 : 256) void add_rmsnorm_vec_kernel(float* __restrict__ x, const TD* __restrict__ delta,
                                                                int parts, size_t part_stride,
                                                                const TW* __restrict__ w, TA* __restrict__ y,
                                                                const int* __restrict__ rows,
@@ -193,7 +195,7 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_vec_kernel(float* __restrict
 }
 
 // Threads and groups a thread: few rows, and rows of three partial sums and more, take as many threads as there are groups
-// (up to 1,024), many rows workgroups of 256.
+// (up to 1,024; at most two groups a thread), many rows workgroups of 256.
 template <typename TA, typename TD, typename TW>
 static void launch_add_rmsnorm_vec(float* x, const void* delta, int parts, size_t part_stride, const void* w, void* y,
                                    const int* rows, const float* after, float eps, int R, int d, hipStream_t stream) {
