@@ -911,9 +911,12 @@ static bool takes_wide(int M, int N, int K, int parts) {
   if (M > 192) return false;
   // the head: from 48 rows, from one row with a long walk along K, and from 8 rows over a vocabulary of 64 K
   // rows and more, which takes 256 weight rows a workgroup (see pick_wide)
-  // (between the two, matrices of which 32 rows a workgroup are one round of the chip stay with gemm_mid_kernel up to 64
-  // rows of A: 12.7 / 14.6 at 64 with 8,192 rows of W)
-  if (N >= 8192 && K < 3072 && M <= 64 && N <= 32 * compute_units()) return false;
+  // Matrices of which 32 rows a workgroup are one round of the chip at most stay with gemm_mid_kernel up to 64 rows of A, which
+  // takes 32 there; K 2048, gemm_mid_kernel / this one at 48 and 64 rows of A: 6,144 rows of W 10.7 / 13.1 and 12.0 / 14.3,
+  // 7,168 11.0 / 13.3 and 12.2 / 14.5, 8,192 11.4 / 13.5 and 12.5 / 14.6, but 8,256 14.7 / 13.6 and 16.5 / 14.7, 12,288 17.2 /
+  // 16.2 and 17.3 / 15.9, 16,384 17.9 / 18.1 and 19.8 / 18.7; K 1024 8,192 rows 7.4 / 8.8 and 8.5 / 9.6, 8,256 9.8 / 9.0 and 11.4 /
+  // 9.9; K 2560 14.1 / 17.6 and 15.8 / 19.1, 19.6 / 17.8 and 21.8 / 19.2.
+  if (parts == 1 && K < 3072 && M <= 64 && N <= 32 * compute_units()) return false;
   if (N >= 8192) return parts == 1 && M <= 128 && (K >= 3072 || M >= 48 || (N >= 65536 && M >= 8));
   // narrow matrices: a walk of twelve stages and more, and enough parts to give half the compute units a
   // workgroup; from three rows on for matrices of 24 M elements and more, above 32 rows for smaller ones

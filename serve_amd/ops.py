@@ -1665,7 +1665,9 @@ def split_k_parts(M: int, N: int, K: int) -> int:
     over the chip allows, slices of at least twelve stages of 64 columns.  Else, for one or two rows, a
     workgroup takes 16 weight rows (about four workgroups per compute unit wanted, slices of at least
     256); from three rows on it takes 32 (one workgroup per compute unit wanted, slices of at least 512)."""
-    if N >= 8192:
+    # (beyond 32 rows of A the last group of 64 weight rows before 8,192 counts as them: K 2048, 8,150 of them at 64 rows 12.5
+    # us whole, 15.5 in two parts)
+    if N >= 8192 or (M > 32 and N > 8192 - 64):
         return 1
     cus = compute_units()
     if M <= WIDE_MAX_ROWS and K % 64 == 0:

@@ -787,6 +787,23 @@ def test_prompt_attention_long_prompts_windows_and_split_keys(Hq, Hk, D, ps):
     attention_case("bfloat16", Hq, Hk, D, ps, [(3100, 200)], seed=514 + D, kernel="dispatch", splits=1)
 
 
+def test_gemm_bf16_one_round_of_workgroups_is_one_kernel():
+    """Which kernel takes a product does not change within one round of the chip (32 weight rows a workgroup), and the results
+    are right on both sides of where it does."""
+    from serve_amd import ops
+    last = 32 * ops.compute_units()
+    wide = ops.gemm_takes_wide
+    for M in (33, 48, 64):
+        assert not any(wide(M, N, 2048) for N in (last - 1024, last - 63, last - 1, last))
+    assert wide(48, last + 1, 2048) and wide(65, last, 2048) and wide(48, last, 3072)
+    for N in (last - 1, last, last + 1):
+        a, w = rnd((48, 832), torch.bfloat16, 10), rnd((N, 832), torch.bfloat16, 11, 0.1)
+        out = torch.full((48, N), float("nan"), device=DEV)
+        ops.gemm_bf16_skinny(a, w, out)
+        # (as below)
+        torch.testing.assert_close(out.double(), a.double() @ w.double().T, atol=2e-6 * 832 ** 0.5, rtol=1e-5)
+
+
 @pytest.mark.parametrize("c_dt", ["bfloat16", "float32"])
 @pytest.mark.parametrize("M", [1, 9, 17, 33, 48, 64, 65])
 @pytest.mark.parametrize("N,K", [(8192, 2048), (8190, 264), (8193, 520), (16384, 1024), (16379, 136), (16385, 520)])
