@@ -681,12 +681,12 @@ extern "C" int sa_gemm_f32_mid_parts(const void* A, const void* W, void* C, int 
 }
 
 // Rows of A whose planes are held at a time: whole tiles of 128, at most a quarter of a gigabyte (what the chip's last
-// cache holds; a product of more rows goes in runs of so many).
+// cache holds; a product of more rows goes in runs of so many).  0: not even one tile of rows this long.
 static int plane_rows(int M, int K) {
   const long long bytes = ((long long)K + 63) / 64 * 64 * 6;                 // of a row
   const long long run = (256LL << 20) / bytes / 128 * 128;
   const long long all = ((long long)M + 127) / 128 * 128;
-  return (int)(run < 128 ? 128 : run < all ? run : all);
+  return (int)(run < all ? run : all);
 }
 
 // ... and behind them the largest sizes of their pieces of 32 rows by 64 columns.
@@ -698,7 +698,7 @@ extern "C" long long sa_gemm_f32_split_bytes(int M, int K) {
 
 // C fp32 [parts, M, N] (1 to 8 parts of K, which the consumer adds in order); `planes`: sa_gemm_f32_split_bytes of
 // scratch memory; the last `tail` rows (0 to 128, fewer than M) go through the kernel of few rows.  Needs K % 4 == 0 and
-// 16-byte aligned A, W and planes.
+// 16-byte aligned A, W and planes.  Rows of more than 349,504 columns all go there, 128 at a time, without scratch memory.
 extern "C" int sa_gemm_f32_split(const void* A, const void* W, void* C, void* planes, int M, int N, int K, int parts, int tail,
                                  hipStream_t stream) {
   if (M <= 0 || N <= 0) return 0;
@@ -708,8 +708,16 @@ extern "C" int sa_gemm_f32_split(const void* A, const void* W, void* C, void* pl
   const int quads = (K + 63) / 64;
   const int run = plane_rows(M, K);
   float* most = (float*)((char*)planes + plane_bytes(M, K));
+  if (run == 0) {
+    for (int row0 = 0; row0 < M; row0 += 128) {
+      const int rc = few_rows((const float*)A + (size_t)row0 * K, W, (float*)C + (size_t)row0 * N, M - row0 < 128 ? M - row0 : 128,
+                              N, K, parts, (size_t)M * N, stream);
+      if (rc != 0) return rc;
+    }
+    return 0;
+  }
   const long long ntiles = ((long long)N + SP_BN - 1) / SP_BN;
-  if ((run / 64) * ntiles > 0x7fffffffLL || quads > 65535) return SA_ERR_ARG;
+  if ((run / 64) * ntiles > 0x7fffffffLL) return SA_ERR_ARG;
   const int tiled = M - tail;
   for (long long row0 = 0; row0 < tiled; row0 += run) {
     const int rows = (int)(tiled - row0 < run ? tiled - row0 : run);

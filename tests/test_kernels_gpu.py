@@ -231,6 +231,19 @@ def test_gemm_f32_by_split_operands_over_the_range_of_floats(M, N, K, parts, ea,
         assert (got[1] == 0).all() and (got[:, 2] == 0).all()
 
 
+@pytest.mark.parametrize("M,N,K,parts", [(129, 2, 349508, 1), (300, 3, 349568, 2), (129, 2, 4194304, 1)])
+def test_gemm_f32_by_split_operands_of_very_long_rows(M, N, K, parts):
+    """Inner sizes of which not even a tile of rows has room in the scratch memory, and beyond what its grid can count."""
+    from serve_amd import ops
+    a, w = torch.randn((M, K), device=DEV), torch.randn((N, K), device=DEV)
+    out = torch.full((parts, M, N), float("nan"), dtype=torch.float32, device=DEV)
+    ops.gemm_f32_split(a, w, out)
+    want = torch.stack([(a * 1.0).double() @ v.double() for v in w], 1)
+    # normal operands: sums of K products in runs of at most 2,048 columns a wave, and of the runs, are off by a few roundings
+    # of their size, about K^0.5 (8 sigma of 2^-24 times the root of the number of runs)
+    assert ((out.double().sum(0) - want).abs() <= 8 * K ** 0.5 * 2.0 ** -24 * max(8, (K / 2048) ** 0.5)).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(24, 1024, 2048), (64, 512, 8192), (100, 512, 8192), (300, 512, 2048), (300, 256, 14336)])
 @pytest.mark.parametrize("signs", [True, False])
 def test_gemm_f32_by_split_operands_is_as_close_as_sums_in_two_levels(M, N, K, signs):
