@@ -542,6 +542,15 @@ def test_paged_attention_tiled_f32_window_standout_and_poison():
                    kernel="tiled")
 
 
+@pytest.mark.parametrize("Hq,Hk,D,ps", [(8, 2, 64, 16), (4, 4, 128, 16), (3, 1, 80, 12)])
+def test_prompt_attention_of_windows_at_the_end_of_long_contexts(Hq, Hk, D, ps):
+    """Masks that reach back so far that a portion reads at most 512 keys, of contexts of thousands: the shape for short
+    contexts, whose first stage then begins anywhere in the context."""
+    segs = [(3000, 60), (900, 17), (4095, 64), (511, 2)]
+    attention_case("bfloat16", Hq, Hk, D, ps, segs, seed=540 + D, kernel="dispatch", window=100, poison=True)
+    attention_case("bfloat16", Hq, Hk, D, ps, segs, seed=541 + D, kernel="dispatch", window=449, poison=True)
+
+
 @pytest.mark.parametrize("Hq,Hk,D,ps", [(1, 1, 16, 4), (4, 2, 64, 16), (3, 1, 80, 12), (8, 2, 128, 64)])
 def test_paged_attention_tiled_f32_at_the_edges_of_tiles(Hq, Hk, D, ps):
     """Rows and keys around the tiles of 16 and 64: contexts that end one before, at and one after a block, alone and behind
