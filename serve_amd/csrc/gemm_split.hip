@@ -403,7 +403,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
 
 // ---------------------------------------------------------------------------------------------
 // Up to 128 rows (decode steps of the 32-bit path): the work is reading W, once.  A workgroup of eight waves owns 32 NT
-// rows of W and all rows of A (MT tiles of 32).  A stage is 128 / NT columns of both (a row of it is 512 / NT bytes),
+// rows of W and MT tiles of 32 rows of A (gridDim.y runs of them; which, see few_rows).  A stage is 128 / NT columns of both (a row of it is 512 / NT bytes),
 // loaded straight into LDS, a kilobyte an instruction, in a ring of NB stages: no registers hold what is on its way.
 // Wave = (tile of W wt, run of 16 columns kc): it reads its fragments (lane l: row l % 32, eight columns from 8 (l / 32)),
 // splits them and multiplies; the waves of a tile add their sums through LDS at the end, in order.  Segment s (16 bytes)
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
 // 1.4e-7 at 64 and 100; operands in 1 .. 2: 0.97e-7 / 0.48e-7 and 0.68e-7, 0.88e-7 / 0.56e-7.
 // From five rows, with K in parts: level with the kernel of few rows of csrc/gemm.hip over 3,072 and 2,048 rows of W at K 2048
 // (9.3 and 8.2 us there, 9.9 and 8.1 here), 21.3 / 18.6 over 2,048 at K 8192.  Up to 128 rows, which is what a stage has room
-// for: at 128 the tiles above take 20, 87 (16,384 rows of W) and 51 us where this takes 17, 67 and 38, and only over
+// for: at 128 the tiles above take 20, 87 (16,384 rows of W) and 51 us where this takes 15, 64 and 37, and only over
 // 128,256 rows of W 366 for 550.
 // ---------------------------------------------------------------------------------------------
 template <int MT, int NT>
@@ -469,7 +469,7 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wt = wave % NT, kc = wave / NT;
   const int r = lane & 31, h = lane >> 5;
-  const int n0 = blockIdx.x * 32 * NT;
+  const int n0 = blockIdx.x * 32 * NT, m0 = blockIdx.y * 32 * MT;
   const int all = (K + COLS - 1) / COLS;
   const int s_begin = (int)((long long)blockIdx.z * all / gridDim.z);
   const int n = (int)((long long)(blockIdx.z + 1) * all / gridDim.z) - s_begin;
@@ -482,7 +482,7 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   for (int d = 0; d < ND; ++d) {
     const int row = (wave * ND + d) * RPI + lane / SEGS;
     const int seg = (lane % SEGS) ^ (row & 15);
-    src[d] = row < 32 * NT ? W + (size_t)min(n0 + row, N - 1) * K : A + (size_t)min(row - 32 * NT, M - 1) * K;
+    src[d] = row < 32 * NT ? W + (size_t)min(n0 + row, N - 1) * K : A + (size_t)min(m0 + row - 32 * NT, M - 1) * K;
     col[d] = seg * 4;
   }
   auto fetch = [&](int s) __attribute__((always_inline)) {    // (past the last stage it is loaded again, and not read)
@@ -593,7 +593,7 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   bool small = false, odd = false;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
-    const int m = mt * 32 + r;
+    const int m = m0 + mt * 32 + r;
 #pragma unroll
     for (int e4 = 0; e4 < 4; ++e4) {
       float v[4];
@@ -625,10 +625,10 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   const bool any_small = __any(small);
   if (!any_small && !__any(odd)) return;
   const int k_begin = s_begin * COLS, k_end = min(K, (s_begin + n) * COLS);
-  const float below = any_small && small_operands(A, 0, 32 * MT, M, W, n0 + wt * 32, 32, N, K, k_begin, k_end) ? limit : -1.f;
+  const float below = any_small && small_operands(A, m0, 32 * MT, M, W, n0 + wt * 32, 32, N, K, k_begin, k_end) ? limit : -1.f;
   if (!odd && !(small && below >= 0.f)) return;
   for (int x = 0; x < MT * 16; ++x) {
-    const int m = (x >> 4) * 32 + r, cn = n0 + wt * 32 + ((x & 15) >> 2) * 8 + h * 4 + (x & 3);
+    const int m = m0 + (x >> 4) * 32 + r, cn = n0 + wt * 32 + ((x & 15) >> 2) * 8 + h * 4 + (x & 3);
     if (m < M && cn < N) redo(A, W, C, m, cn, N, K, k_begin, k_end, below);
   }
 }
@@ -647,25 +647,29 @@ static int launch_f32_wide(const void* A, const void* W, void* C, int M, int N, 
     if (e != hipSuccess) return (int)e;
     if (dev >= 0 && dev < 64) sized[dev] = true;
   }
-  hipLaunchKernelGGL((gemm_f32_wide_kernel<MT, NT, NB>), dim3((N + 32 * NT - 1) / (32 * NT), 1, parts), dim3(512), lds,
+  hipLaunchKernelGGL((gemm_f32_wide_kernel<MT, NT, NB>), dim3((N + 32 * NT - 1) / (32 * NT), (M + 32 * MT - 1) / (32 * MT), parts), dim3(512), lds,
                      stream, (const float*)A, (const float*)W, (float*)C, M, N, K, part_stride);
   SA_LAUNCH_CHECK();
   return 0;
 }
 
+// Up to 128 rows.  What a workgroup takes: 32 rows of A and 32 of W where that is one round of the chip at most, 32 and 64
+// over slices of up to 1,024 columns, 64 and 32, and only then all rows of A, so that W is read once.  One round costs
+// by what a workgroup does alone, so the smallest ones that still are one round win: K 2048, 100 rows, all rows of A a
+// workgroup / so, us: 512 rows of W 55.7 / 14.9, 3,072 57 / 22, 512 in eight parts 14.4 / 7.4, 8,192 57 / 37.5 (64 and 64); 64 rows
+// over 512 21.4 / 14.8; K 256, 100 rows, 2,048 of W 14.1 / 6.3.  Beyond one round W counts: 16,384 rows of it, 128 of A, 64 with
+// all and 78 with 64 a workgroup, in 8,192 in two parts 37 and 43.
 static int few_rows(const void* A, const void* W, void* C, int M, int N, int K, int parts, size_t part_stride, hipStream_t stream) {
-  // (four tiles of A have no registers for sums in two levels: over a long inner size twice two of them)
-  if (M > 96 && K / parts > 4096) {
-    const int rc = few_rows(A, W, C, 64, N, K, parts, part_stride, stream);
-    return rc != 0 ? rc : few_rows((const float*)A + (size_t)64 * K, W, (float*)C + (size_t)64 * N, M - 64, N, K, parts, part_stride, stream);
-  }
-  // 64 rows of W a workgroup, or 32 where those would leave half of the chip idle (up to 64 rows of A: LDS)
-  if (M <= 64 && (long long)((N + 63) / 64) * parts <= compute_units() / 2) {
-    if (M <= 32) return launch_f32_wide<1, 1, 3>(A, W, C, M, N, K, parts, part_stride, stream);
-    return launch_f32_wide<2, 1, 3>(A, W, C, M, N, K, parts, part_stride, stream);
-  }
+  const long long cus = compute_units();
+  const long long w32 = (long long)((N + 31) / 32) * parts, w64 = (long long)((N + 63) / 64) * parts;
+  const int a32 = (M + 31) / 32, a64 = (M + 63) / 64;
+  if (w32 * a32 <= cus) return launch_f32_wide<1, 1, 3>(A, W, C, M, N, K, parts, part_stride, stream);
+  if (w64 * a32 <= cus && K / parts <= 1024) return launch_f32_wide<1, 2, 3>(A, W, C, M, N, K, parts, part_stride, stream);
+  if (w32 * a64 <= cus) return launch_f32_wide<2, 1, 3>(A, W, C, M, N, K, parts, part_stride, stream);
   if (M <= 32) return launch_f32_wide<1, 2, 3>(A, W, C, M, N, K, parts, part_stride, stream);
-  if (M <= 64) return launch_f32_wide<2, 2, 3>(A, W, C, M, N, K, parts, part_stride, stream);
+  // (four tiles of A have no registers for sums in two levels: not over a long inner size)
+  if (M <= 64 || w64 * a64 <= cus || (M > 96 && K / parts > 4096))
+    return launch_f32_wide<2, 2, 3>(A, W, C, M, N, K, parts, part_stride, stream);
   if (M <= 96) return launch_f32_wide<3, 2, 2>(A, W, C, M, N, K, parts, part_stride, stream);
   return launch_f32_wide<4, 2, 2>(A, W, C, M, N, K, parts, part_stride, stream);
 }

@@ -163,6 +163,31 @@ def test_gemm_f32_by_split_operands(M, N, K, parts):
     assert torch.equal(got[0].sign(), want[0].sign()) and torch.equal(got[4].sign(), want[4].sign())
 
 
+# (256 compute units)  32 x 32 rows a workgroup; 32 x 64; 64 x 32; 64 x 64 in two runs, the same over a long inner size; all rows
+@pytest.mark.parametrize("M,N,K,parts", [(65, 70, 260, 2), (128, 2048, 36, 1), (100, 2100, 260, 1), (97, 2049, 1024, 1), (128, 2100, 1100, 1),
+                                         (65, 4096, 2052, 2), (100, 4200, 260, 1), (97, 8200, 4100, 1), (70, 8300, 132, 1), (100, 8300, 132, 1)])
+def test_gemm_f32_of_few_rows_in_runs(M, N, K, parts):
+    """Rows of A in runs of 32 and 64 a workgroup: ordinary rows, rows of zeros, very small ones beside a very large one of W, and
+    infinities, in every run."""
+    from serve_amd import ops
+    a, w = rnd((M, K), torch.float32, 53), rnd((N, K), torch.float32, 54, 0.1)
+    a[33], a[M - 1] = 0, a[M - 1] * 2.0 ** -110
+    a[40] *= 2.0 ** -127
+    w[5] *= 2.0 ** 100
+    out = torch.full((parts, M, N), float("nan"), dtype=torch.float32, device=DEV)
+    ops.gemm_f32_mid_parts(a, w, out)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    got = out.double().sum(0)
+    # (as above)
+    assert ((got - want).abs() <= size * (2.0 ** -23 + (6 * (K // 16 + 1) + 16) * 2.0 ** -24) + parts * 2.0 ** -149).all()
+    assert (got[33] == 0).all()
+    a[0, 1], a[M - 1, K - 1] = float("inf"), -float("inf")
+    ops.gemm_f32_mid_parts(a, w, out)
+    want, got = a.double() @ w.double().T, out.double().sum(0)
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and not torch.isnan(got).any()
+    assert torch.equal(got[0].sign(), want[0].sign()) and torch.equal(got[M - 1].sign(), want[M - 1].sign())
+
+
 @pytest.mark.parametrize("M,N,K,parts", [(129, 70, 36, 1), (161, 64, 260, 2), (257, 200, 132, 3), (319, 129, 68, 1), (383, 4100, 64, 1)])
 def test_gemm_f32_by_split_operands_with_the_end_cut_off(monkeypatch, M, N, K, parts):
     """The rows behind the last whole tile through the kernel of few rows: the same sums as of those rows alone, in every
