@@ -7,7 +7,7 @@
 //
 // Three kernels: gemm_nt_rows_kernel for up to 8 rows of float32 throughout (more are gemm_split.hip's, and from five on),
 // gemm_nt_mfma32_kernel (the matrix cores' float32 instruction, 128 x 128 tiles) for mixed storage with rows whose
-// length is a multiple of four, and gemm_nt_kernel for everything else: a 256-thread block owns a 64x64 tile of C; K
+// length is a multiple of four and for many short ones of float32 (ops.f32_short), and gemm_nt_kernel for everything else: a 256-thread block owns a 64x64 tile of C; K
 // advances in slices of 16 through LDS; each thread accumulates a 4x4 sub-tile with v_fma_f32.  Every edge (M,
 // N, K not multiples of the tile) is guarded, so any size is accepted.
 #include "common.h"
@@ -347,12 +347,7 @@ extern "C" int sa_gemm_nt(const void* A, int a_dtype, const void* W, int w_dtype
   } while (0)
   const int code = a_dtype * 4 + w_dtype * 2 + c_dtype;
   switch (code) {
-    case 0:                         // (what is aligned and has rows of whole fours goes to gemm_split.hip)
-      grid = dim3((N + GT_N - 1) / GT_N, (M + GT_M - 1) / GT_M);
-      if (grid.y > 65535) return SA_ERR_ARG;
-      hipLaunchKernelGGL((gemm_nt_kernel<float, float, float>), grid, block, 0, stream, (const float*)A, (const float*)W,
-                         (float*)C, M, N, K);
-      break;
+    case 0: GO(float, float, float); break;      // (aligned rows of whole fours that are not short go to gemm_split.hip)
     case 1: GO(float, float, bf16_t); break;
     case 2: GO(float, bf16_t, float); break;
     case 3: GO(float, bf16_t, bf16_t); break;

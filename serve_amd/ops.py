@@ -161,7 +161,7 @@ def gemm_nt(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor
     _check(w.shape[1] == K, f"gemm: inner sizes differ ({K} vs {w.shape[1]})")
     _check(out.shape == (M, N), f"gemm: output must be [{M}, {N}]")
     if out.dtype == torch.float32:
-        if gemm_f32_split_available(a, w):
+        if gemm_f32_split_available(a, w) and not f32_short(M, N, K):
             return gemm_f32_split(a, w, out)
         # (5 to 8 rows of a narrow matrix leave most of the chip without a workgroup there: 9.7 us with the kernel of few
         # rows, 15.4 with this one, over 3,072 rows of W at K 2048, 21.6 and 45.2 over 2,048 at K 8192; level over 16,384 at
@@ -177,6 +177,16 @@ def gemm_nt(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor) -> torch.Tensor
 
 # from this many rows on, products of float32 take the bf16 matrix cores, every float split into three bf16 numbers
 F32_SPLIT_MIN_ROWS = 129
+
+
+def f32_short(M: int, N: int, K: int) -> bool:
+    """Whether so many rows are too short for a launch of their own that splits them, and take the matrix cores' float32
+    instruction in one launch (csrc/gemm.hip).  That / the split product, which counts in 64 columns, in us: K 16, 300 rows over
+    1,024 of W 5.9 / 9.9, 4,096 over 4,096 18 / 33; K 64 12.4 / 16.0 (2,048 over 2,048) and 32 / 35, but 57 / 55 (4,096 over 8,192);
+    K 96 12.0 / 11.3 (300 over 256), 13.7 / 16.2 (700 over 3,072) and 138 / 152 (4,096 over 16,384); K 128 14.5 / 11.5 and 49 / 46."""
+    if K <= 64:
+        return K <= 32 or M * N < 1 << 25
+    return K < 128 and M * N >= 1 << 21
 
 
 def gemm_f32_split_available(a: torch.Tensor, w: torch.Tensor) -> bool:

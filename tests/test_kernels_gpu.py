@@ -188,6 +188,30 @@ def test_gemm_f32_of_few_rows_in_runs(M, N, K, parts):
     assert torch.equal(got[0].sign(), want[0].sign()) and torch.equal(got[M - 1].sign(), want[M - 1].sign())
 
 
+@pytest.mark.parametrize("M,N,K", [(129, 1, 4), (300, 130, 16), (257, 1030, 32), (130, 70, 60), (513, 4100, 96), (130, 70, 96)])
+def test_gemm_f32_of_short_rows(monkeypatch, M, N, K):
+    """Many rows of few columns in one launch, which kernel on both sides of the line, and what is not finite."""
+    from serve_amd import ops
+    short = ops.f32_short
+    assert short(129, 8, 32) and short(4096, 16384, 32) and short(2048, 2048, 64) and not short(8192, 4096, 64)
+    assert not short(300, 256, 68) and short(700, 3072, 124) and not short(4096, 16384, 128)
+    calls = []
+    split = ops.gemm_f32_split
+    monkeypatch.setattr(ops, "gemm_f32_split", lambda *x: calls.append(0) or split(*x))
+    a, w = rnd((M, K), torch.float32, 55), rnd((N, K), torch.float32, 56, 0.1)
+    a[1] = 0
+    out = torch.full((M, N), float("nan"), dtype=torch.float32, device=DEV)
+    ops.gemm_nt(a, w, out)
+    assert bool(calls) != short(M, N, K)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    # (a rounding of a running sum, at most `size`, for every two columns at most, and 2^-24 of every product)
+    assert ((out.double() - want).abs() <= size * (K / 2 + 2) * 2.0 ** -24).all() and (out[1] == 0).all()
+    a[0, K // 2], a[3, 0] = float("inf"), float("nan")
+    ops.gemm_nt(a, w, out)
+    want = a.double() @ w.double().T
+    assert torch.equal(torch.isnan(out), torch.isnan(want)) and torch.equal(torch.isinf(out), torch.isinf(want))
+
+
 @pytest.mark.parametrize("M,N,K,parts", [(129, 70, 36, 1), (161, 64, 260, 2), (257, 200, 132, 3), (319, 129, 68, 1), (383, 4100, 64, 1)])
 def test_gemm_f32_by_split_operands_with_the_end_cut_off(monkeypatch, M, N, K, parts):
     """The rows behind the last whole tile through the kernel of few rows: the same sums as of those rows alone, in every
