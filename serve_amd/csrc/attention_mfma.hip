@@ -1116,8 +1116,14 @@ extern "C" int sa_attention_mfma_head_dim() { return HD; }
 // 10.2 / 6.1, 256 10.7 / 9.5, 512 13.7 / 13.6, 1024 20.2 / 22.6; 24 ragged ones up to 256 56.2 / 22.4, 8 of 256
 // 20.1 / 13.9, 4 of 512 22.7 / 20.7, 64 of 33 35.4 / 14.7, 8 ragged ones up to 512 41.7 / 21.9; portions of 100 tokens,
 // ten over contexts of 300 26.7 / 18.9, two over 900 18.7 / 21.9; heads of 128: 24 ragged ones up to 256 69.6 / 35.8, 4 of
-// 512 32.1 / 32.4, 2 of 1024 41.4 / 49.3.  512 is where the two meet, for both.
+// 512 32.1 / 32.4, 2 of 1024 41.4 / 49.3.  512 is where the two meet, for both, where the rows fill the chip.
+// A step of at most one workgroup a compute unit takes what one workgroup takes, and there four waves one after the other over
+// all keys lose sooner: one portion of 100 tokens, 400 keys / 500 in all, heads of 64 14.1 / 13.7 and 14.1 / 14.7, of 128 20.4 / 19.6
+// and 20.1 / 21.1, of 96 (padded in LDS) 16.0 / 16.1 and 15.7 / 17.6, of 16 9.4 / 10.7 and 9.3 / 11.3; 20 tokens over 490 keys
+// 13.4 / 13.8, 18.8 / 19.8, 15.1 / 16.6, 7.9 / 10.7; one prompt of 300 tokens 14.4 / 11.5, 18.4 / 16.9, 14.1 / 13.5, 9.4 / 8.7; 16 tokens
+// whose mask reaches back 256 keys of 3,000, a range that begins anywhere in a stage, 13.1 / 13.4, 17.2 / 18.6, 13.1 / 15.8, 8.5 / 11.0.
 constexpr int LIGHT_MAX_CTX = 512;
+constexpr int LIGHT_MAX_CTX_OF_FEW = HD == 64 ? 416 : 320;
 
 // A step whose segments have at most 16 rows each (single decoded tokens) takes the one-wave kernel,
 // any other the prompt kernel.  `in_workgroup` (such steps only, num_splits 1): the key range of every
@@ -1178,7 +1184,11 @@ extern "C" int sa_paged_attention_mfma(const void* q, int q_stride, void* out, c
     // compute units, a workgroup takes row groups w and last - w: under the causal mask the two
     // together are one full context long, so all finish at about the same time.
     const long long rows = (long long)max_q_len * G;
-    const bool light = max_ctx_len > 0 && max_ctx_len <= LIGHT_MAX_CTX;
+    const int reach = window > 0 ? window : chunk;                 // (one row's; a tile's rows have more, and not whole stages)
+    const int walk = reach > 0 ? min(reach + 128 / G, max_ctx_len) + 64 : max_ctx_len;
+    const long long tiles = max((long long)B, ((long long)T * G + 127) / 128);     // (of 128 rows, at least)
+    const bool light = max_ctx_len > 0 && max_ctx_len <= LIGHT_MAX_CTX &&
+                       (tiles * Hk > compute_units() || walk <= LIGHT_MAX_CTX_OF_FEW);
     const int kw = light ? 1 : rows > 64 ? 2 : 4;
     const long long tile_rows = light ? 128 : 256 / kw;
     const long long groups = (rows + tile_rows - 1) / tile_rows;

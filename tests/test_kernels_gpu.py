@@ -591,6 +591,15 @@ def test_paged_attention_tiled_f32_window_standout_and_poison():
                    kernel="tiled")
 
 
+@pytest.mark.parametrize("Hq,Hk,D,ps", [(8, 2, 16, 16), (8, 2, 64, 16), (6, 2, 96, 8), (4, 4, 128, 4)])
+@pytest.mark.parametrize("segs,window", [([(300, 20)], None), ([(301, 20)], None), ([(396, 20)], None), ([(397, 20)], None), ([(0, 320)], None),
+                                         ([(0, 417), (5, 30)], None), ([(480, 20)] * 150, None), ([(300, 20)], 200), ([(900, 17), (0, 3)], 256),
+                                         ([(300, 200)], 230)])
+def test_prompt_attention_on_both_sides_of_the_short_contexts(Hq, Hk, D, ps, segs, window):
+    """Around the lines between the two shapes of workgroups: keys, masks that reach back so many, and how many rows there are."""
+    attention_case("bfloat16", Hq, Hk, D, ps, segs, seed=550 + D, kernel="dispatch", window=window, poison=True)
+
+
 @pytest.mark.parametrize("Hq,Hk,D,ps", [(8, 2, 64, 16), (4, 4, 128, 16), (3, 1, 80, 12)])
 def test_prompt_attention_of_windows_at_the_end_of_long_contexts(Hq, Hk, D, ps):
     """Masks that reach back so far that a portion reads at most 512 keys, of contexts of thousands: the shape for short
