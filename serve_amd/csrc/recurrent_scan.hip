@@ -813,8 +813,9 @@ __global__ __launch_bounds__(256) void gla_decay_kernel(const float* __restrict_
   decay[idx] = rs_logsigmoid(z[idx] + (bias ? bias[c] : 0.f)) * inv_tau;
 }
 
-// four values a thread (C a multiple of four, 16-byte aligned arrays): 2,000 x 4,096 of them in 17 us, 19 one by one (the
-// logarithm's arithmetic is what is left)
+// four values a thread (C a multiple of four, 16-byte aligned arrays): 2,000 x 4,096 of them in 27 us, 31 one by one (the
+// logarithm's arithmetic is what is left).  Few values go one by one, four logarithms one after the other being longer than the
+// launch: 8 x 4,096 2.5 us, 3.1 in fours; level from some 1,600 a compute unit (100 x 4,096 3.67 / 3.66, 256 x 2,048 4.07 / 3.87)
 __global__ __launch_bounds__(256) void gla_decay_vec_kernel(const float* __restrict__ z, const float* __restrict__ bias,
                                                             float inv_tau, float* __restrict__ decay, long long quads,
                                                             int C4) {
@@ -839,7 +840,7 @@ extern "C" int sa_gla_decay(const float* z, const float* bias, float tau, float*
   const long long total = (long long)T * C;
   const long long blocks = (total + 255) / 256;
   if (blocks > 0x7fffffffLL) return SA_ERR_ARG;
-  if (C % 4 == 0 && !(((uintptr_t)z | (uintptr_t)decay | (uintptr_t)bias) & 15)) {
+  if (total >= 1600LL * compute_units() && C % 4 == 0 && !(((uintptr_t)z | (uintptr_t)decay | (uintptr_t)bias) & 15)) {
     hipLaunchKernelGGL(gla_decay_vec_kernel, dim3((unsigned)((total / 4 + 255) / 256)), dim3(256), 0, stream, z, bias, 1.f / tau,
                        decay, total / 4, C / 4);
     SA_LAUNCH_CHECK();
