@@ -490,6 +490,10 @@ static int try_rope_kv_vec(const void* qkv, long long row_stride, void* q_out, i
   const size_t tile_bytes = (size_t)tpb * ((size_t)Hk * Dv + 8) * 2;
   const bool aligned = !(((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_pages | (uintptr_t)v_pages | (uintptr_t)bias |
                           (uintptr_t)freq | (uintptr_t)wq | (uintptr_t)wk) & 15);
+  // (narrow rows: their sums of squares, a wave after the other, and a barrier are longer than the kernel of one value a
+  // thread.  That / this one, us: 4 heads of 16 on 2, 8 tokens 4.1 / 5.0, 2,000 5.7 / 7.2; 8 of 64 on 2 4.5 / 5.0 at 64
+  // tokens, 5.4 / 5.2 at 300; 16 of 64 on 4 4.7 / 4.6 at one, 6.2 / 5.1 at 65)
+  if (NORM && (Hq + 2 * Hk) * D < (T <= 64 ? 1536 : 768)) return 0;
   if (act_dtype != SA_BF16 || adjacent || (rot & 15) || ((D | Dv | Dp) & 7) || (row_stride & 7) || !aligned ||
       tile_bytes > room)
     return 0;
