@@ -118,7 +118,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
 // * One that numbers below 2^-126 may have reached.  Taking every plane and every product of planes below that as zero
 //   would change a sum of K products by less than 3 K 2^-126 (|a| + |w|) + 6 K 2^-126, with the largest |a| and |w| of the
 //   workgroup's rows.  That is nothing (2^-26 of it) to a result above redo_limit.  The others, the zeros among them, are
-//   computed again if the operands of the workgroup's rows are small enough for it: no plane of a number of 2^-103 and
+//   computed again if the operands of the rows they come from are small enough for it: no plane of a number of 2^-103 and
 //   more is below 2^-126, and products of planes that are make 2^-29 of the numbers' product where that is 2^-94 and more.
 //   Results of rows of zeros, and small ones of ordinary operands, so stay as they are.
 __device__ __forceinline__ float redo_limit(float most_a, float most_w, int K) {
@@ -146,10 +146,25 @@ __device__ __forceinline__ uint32_t least_key(const float* X, int row0, int rows
   return key;
 }
 
-// Whether numbers below 2^-126 can have come up in the products of these rows of A and W.  For a whole wave.
-__device__ __forceinline__ bool small_operands(const float* A, int m0, int ms, int M, const float* W, int n0, int ns, int N, int K,
-                                           int k_begin, int k_end) {
-  const uint32_t ka = least_key(A, m0, ms, M, K, k_begin, k_end), kw = least_key(W, n0, ns, N, K, k_begin, k_end);
+// The same of one row.
+__device__ __forceinline__ uint32_t least_key(const float* row, int k_begin, int k_end) {
+  const int lane = threadIdx.x & 63;
+  uint32_t key = 0xffffffffu;
+  for (int k = k_begin + lane * 4; k < k_end; k += 16 * 256) {
+    f32x4_t v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const f32x4_t*>(row + min(k + 256 * i, k_end - 4));
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) key = min(key, (__float_as_uint(v[i][e]) << 1) - 1u);
+  }
+  for (int o = 32; o > 0; o >>= 1) key = min(key, (uint32_t)__shfl_xor((int)key, o, SA_WAVE));
+  return key;
+}
+
+// Whether numbers below 2^-126 can have come up in products of operands with these keys.
+__device__ __forceinline__ bool small_operands(uint32_t ka, uint32_t kw) {
   if (ka == 0xffffffffu || kw == 0xffffffffu) return false;          // (nothing but zeros)
   const float a = __uint_as_float((ka + 1u) >> 1), w = __uint_as_float((kw + 1u) >> 1);
   return a < 0x1p-103f || w < 0x1p-103f || a * w < 0x1p-94f;
@@ -169,6 +184,32 @@ __device__ __noinline__ void redo(const float* A, const float* W, float* C, int 
     for (int e = 0; e < 4; ++e) sum = fma((double)a[e], (double)w[e], sum);
   }
   *cp = (float)sum;
+}
+
+// A wave's small results, a bit each in `small`, one at a time by the two rows they come from: sums of ordinary operands that
+// cancel to zero, of which large products have one here and there (2,048 x 16,384 of 2,048 columns: one or two in all), and
+// those of rows of zeros, which go together.  (512 x 8,192 results, K 2048, one of them zero: 134 us with
+// the wave's rows searched as a whole for it, 105 so and without it; 24 rows, one of zeros, over 16,384: 61 and 32, 28 without it.)  True where some are left after SP_FEW: the wave's rows are then searched as a whole,
+// which takes longer (K 2048: 30 us).  `row_of` and `col_of` give a bit's place, `in_row` and `in_col` this lane's bits of a
+// row of A and of one of W.  For a whole wave.
+#define SP_FEW 8
+template <typename RowOf, typename ColOf, typename InRow, typename InCol>
+__device__ __forceinline__ bool settle(const float* A, const float* W, float* C, unsigned long long& small, int N, int K, int k_begin,
+                                       int k_end, float limit, RowOf row_of, ColOf col_of, InRow in_row, InCol in_col) {
+  const int lane = threadIdx.x & 63;
+  for (int turn = 0; turn < SP_FEW; ++turn) {
+    const unsigned long long lanes = __ballot(small != 0);
+    if (!lanes) return false;
+    const int l = __builtin_ctzll(lanes);
+    const int x = small ? __builtin_ctzll(small) : 0;
+    const int m = __builtin_amdgcn_readlane(row_of(x), l), n = __builtin_amdgcn_readlane(col_of(x), l);
+    const uint32_t ka = least_key(A + (size_t)m * K, k_begin, k_end), kw = least_key(W + (size_t)n * K, k_begin, k_end);
+    if (small_operands(ka, kw) && lane == l) redo(A, W, C, m, n, N, K, k_begin, k_end, limit);
+    if (lane == l) small &= small - 1;
+    if (ka == 0xffffffffu) small &= ~in_row(m);
+    if (kw == 0xffffffffu) small &= ~in_col(n);
+  }
+  return __any(small != 0);
 }
 
 __device__ __forceinline__ uint32_t lds_offset(const void* p) {
@@ -371,7 +412,8 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
   __syncthreads();
   const float limit = redo_limit(fmaxf(fmaxf(sizes[0], sizes[1]), fmaxf(sizes[2], sizes[3])),
                                  fmaxf(fmaxf(sizes[4], sizes[5]), fmaxf(sizes[6], sizes[7])), K);
-  bool small = false, odd = false;
+  unsigned long long small = 0;          // which results of this lane are
+  bool odd = false;
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -383,19 +425,27 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
         const float v = total[i][j][e];
         if (m < M && n < N) {
           C[(size_t)m * N + n] = v;
-          small |= fabsf(v) <= limit;
+          small |= fabsf(v) <= limit ? 1ull << (i * 32 + j * 16 + e) : 0ull;
           odd |= !(fabsf(v) < INFINITY);
         }
       }
     }
-  const bool any_small = __any(small);
-  if (!any_small && !__any(odd)) return;
+  if (!__any(small != 0) && !__any(odd)) return;
   const int k_begin = s_begin * 16, k_end = min(K, s_end * 16);
-  const float below = any_small && small_operands(A, m0 + wm * 32 * TI, 32 * TI, M, W, n0 + wn * 64, 64, N, K, k_begin, k_end) ? limit : -1.f;
-  if (!odd && !(small && below >= 0.f)) return;
+  const int mw = m0 + wm * 32 * TI, nw = n0 + wn * 64;
+  auto row_of = [&](int x) { return mw + (x >> 5) * 32 + 8 * ((x & 15) >> 2) + 4 * h + (x & 3); };
+  auto col_of = [&](int x) { return nw + ((x >> 4) & 1) * 32 + r32; };
+  auto in_row = [&](int m) {
+    const int q = (m - mw) & 31;
+    return ((q >> 2) & 1) == h ? 0x10001ull << (((m - mw) & 32) + (q >> 3) * 4 + (q & 3)) : 0ull;
+  };
+  auto in_col = [&](int n) { return ((n - nw) & 31) == r32 ? 0x0000ffff0000ffffull << (((n - nw) & 32) >> 1) : 0ull; };
+  const bool left = settle(A, W, C, small, N, K, k_begin, k_end, limit, row_of, col_of, in_row, in_col);
+  const float below = left && small_operands(least_key(A, mw, 32 * TI, M, K, k_begin, k_end),
+                                             least_key(W, nw, 64, N, K, k_begin, k_end)) ? limit : -1.f;
+  if (!odd && !(small != 0 && below >= 0.f)) return;
   for (int x = 0; x < TI * 32; ++x) {
-    const int m = m0 + wm * 32 * TI + (x >> 5) * 32 + 8 * ((x & 15) >> 2) + 4 * h + (x & 3);
-    const int n = n0 + wn * 64 + ((x >> 4) & 1) * 32 + r32;
+    const int m = row_of(x), n = col_of(x);
     if (m >= M || n >= N) continue;
     redo(A, W, C, m, n, N, K, k_begin, k_end, below);
   }
@@ -590,7 +640,7 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
     most_w = fmaxf(most_w, sizes[8 + i]);
   }
   const float limit = redo_limit(most_a, most_w, K);
-  bool small = false, odd = false;
+  bool any_small = false, odd = false;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int m = m0 + mt * 32 + r;
@@ -610,7 +660,7 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
       float* cp = C + (size_t)m * N + cn;
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        small |= cn + c < N && fabsf(v[c]) <= limit;
+        any_small |= cn + c < N && fabsf(v[c]) <= limit;
         odd |= cn + c < N && !(fabsf(v[c]) < INFINITY);
       }
       if (cn + 3 < N && (((uintptr_t)cp) & 15) == 0) {
@@ -622,13 +672,29 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
       }
     }
   }
-  const bool any_small = __any(small);
-  if (!any_small && !__any(odd)) return;
+  if (!__any(any_small) && !__any(odd)) return;
   const int k_begin = s_begin * COLS, k_end = min(K, (s_begin + n) * COLS);
-  const float below = any_small && small_operands(A, m0, 32 * MT, M, W, n0 + wt * 32, 32, N, K, k_begin, k_end) ? limit : -1.f;
-  if (!odd && !(small && below >= 0.f)) return;
+  const int nw = n0 + wt * 32;
+  auto row_of = [&](int x) { return m0 + (x >> 4) * 32 + r; };
+  auto col_of = [&](int x) { return nw + ((x & 15) >> 2) * 8 + h * 4 + (x & 3); };
+  auto in_row = [&](int m) { return ((m - m0) & 31) == r ? 0xffffull << ((m - m0) >> 5) * 16 : 0ull; };
+  auto in_col = [&](int n) {
+    const int q = n - nw;
+    return ((q >> 2) & 1) == h ? 0x0001000100010001ull << ((q >> 3) * 4 + (q & 3)) : 0ull;
+  };
+  unsigned long long small = 0;                              // which of them, from what this lane has just stored
+#pragma unroll 16
   for (int x = 0; x < MT * 16; ++x) {
-    const int m = m0 + (x >> 4) * 32 + r, cn = n0 + wt * 32 + ((x & 15) >> 2) * 8 + h * 4 + (x & 3);
+    const int m = row_of(x), cn = col_of(x);
+    const float v = C[(size_t)min(m, M - 1) * N + min(cn, N - 1)];
+    small |= m < M && cn < N && fabsf(v) <= limit ? 1ull << x : 0ull;
+  }
+  const bool left = settle(A, W, C, small, N, K, k_begin, k_end, limit, row_of, col_of, in_row, in_col);
+  const float below = left && small_operands(least_key(A, m0, 32 * MT, M, K, k_begin, k_end),
+                                             least_key(W, nw, 32, N, K, k_begin, k_end)) ? limit : -1.f;
+  if (!odd && !(small != 0 && below >= 0.f)) return;
+  for (int x = 0; x < MT * 16; ++x) {
+    const int m = row_of(x), cn = col_of(x);
     if (m < M && cn < N) redo(A, W, C, m, cn, N, K, k_begin, k_end, below);
   }
 }

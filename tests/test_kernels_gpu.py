@@ -280,6 +280,35 @@ def test_gemm_f32_by_split_operands_over_the_range_of_floats(M, N, K, parts, ea,
         assert (got[1] == 0).all() and (got[:, 2] == 0).all()
 
 
+@pytest.mark.parametrize("M,N,K,parts", [(24, 70, 516, 1), (70, 8300, 260, 1), (100, 130, 260, 2), (130, 129, 516, 1), (300, 640, 1028, 1)])
+@pytest.mark.parametrize("count", [1, 5, 200])
+def test_gemm_f32_by_split_operands_where_a_few_results_are_zero(M, N, K, parts, count):
+    """Sums that cancel to nothing among ordinary ones, and sums that only small numbers beside large ones make, a few or many in a
+    wave's share: the first stay zeros, the others are computed again."""
+    from serve_amd import ops
+    run = ops.gemm_f32_mid_parts if M <= ops.F32_MID_MAX_ROWS else ops.gemm_f32_split
+    a, w = rnd((M, K), torch.float32, 57), rnd((N, K), torch.float32, 58)
+    g = torch.Generator().manual_seed(59)
+    rows, cols = (torch.randperm(x, generator=g)[:min(count, x - 2)].tolist() for x in (M, N))
+    for i, m in enumerate(rows):
+        a[m] = 0
+        a[m, 4], a[m, 9] = 1.5, -1.5
+        if i % 2:
+            a[m, 4], a[m, 9] = 2.0 ** -140, 2.0 ** -127
+    for n in cols:
+        w[n, 9] = w[n, 4]
+        if n % 2:
+            w[n, 4], w[n, 9] = 2.0 ** 100, 1.3 * 2.0 ** 99
+    out = torch.full((parts, M, N), float("nan"), dtype=torch.float32, device=DEV)
+    run(a, w, out)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    got = out.double().sum(0)
+    # (as above)
+    assert ((got - want).abs() <= size * (2.0 ** -23 + (6 * (K // 16 + 1) + 16) * 2.0 ** -24) + parts * 2.0 ** -149).all()
+    zero = [n for n in cols if n % 2 == 0]
+    assert (got[rows[::2]][:, zero] == 0).all()
+
+
 @pytest.mark.parametrize("M,N,K,parts", [(129, 2, 349508, 1), (300, 3, 349568, 2), (129, 2, 4194304, 1)])
 def test_gemm_f32_by_split_operands_of_very_long_rows(M, N, K, parts):
     """Inner sizes of which not even a tile of rows has room in the scratch memory, and beyond what its grid can count."""
