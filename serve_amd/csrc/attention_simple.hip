@@ -382,10 +382,11 @@ static int launch_tiled(const void* q, int q_stride, void* out, const void* k_pa
 // the keys outside the range are masked where the scores are.  Before (the pages looked up by every lane, keys and values
 // in two trips of eight) / now, with the merge, 32 heads on 8, us: heads of 64, 24 requests at context 300 23.6 / 19.3, 64
 // at 400 29.8 / 26.2, 8 at 4,096 28.6 / 25.0, one at 8,192 21.0 / 17.2; heads of 96 23.9 / 16.4, 28.3 / 20.6, 26.2 / 20.1,
-// 21.5 / 17.0; heads of 128 33.9 / 28.4, 54.0 / 47.4, 54.7 / 48.3, 29.9 / 27.0 (64 at 2,000: 1.05 GB in 178 us, 204 before).
+// 21.5 / 17.0 (of 96 over much to read, which wants two waves a SIMD: 8 at 4,096 on 32 heads 46.7 / 35.2, 51 with registers for
+// one, 64 at 513 48.1 / 36.3; of 112 49.4 / 39.5); heads of 128 33.9 / 28.4, 54.0 / 47.4, 54.7 / 48.3, 29.9 / 27.0 (64 at 2,000: 1.05 GB in 178 us, 204 before).
 // ---------------------------------------------------------------------------------------------
 template <int DV, int GR>   // D / 16; query heads per wave
-__global__ __launch_bounds__(64, DV <= 4 ? 2 : 1) void paged_attention_decode_f32_kernel(
+__global__ __launch_bounds__(64, 2) void paged_attention_decode_f32_kernel(
     const float* __restrict__ q, int q_stride, float* __restrict__ out, const float* __restrict__ k_pages,
     const float* __restrict__ v_pages, const int* __restrict__ block_table, int max_pages,
     const int* __restrict__ cu_q, const int* __restrict__ ctx_len, int Hq, int Hk, int page_size, float scale,
@@ -446,7 +447,7 @@ __global__ __launch_bounds__(64, DV <= 4 ? 2 : 1) void paged_attention_decode_f3
   look_up(min(b_first, b_hi) * 64, page, place);
   for (int kb = b_first * 64; kb <= b_last * 64; kb += 64) {
     // all loads of the block before anything waits: the time of a short context is this chain's
-    constexpr int KN = DV <= 4 ? 4 : 2;             // keys of a lane fetched at a time (wide heads: registers are short)
+    constexpr int KN = DV <= 4 ? 4 : GR == 4 && DV >= 6 ? 1 : 2;  // keys of a lane fetched at a time (wide heads: registers are short)
     float4 kv[KN][DV];
     auto fetch_k = [&](int first) __attribute__((always_inline)) {
 #pragma unroll
@@ -461,7 +462,7 @@ __global__ __launch_bounds__(64, DV <= 4 ? 2 : 1) void paged_attention_decode_f3
     fetch_k(0);
     // values: four keys of a dim are one load (they lie in one page, at a multiple of four; keys outside the range are
     // read from the page of its nearest key, at their own place in it)
-    constexpr int VN = NA == 1 ? 16 : 8;            // groups of four keys fetched at a time
+    constexpr int VN = NA == 1 ? 16 : GR == 4 && DV >= 7 ? 4 : 8;  // groups of four keys fetched at a time
     float4 vv[VN][NA];
     uint32_t voff[NA];
 #pragma unroll
