@@ -188,10 +188,10 @@ __device__ __noinline__ void redo(const float* A, const float* W, float* C, int 
 
 // A wave's small results, a bit each in `small`, one at a time by the two rows they come from: sums of ordinary operands that
 // cancel to zero, of which large products have one here and there (2,048 x 16,384 of 2,048 columns: one or two in all), and
-// those of rows of zeros, which go together.  (512 x 8,192 results, K 2048, one of them zero: 134 us with
-// the wave's rows searched as a whole for it, 105 so and without it; 24 rows, one of zeros, over 16,384: 61 and 32, 28 without it.)  True where some are left after SP_FEW: the wave's rows are then searched as a whole,
-// which takes longer (K 2048: 30 us).  `row_of` and `col_of` give a bit's place, `in_row` and `in_col` this lane's bits of a
-// row of A and of one of W.  For a whole wave.
+// those of rows of zeros, which go together.  (512 x 8,192 results, K 2048, one of them zero: 134 us with the wave's rows
+// searched as a whole for it, 105 so and without it; 24 rows, one of zeros, over 16,384: 61 and 32, 28 without it.)  True
+// where some are left after SP_FEW: the wave's rows are then searched as a whole, 30 us at K 2048.  `row_of` and `col_of`
+// give a bit's place, `in_row` and `in_col` this lane's bits of a row of A and of one of W.  For a whole wave.
 #define SP_FEW 8
 template <typename RowOf, typename ColOf, typename InRow, typename InCol>
 __device__ __forceinline__ bool settle(const float* A, const float* W, float* C, unsigned long long& small, int N, int K, int k_begin,
