@@ -42,6 +42,7 @@ SOURCES: Dict[str, str] = {
     "attention_simple": "attention_simple.hip",
     "sampling": "sampling.hip",
     "gemm_mfma": "gemm_mfma.hip",
+    "gemm_experts": "gemm_experts.hip",
     "attention_mfma": "attention_mfma.hip",
     "membench": "membench.hip",
     "blaslt": "blaslt.hip",

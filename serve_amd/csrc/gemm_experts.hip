@@ -1,0 +1,283 @@
+// The two products of routed experts for prompt portions, bf16 with float32 sums, over tiles of one expert's rows from lists
+// that csrc/moe.hip has built on the device.
+//
+// What bounds them: reading the experts' matrices once (32 experts of 2,048 x 1,024: 403 MB).  So an expert's rows are one
+// tile up to 256 of them (beyond that, tiles of equal size), and a workgroup takes 256 weight rows: with 32 experts that is
+// one round of the chip for either product, and a row of activations is fetched by 8 workgroups.  Which these are: a die
+// takes a run of (tile, weight rows), so the workgroups that read the same activations share an L2, which then holds one
+// expert's at a time.
+//
+// Measured, 1,000 tokens, 4 of 32 experts of 2,048 x 1,024, us: gate/up 88 -> 62 and down 67 -> 43 against tiles of 128 rows
+// by 128 weight rows in the order of the grid (an expert with 130 rows read its matrices twice, and every die all of the
+// activations).  Of the two, 72 us are the weights' stream (5.6 TB/s; without loads 41 us, without loads and products 23).
+#include "common.h"
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef float floatx4_t __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
+
+union Frag {
+  u32x4_t r;
+  bf16x8_t v;
+};
+
+typedef __attribute__((address_space(3))) u32x4_t* lds_ptr_t;
+typedef const __attribute__((address_space(1))) void* gptr_t;
+
+// all but the newest n of this wave's loads have landed
+#define SA_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xf) | (((n) >> 4) << 14) | (0x7 << 4) | (0xf << 8))
+
+#define EX_TILE_ROWS 256
+#define EX_LDS (160 * 1024)        // of a workgroup, which has a compute unit to itself
+
+// FIRST: act[r] = gate(Wg_e x, Wu_e x) with x = A[perm[r] / top], W [2, E, N, K] (gates, then ups, `up_offset` rows apart).
+// else:  C[perm[r]] = W_e A[r], W [E, N, K].  r: grouped rows of this tile.
+struct ExpertArgs {
+  const bf16_t* A;
+  const bf16_t* W;
+  void* C;
+  int N, K, up_offset, gx, top, gate_kind;
+  float gate_limit;
+  const int* perm;
+  const int* tile_expert;
+  const int* tile_row0;     // of every tile, and behind the last the number of grouped rows
+  const int* num_tiles;
+  const float* in_wts;      // FIRST: fp32 [token * top + k], multiplies gate and up sums before the gate (null: not)
+};
+
+// Eight waves: two groups of 16 RT rows times four groups of 16 CT weight rows (FIRST: half of a group's are gates, the other
+// half their ups, so that a pair meets in a lane).  A stage is 64 columns of both operands, loaded straight into LDS, a
+// kilobyte (8 rows of 128 bytes) an instruction; segment s of row r lies at slot s ^ ((r >> 1) & 7), so that the lanes a
+// 16-byte LDS read serves together touch every bank once.  Weights come from memory and activations mostly from the die's L2,
+// which needs fewer stages ahead: two rings, the weights' filled by waves 0 to 3 and the activations' by waves 4 to 7, since a
+// wave's loads land in order and would otherwise wait for each other.
+template <int CT, int RT, bool FIRST>
+__device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, int e, int row0, int M, int col0,
+                                            int first) {
+  constexpr int BM = 32 * RT, BN = 64 * CT;
+  constexpr int COLS = FIRST ? BN / 2 : BN;
+  constexpr int A_BYTES = BM * 128, W_BYTES = BN * 128;
+  // stages of the rings: of the weights as many as there is room for beside two of the activations
+  constexpr int NW = CT == 2 ? 6 : 4 * W_BYTES + 2 * A_BYTES <= EX_LDS ? 4 : 3;
+  constexpr int ROOM = (EX_LDS - NW * W_BYTES) / A_BYTES;
+  constexpr int NA = ROOM > 4 ? 4 : ROOM;
+  static_assert(NA >= 2 && NW >= 3 && NW * W_BYTES + NA * A_BYTES <= EX_LDS, "the LDS of a compute unit");
+  constexpr int WI = 2 * CT;                       // instructions a stage and wave: 64 CT weight rows over four waves
+  constexpr int NI = WI > RT ? WI : RT;            // (of the activations: 32 RT rows over four waves)
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int g = lane >> 4, c = lane & 15;
+  const int rg = wave >> 2, cg = wave & 3;
+  const int K = p.K, N = p.N;
+  const bool loads_w = wave < 4;
+  const int lw = wave & 3;
+
+  const bf16_t* src[NI];
+  if (loads_w) {
+    const bf16_t* W = p.W + (size_t)e * N * K;
+#pragma unroll
+    for (int d = 0; d < WI; ++d) {
+      const int row = (lw * WI + d) * 8 + (lane >> 3);
+      const int seg = (lane & 7) ^ ((row >> 1) & 7);
+      int n;
+      if (FIRST) {
+        const int in = row % (16 * CT);
+        n = min(col0 + (row / (16 * CT)) * 8 * CT + in % (8 * CT), N - 1) + (in >= 8 * CT ? p.up_offset : 0);
+      } else {
+        n = min(col0 + row, N - 1);
+      }
+      src[d] = W + (size_t)n * K + seg * 8;
+    }
+  } else {
+#pragma unroll
+    for (int d = 0; d < RT; ++d) {
+      const int row = (lw * RT + d) * 8 + (lane >> 3);
+      const int seg = (lane & 7) ^ ((row >> 1) & 7);
+      const int r = row0 + min(row, M - 1);
+      src[d] = p.A + (size_t)(FIRST ? p.perm[r] / p.top : r) * K + seg * 8;
+    }
+  }
+  const lds_ptr_t as = (lds_ptr_t)lds, ws = as + NA * (A_BYTES / 16);
+  const uint32_t lds_base = (uint32_t)(uintptr_t)as;
+  const uint32_t a_addr = lds_base + (uint32_t)((rg * RT * 16 + c) * 128);
+  const uint32_t w_addr = lds_base + NA * A_BYTES + (uint32_t)((cg * CT * 16 + c) * 128);
+  const uint32_t slot0 = (uint32_t)((g ^ ((c >> 1) & 7)) * 16), slot1 = (uint32_t)(((4 + g) ^ ((c >> 1) & 7)) * 16);
+
+  const int nstages = K >> 6;
+  const int rot = first % nstages;
+  auto column = [&](int s) __attribute__((always_inline)) {
+    int t = min(s, nstages - 1) + rot;             // past the last stage: the last again (nobody reads it)
+    if (t >= nstages) t -= nstages;
+    return t * 64;
+  };
+  auto fetch_w = [&](int s) __attribute__((always_inline)) {
+    const int k0 = column(s);
+#pragma unroll
+    for (int d = 0; d < WI; ++d)
+      __builtin_amdgcn_global_load_lds((gptr_t)(src[d] + k0), (__attribute__((address_space(3))) void*)
+                                       (ws + (s % NW) * (W_BYTES / 16) + (lw * WI + d) * 64), 16, 0, 0);
+  };
+  auto fetch_a = [&](int s) __attribute__((always_inline)) {
+    const int k0 = column(s);
+#pragma unroll
+    for (int d = 0; d < RT; ++d)
+      __builtin_amdgcn_global_load_lds((gptr_t)(src[d] + k0), (__attribute__((address_space(3))) void*)
+                                       (as + (s % NA) * (A_BYTES / 16) + (lw * RT + d) * 64), 16, 0, 0);
+  };
+
+  floatx4_t acc[RT][CT];
+#pragma unroll
+  for (int mt = 0; mt < RT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < CT; ++nt) acc[mt][nt] = (floatx4_t){0.f, 0.f, 0.f, 0.f};
+
+  if (loads_w) {
+#pragma unroll
+    for (int i = 0; i < NW - 1; ++i) fetch_w(i);
+  } else {
+#pragma unroll
+    for (int i = 0; i < NA - 1; ++i) fetch_a(i);
+  }
+  for (int s = 0; s < nstages; ++s) {
+    if (loads_w) SA_WAIT_VMCNT(WI * (NW - 2));     // this wave's part of stage s lies in LDS
+    else SA_WAIT_VMCNT(RT * (NA - 2));
+    __builtin_amdgcn_s_barrier();                  // everybody's does, and everybody has read the stage before
+    if (loads_w) fetch_w(s + NW - 1);
+    else fetch_a(s + NA - 1);
+    const uint32_t ao = a_addr + (uint32_t)((s % NA) * A_BYTES), wo = w_addr + (uint32_t)((s % NW) * W_BYTES);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // (the reads are written as instructions of their own: the compiler does not see the loads into LDS as stores, and
+      // would otherwise wait for all of them before every read)
+      Frag af[RT], wf[CT];
+#pragma unroll
+      for (int nt = 0; nt < CT; ++nt)
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(wf[nt].r) : "v"(wo + (h ? slot1 : slot0)), "n"(nt * 16 * 128));
+#pragma unroll
+      for (int mt = 0; mt < RT; ++mt)
+        asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(af[mt].r) : "v"(ao + (h ? slot1 : slot0)), "n"(mt * 16 * 128));
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int nt = 0; nt < CT; ++nt) asm volatile("" : "+v"(wf[nt].r));
+#pragma unroll
+      for (int mt = 0; mt < RT; ++mt) asm volatile("" : "+v"(af[mt].r));
+#pragma unroll
+      for (int mt = 0; mt < RT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < CT; ++nt)
+          acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[nt].v, af[mt].v, acc[mt][nt], 0, 0, 0);
+    }
+  }
+  SA_WAIT_VMCNT(0);                                // (loads into LDS beyond the last stage)
+
+  // lane l holds C[m = row tile's row l % 16][n = 4 (l / 16) .. + 3] of every tile pair
+#pragma unroll
+  for (int mt = 0; mt < RT; ++mt) {
+    const int m = (rg * RT + mt) * 16 + c;
+    if (m >= M) continue;
+    const int r = row0 + m;
+    const int at = FIRST && !p.in_wts ? 0 : p.perm[r];
+    const float in_w = FIRST && p.in_wts ? p.in_wts[at] : 1.f;   // (a weight on the input: gate and up are linear in it)
+#pragma unroll
+    for (int nt = 0; nt < (FIRST ? CT / 2 : CT); ++nt) {
+      const int n = col0 + cg * (COLS / 4) + nt * 16 + 4 * g;
+      float o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if constexpr (FIRST) {
+          const float gt = acc[mt][nt][i] * in_w, up = acc[mt][nt + CT / 2][i] * in_w;
+          // (the plain gate with the fast exponential, as in the dense feed-forward's products)
+          o[i] = p.gate_kind == SA_GATE_SILU ? (gt / (1.f + __expf(-gt))) * up : gate_mul(gt, up, p.gate_kind, p.gate_limit);
+        } else {
+          o[i] = acc[mt][nt][i];
+        }
+      }
+      if (n < N) {                                 // (N is a multiple of 64)
+        if constexpr (FIRST) {
+          union { bf16_t h[4]; uint2 u; } q;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) q.h[i] = from_float<bf16_t>(o[i]);
+          *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.C) + (size_t)r * N + n) = q.u;
+        } else {
+          *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.C) + (size_t)at * N + n) = make_float4(o[0], o[1], o[2], o[3]);
+        }
+      }
+    }
+  }
+}
+
+template <int CT, bool FIRST>
+__global__ __launch_bounds__(512, 2) void expert_product_kernel(ExpertArgs p) {
+  extern __shared__ __attribute__((aligned(16))) u32x4_t expert_lds[];
+  // neighbouring workgroups run on different dies: a die takes a run of the work, the weight rows of one tile together
+  const int tiles = *p.num_tiles;
+  const int work = tiles * p.gx;
+  const int die = blockIdx.x & 7, place = blockIdx.x >> 3;
+  const int share = work >> 3, more = work & 7;
+  if (place >= share + (die < more ? 1 : 0)) return;       // (the grid is the worst case)
+  const int t = die * share + min(die, more) + place;
+  const int tile = t / p.gx;
+  const int col0 = (t - tile * p.gx) * (FIRST ? 32 * CT : 64 * CT);
+  const int e = p.tile_expert[tile], row0 = p.tile_row0[tile];
+  const int M = p.tile_row0[tile + 1] - row0;              // the next tile, or the end, follows at once
+  // Workgroups begin at different columns, also from die to die: rows of W lie a power of two apart, and the same columns of
+  // many rows are in a few channels of the memory (1,000 tokens, both products: 105 us so, 112 with an order that repeats from
+  // die to die, 118 with one of eight places, 120 where all begin at the first column).
+  const int nstages = p.K >> 6;
+  const int first = place + (nstages >= 8 ? nstages >> 3 : 1) * die;
+  if (M <= 32) expert_tile<CT, 1, FIRST>(p, expert_lds, e, row0, M, col0, first);
+  else if (M <= 64) expert_tile<CT, 2, FIRST>(p, expert_lds, e, row0, M, col0, first);
+  else if (M <= 128) expert_tile<CT, 4, FIRST>(p, expert_lds, e, row0, M, col0, first);
+  else if (M <= 160) expert_tile<CT, 5, FIRST>(p, expert_lds, e, row0, M, col0, first);
+  else if (M <= 192) expert_tile<CT, 6, FIRST>(p, expert_lds, e, row0, M, col0, first);
+  else expert_tile<CT, 8, FIRST>(p, expert_lds, e, row0, M, col0, first);
+}
+
+template <int CT, bool FIRST>
+static int launch(ExpertArgs p, int max_tiles, hipStream_t stream) {
+  p.gx = (p.N + (FIRST ? 32 : 64) * CT - 1) / ((FIRST ? 32 : 64) * CT);
+  const long long grid = ((long long)p.gx * max_tiles + 7) / 8 * 8;
+  if (max_tiles < 1 || grid > 0x7fffffffLL) return SA_ERR_ARG;
+  auto kernel = expert_product_kernel<CT, FIRST>;
+  static bool allowed[64] = {};                    // (per device: more than 64 KB of LDS has to be asked for)
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return SA_ERR_ARG;
+  if (!allowed[dev]) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, EX_LDS);
+    if (e != hipSuccess) return (int)e;
+    allowed[dev] = true;
+  }
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), EX_LDS, stream, p);
+  SA_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" int sa_expert_tile_rows() { return EX_TILE_ROWS; }
+
+// Lists from sa_moe_group with tiles of sa_expert_tile_rows() rows at most (max_tiles: the grid's worst case, rows /
+// tile rows + E).  bf16; d and F multiples of 64 (whole stages of K).
+//   gate/up: h [T, d] gathered by perm / top, Wgu [2, E, F, d] -> act [rows, F] = gate(gate, up)
+//            (in_wts, fp32 [T top] or null: both sums times the row's weight first, for weights on the experts' inputs)
+//   down:    act [rows, F], Wd [E, d, F] -> yk [T top, d] fp32 at row perm[r]
+extern "C" int sa_expert_products(const void* h, const void* Wgu, const void* Wd, void* act, float* yk, int E, int d, int F,
+                                  int max_tiles, const int* perm, const int* tile_expert, const int* tile_row0,
+                                  const int* num_tiles, int top, int gate_kind, float gate_limit, const float* in_wts,
+                                  hipStream_t stream) {
+  if (E <= 0 || d <= 0 || F <= 0 || (d & 63) || (F & 63) || top <= 0) return SA_ERR_ARG;
+  if (gate_kind < 0 || gate_kind >= SA_GATE_KINDS || (long long)E * F > 0x7fffffffLL) return SA_ERR_ARG;
+  ExpertArgs p = {(const bf16_t*)h, (const bf16_t*)Wgu, act, F, d, E * F, 0, top, gate_kind, gate_limit,
+                  perm, tile_expert, tile_row0, num_tiles, in_wts};
+  // 256 weight rows a workgroup where that still gives most compute units one (every expert chosen), else 128
+  const int cus = compute_units();
+  const int rc = (long long)E * ((F + 127) / 128) * 4 >= 3ll * cus ? launch<4, true>(p, max_tiles, stream)
+                                                                  : launch<2, true>(p, max_tiles, stream);
+  if (rc != 0) return rc;
+  p.A = (const bf16_t*)act;
+  p.W = (const bf16_t*)Wd;
+  p.C = yk;
+  p.N = d;
+  p.K = F;
+  p.in_wts = nullptr;
+  return (long long)E * ((d + 255) / 256) * 4 >= 3ll * cus ? launch<4, false>(p, max_tiles, stream)
+                                                           : launch<2, false>(p, max_tiles, stream);
+}

@@ -144,7 +144,8 @@ __device__ __forceinline__ void route_token(const float* __restrict__ z, int* __
 // ---------------------------------------------------------------------------------------------
 #define MOE_LDS_EXPERTS 1024
 // counts, running sums and tiles, then the rows' places; `cursor`: E counters, in LDS or in memory
-__device__ __forceinline__ void group_rows(const int* ids, int n, int E, int tile_rows, int* __restrict__ offsets,
+// even: an expert's tiles are of equal size, in whole sixteens, and not full ones with what is left in the last
+__device__ __forceinline__ void group_rows(const int* ids, int n, int E, int tile_rows, bool even, int* __restrict__ offsets,
                                            int* cursor, int* __restrict__ perm, int* __restrict__ tile_expert,
                                            int* __restrict__ tile_row0, int* __restrict__ num_tiles) {
   for (int i = threadIdx.x; i < n; i += blockDim.x)
@@ -173,9 +174,11 @@ __device__ __forceinline__ void group_rows(const int* ids, int n, int E, int til
         offsets[e] = first;
         cursor[e] = first;
       }
+      // (tile_rows is a whole number of sixteens, so this is at most tile_rows, and the last tile still has a row)
+      const int per = even && mine > 0 ? ((c + mine - 1) / mine + 15) / 16 * 16 : tile_rows;
       for (int i = 0; i < mine; ++i) {
         tile_expert[tiles + before - mine + i] = e;
-        tile_row0[tiles + before - mine + i] = first + i * tile_rows;
+        tile_row0[tiles + before - mine + i] = first + i * per;
       }
       run += __shfl(rows, SA_WAVE - 1, SA_WAVE);
       tiles += __shfl(before, SA_WAVE - 1, SA_WAVE);
@@ -191,7 +194,7 @@ __device__ __forceinline__ void group_rows(const int* ids, int n, int E, int til
     if (ids[i] < E) perm[atomicAdd(&cursor[ids[i]], 1)] = i;
 }
 
-__global__ __launch_bounds__(1024) void moe_group_kernel(const int* ids, int n, int E, int tile_rows,
+__global__ __launch_bounds__(1024) void moe_group_kernel(const int* ids, int n, int E, int tile_rows, bool even,
                                                          int* __restrict__ offsets, int* __restrict__ cursor,
                                                          int* __restrict__ perm, int* __restrict__ tile_expert,
                                                          int* __restrict__ tile_row0, int* __restrict__ num_tiles,
@@ -212,8 +215,8 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* ids, int n, 
                   threadIdx.x & (SA_WAVE - 1), over_all, wscale, corr);
   }
   __syncthreads();
-  if (in_lds) group_rows(ids, n, E, tile_rows, offsets, lds_cursor, perm, tile_expert, tile_row0, num_tiles);
-  else group_rows(ids, n, E, tile_rows, offsets, cursor, perm, tile_expert, tile_row0, num_tiles);
+  if (in_lds) group_rows(ids, n, E, tile_rows, even, offsets, lds_cursor, perm, tile_expert, tile_row0, num_tiles);
+  else group_rows(ids, n, E, tile_rows, even, offsets, cursor, perm, tile_expert, tile_row0, num_tiles);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -625,7 +628,7 @@ extern "C" int sa_moe_experts(const void* h, int act_dtype, int* ids, const void
   const int tiles = (int)((n + tile_rows - 1) / tile_rows) + E;
   if (logits && (T > MOE_ROUTE_INSIDE || !wts || outputs < E || ldz < outputs || top > outputs || (corr && over_all != 1)))
     return SA_ERR_ARG;
-  hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), 0, stream, ids, (int)n, E, tile_rows, offsets, cursor, perm,
+  hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), 0, stream, ids, (int)n, E, tile_rows, false, offsets, cursor, perm,
                      tile_expert, tile_row0, num_tiles, logits, ldz, ids, wts, top, over_all, wscale, corr, outputs);
   SA_LAUNCH_CHECK();
   dim3 block(256);
@@ -675,13 +678,13 @@ extern "C" int sa_moe_experts(const void* h, int act_dtype, int* ids, const void
   return 0;
 }
 
-// Only the grouping (and, with logits, the routing): the lists for products that another library runs over tiles of
-// `tile_rows` grouped rows.  ints: as for sa_moe_experts, with max_tiles = sa_moe_max_tiles(T top, E).
+// Only the grouping (and, with logits, the routing): the lists for products that another library runs over tiles of up to
+// `tile_rows` grouped rows (a multiple of 16), an expert's of equal size.  ints: as for sa_moe_experts, with max_tiles = sa_moe_max_tiles(T top, E).
 extern "C" int sa_moe_group(int* ids, int* ints, int T, int top, int E, int tile_rows, const float* logits, int ldz,
                             float* wts, int over_all, float wscale, const float* corr, int outputs, hipStream_t stream) {
   if (T <= 0) return 0;
   const long long n = (long long)T * top;
-  if (E <= 0 || top <= 0 || tile_rows < 16 || n > 0x3fffffffLL) return SA_ERR_ARG;
+  if (E <= 0 || top <= 0 || tile_rows < 16 || (tile_rows & 15) || n > 0x3fffffffLL) return SA_ERR_ARG;
   if (logits && (T > MOE_ROUTE_INSIDE || !wts || outputs < E || ldz < outputs || top > outputs || (corr && over_all != 1)))
     return SA_ERR_ARG;
   const int max_tiles = sa_moe_max_tiles((int)n, E);
@@ -691,7 +694,7 @@ extern "C" int sa_moe_group(int* ids, int* ints, int T, int top, int E, int tile
   int* tile_expert = perm + n;
   int* tile_row0 = tile_expert + max_tiles;
   int* num_tiles = tile_row0 + max_tiles;
-  hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), 0, stream, ids, (int)n, E, tile_rows, offsets, cursor, perm,
+  hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(1024), 0, stream, ids, (int)n, E, tile_rows, true, offsets, cursor, perm,
                      tile_expert, tile_row0, num_tiles, logits, ldz, ids, wts, top, over_all, wscale, corr, outputs);
   SA_LAUNCH_CHECK();
   return 0;

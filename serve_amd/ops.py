@@ -1501,19 +1501,19 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, w_gate: torch.Tensor, w_up: 
         _check(weights is not None and weights.dtype == torch.float32 and weights.shape == (T, top)
                and weights.is_contiguous(), "weights on the experts' inputs must be contiguous fp32 [T, top]")
     if n > MOE_WIDE_MIN_ROWS and logits is None and moe_wide_available(h, w_gate, w_up, w_down):
-        # prompt portions: the grouping here, the two products over tiles of 128 rows with both operands through LDS
-        wide = load_library("gemm_mfma")
-        rows = int(wide.sa_moe_wide_tile_rows())
+        # prompt portions: the grouping here, the two products over tiles of up to 256 rows with both operands through LDS
+        wide = load_library("gemm_experts")
+        rows = int(wide.sa_expert_tile_rows())
         _ret(lib.sa_moe_group(_ptr(ids), _ptr(ints), c_int(T), c_int(top), c_int(E), c_int(rows), c_void_p(0), c_int(0),
                               c_void_p(0), c_int(0), c_float(1.0), c_void_p(0), c_int(outputs), _stream()), "moe_group")
         o = 4
         perm = ints.data_ptr() + o * (2 * E + 1)
         tile_expert = perm + o * n
         tile_row0, num_tiles = tile_expert + o * tiles, tile_expert + o * 2 * tiles
-        _ret(wide.sa_moe_wide(_ptr(h), _ptr(w_gate), _ptr(w_down), _ptr(act), _ptr(yk), c_int(E), c_int(d), c_int(F),
+        _ret(wide.sa_expert_products(_ptr(h), _ptr(w_gate), _ptr(w_down), _ptr(act), _ptr(yk), c_int(E), c_int(d), c_int(F),
                               c_int(-(-n // rows) + E), c_void_p(perm), c_void_p(tile_expert),
                               c_void_p(tile_row0), c_void_p(num_tiles), c_int(top), c_int(GATES[gate]), c_float(limit),
-                              _ptr(weights if weight_inputs else None), _stream()), "moe_wide")
+                              _ptr(weights if weight_inputs else None), _stream()), "expert_products")
         return yk
     ldz = 0
     if logits is not None:

@@ -573,11 +573,40 @@ def test_steps_with_prompt_portions_replayed_from_graphs(tmp_path, dtype):
     assert compared > 3 * count
 
 
+# (256 compute units)  128 weight rows a workgroup in both products; 256 in the first, in both, and in the second, over one stage and more
+@pytest.mark.parametrize("d,F,E", [(64, 64, 14), (128, 2048, 14), (1152, 3264, 15), (3392, 192, 14)])
+def test_experts_products_at_the_edges_of_tiles(d, F, E):
+    """Experts with as many rows as a tile of every size takes and with one more, two and three tiles of equal size, none; widths
+    that are no whole share of a workgroup."""
+    from serve_amd import ops
+    counts = ([1, 32, 33, 64, 65, 128, 129, 160, 161, 192, 193, 256, 0, 257, 545] * 2)[:E]
+    T = sum(counts)
+    g = torch.Generator().manual_seed(d + F)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=g)].int()[:, None].cuda()
+    gc = torch.Generator("cuda").manual_seed(d + F)
+    h = torch.randn((T, d), device="cuda", generator=gc).bfloat16()
+    wgu = (torch.randn((2, E, F, d), device="cuda", generator=gc) * d ** -0.5).bfloat16()
+    wd = (torch.randn((E, d, F), device="cuda", generator=gc) * F ** -0.5).bfloat16()
+    w = torch.rand((T, 1), device="cuda", generator=gc) + 0.5
+    assert T > ops.MOE_WIDE_MIN_ROWS and ops.moe_wide_available(h, wgu[0], wgu[1], wd)
+    for weights in (None, w):
+        yk = torch.full((T, d), float("nan"), dtype=torch.float32, device="cuda")
+        ops.moe_experts(h, ids, wgu[0], wgu[1], wd, yk, weights=weights, weight_inputs=weights is not None)
+        for e in range(E):
+            t = (ids[:, 0] == e).nonzero()[:, 0]
+            x = h[t].double() * (1.0 if weights is None else weights[t].double())
+            z = x @ wgu[0, e].double().T
+            act = z * torch.sigmoid(z) * (x @ wgu[1, e].double().T)
+            # the gated values are rounded to bf16's eight bits, by 2^-8 of each at most; the rest is float32 (a tenth of that is far more)
+            bound = 1.1 * 2.0 ** -8 * (act.abs() @ wd[e].double().abs().T)
+            assert torch.isfinite(yk[t]).all() and ((yk[t].double() - act @ wd[e].double().T).abs() <= bound).all(), (e, counts[e])
+
+
 @pytest.mark.parametrize("gate,limit", [("silu", 0.0), ("clamped_swish", 0.8)])
 @pytest.mark.parametrize("T,d,F,E,top", [(700, 128, 192, 5, 2), (300, 64, 64, 9, 4), (2048, 256, 128, 6, 1)])
 def test_experts_of_many_rows_with_both_operands_through_lds(T, d, F, E, top, gate, limit):
     """More than 1,024 (token, k) rows in bf16 with widths that are multiples of 64 and the gates' and ups' matrices in
-    one tensor: tiles of 128 grouped rows; experts with no row, with a few, and with several tiles of rows."""
+    one tensor: tiles of up to 256 grouped rows; experts with no row, with a few, and with several tiles of rows."""
     from serve_amd import ops
     torch.manual_seed(T + E)
     h = torch.randn(T, d, device="cuda").bfloat16()
