@@ -461,7 +461,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
 // and 4-7, 8-11, 16-19, 28-31, and rows of 256 bytes and more then touch every bank once.
 // gridDim.z parts of K, each with sums [M, N] of its own.
 //
-// Measured, the float32 matrix instruction / this kernel in us (weights not in a cache): K 2048, 16,384 rows of W 43 / 32 at
+// Measured, the float32 matrix instruction / this kernel in us (weights not in a cache): K 2048, 16,384 rows of W 43 / 30 at
 // 24 rows of A, 65 / 41 at 64, 121 / 67 at 128; 3,072 rows of W in four parts 20 / 10, 2,048 in eight 8.7 / 8.3; K 8192, 2,048
 // rows in eight parts 24 / 19; 128,256 rows 315 / 219 at 24, 489 / 332 at 64, 965 / 550 at 128.  A step at 24 rows reads
 // its 134 MB at 4.2 TB/s; from 64 rows on the splits of A, which every workgroup makes again, weigh as much.  Distance to
@@ -535,8 +535,17 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
     src[d] = row < 32 * NT ? W + (size_t)min(n0 + row, N - 1) * K : A + (size_t)min(m0 + row - 32 * NT, M - 1) * K;
     col[d] = seg * 4;
   }
+  // Workgroups begin at different stages, which depend on the rows of W only: neighbours on a die one apart, dies an eighth of
+  // the walk.  Rows lie a power of two apart, so that the same columns of many rows are in one channel of a die's L2 and a few
+  // of the memory: 24 rows, four steps of the 1B shape 7.80 ms where all begin at the first column, 7.38 so, and 8.35 where a
+  // die's workgroups begin eight stages apart (as with the number of the workgroup modulo the stages).
+  const int ahead = n > 0 ? (int)(((blockIdx.x >> 3) + (blockIdx.x & 7) * (n >= 8 ? n >> 3 : 1)) % (unsigned)n) : 0;
+  auto stage_of = [&](int s) __attribute__((always_inline)) {
+    const int t = min(s, n - 1) + ahead;
+    return s_begin + (t >= n ? t - n : t);
+  };
   auto fetch = [&](int s) __attribute__((always_inline)) {    // (past the last stage it is loaded again, and not read)
-    const int k0 = (s_begin + min(s, n - 1)) * COLS;
+    const int k0 = stage_of(s) * COLS;
     unsigned char* at = ring + (s % NB) * STAGE + wave * ND * 1024;
 #pragma unroll
     for (int d = 0; d < ND; ++d)
@@ -576,8 +585,8 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
         const uint32_t off = (uint32_t)((s % NB) * STAGE);
         Frag8 wf[2], af[MT][2];
         read_rows<MT, NT>(wf, af, w0 + off, w1 + off, a0 + off, a1 + off);
-        const int k = (s_begin + s) * COLS + kc * 16 + h * 8;
-        if ((s_begin + s + 1) * COLS > K) {                    // the last columns: beyond K the operand of A is zero
+        const int at = stage_of(s), k = at * COLS + kc * 16 + h * 8;
+        if ((at + 1) * COLS > K) {                             // the last columns: beyond K the operand of A is zero
           const u32x4_t zero4 = {0u, 0u, 0u, 0u};
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) {
