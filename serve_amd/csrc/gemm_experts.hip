@@ -36,7 +36,7 @@ struct ExpertArgs {
   const bf16_t* A;
   const bf16_t* W;
   void* C;
-  int N, K, up_offset, gx, top, gate_kind;
+  int N, K, up_offset, gx, E, top, gate_kind;
   float gate_limit;
   const int* perm;
   const int* tile_expert;
@@ -224,7 +224,10 @@ __global__ __launch_bounds__(512, 2) void expert_product_kernel(ExpertArgs p) {
   // many rows are in a few channels of the memory (1,000 tokens, both products: 105 us so, 112 with an order that repeats from
   // die to die, 118 with one of eight places, 120 where all begin at the first column).
   const int nstages = p.K >> 6;
-  const int first = place + (nstages >= 8 ? nstages >> 3 : 1) * die;
+  // The place in a list of all experts' weight rows says where, not the one in the grid, so that a row's sums do not depend on
+  // what else is in the step.
+  const int u = e * p.gx + t - tile * p.gx, part = max(1, p.E * p.gx >> 3);
+  const int first = u % part + (nstages >= 8 ? nstages >> 3 : 1) * (u / part);
   if (M <= 32) expert_tile<CT, 1, FIRST>(p, expert_lds, e, row0, M, col0, first);
   else if (M <= 64) expert_tile<CT, 2, FIRST>(p, expert_lds, e, row0, M, col0, first);
   else if (M <= 128) expert_tile<CT, 4, FIRST>(p, expert_lds, e, row0, M, col0, first);
@@ -265,7 +268,7 @@ extern "C" int sa_expert_products(const void* h, const void* Wgu, const void* Wd
                                   hipStream_t stream) {
   if (E <= 0 || d <= 0 || F <= 0 || (d & 63) || (F & 63) || top <= 0) return SA_ERR_ARG;
   if (gate_kind < 0 || gate_kind >= SA_GATE_KINDS || (long long)E * F > 0x7fffffffLL) return SA_ERR_ARG;
-  ExpertArgs p = {(const bf16_t*)h, (const bf16_t*)Wgu, act, F, d, E * F, 0, top, gate_kind, gate_limit,
+  ExpertArgs p = {(const bf16_t*)h, (const bf16_t*)Wgu, act, F, d, E * F, 0, E, top, gate_kind, gate_limit,
                   perm, tile_expert, tile_row0, num_tiles, in_wts};
   // 256 weight rows a workgroup where that still gives most compute units one (every expert chosen), else 128
   const int cus = compute_units();
