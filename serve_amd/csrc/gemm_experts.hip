@@ -27,7 +27,6 @@ typedef const __attribute__((address_space(1))) void* gptr_t;
 // all but the newest n of this wave's loads have landed
 #define SA_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xf) | (((n) >> 4) << 14) | (0x7 << 4) | (0xf << 8))
 
-#define EX_TILE_ROWS 256
 #define EX_LDS (160 * 1024)        // of a workgroup, which has a compute unit to itself
 
 // FIRST: act[r] = gate(Wg_e x, Wu_e x) with x = A[perm[r] / top], W [2, E, N, K] (gates, then ups, `up_offset` rows apart).
@@ -255,9 +254,19 @@ static int launch(ExpertArgs p, int max_tiles, hipStream_t stream) {
   return 0;
 }
 
-extern "C" int sa_expert_tile_rows() { return EX_TILE_ROWS; }
+// The most rows of a tile (a multiple of 16), for `rows` (token, k) rows of E experts of width F: 256, so that an expert's matrices
+// are read once; 192 where the mean is so near 256 that some experts would have one tile and others two; 128 where there would be
+// too few tiles for the chip.  Both products with tiles of 128 / 192 / 256 rows, us: 32 experts of 2,048 x 1,024 at 3,600 rows
+// 171 / 110 / 109, at 6,000 164 / 191 / 138, at 8,000 232 / 170 / 229, at 10,000 233 / 194 / 193; 16 of them at 4,000 rows
+// 124 / 98 / 144; 64 of 4,096 x 1,536 at 8,800 rows 831 / 599 / 599, at 16,000 1,147 / 936 / 887; 8 of 2,048 x 1,024 at 1,400 rows
+// 49 / 69 / 69.
+extern "C" int sa_expert_tile_rows(int rows, int E, int F) {
+  const long long tiles = (rows + 255ll) / 256 > E ? (rows + 255ll) / 256 : E;
+  if (tiles * ((F + 63) / 64) * 4 < 3ll * compute_units()) return 128;
+  return rows > 230ll * E && rows < 300ll * E ? 192 : 256;
+}
 
-// Lists from sa_moe_group with tiles of sa_expert_tile_rows() rows at most (max_tiles: the grid's worst case, rows /
+// Lists from sa_moe_group with tiles of sa_expert_tile_rows(...) rows at most (max_tiles: the grid's worst case, rows /
 // tile rows + E).  bf16; d and F multiples of 64 (whole stages of K).
 //   gate/up: h [T, d] gathered by perm / top, Wgu [2, E, F, d] -> act [rows, F] = gate(gate, up)
 //            (in_wts, fp32 [T top] or null: both sums times the row's weight first, for weights on the experts' inputs)
@@ -273,7 +282,7 @@ extern "C" int sa_expert_products(const void* h, const void* Wgu, const void* Wd
   // 256 weight rows a workgroup where that still gives most compute units one (every expert chosen), else 128
   const int cus = compute_units();
   const int rc = (long long)E * ((F + 127) / 128) * 4 >= 3ll * cus ? launch<4, true>(p, max_tiles, stream)
-                                                                  : launch<2, true>(p, max_tiles, stream);
+                                                                    : launch<2, true>(p, max_tiles, stream);
   if (rc != 0) return rc;
   p.A = (const bf16_t*)act;
   p.W = (const bf16_t*)Wd;
@@ -282,5 +291,5 @@ extern "C" int sa_expert_products(const void* h, const void* Wgu, const void* Wd
   p.K = F;
   p.in_wts = nullptr;
   return (long long)E * ((d + 255) / 256) * 4 >= 3ll * cus ? launch<4, false>(p, max_tiles, stream)
-                                                           : launch<2, false>(p, max_tiles, stream);
+                                                              : launch<2, false>(p, max_tiles, stream);
 }

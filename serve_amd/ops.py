@@ -1458,6 +1458,18 @@ MOE_ROUTE_INSIDE = 16      # up to this many tokens the experts' call does the r
 MOE_WIDE_MIN_ROWS = 1024   # more (token, k) rows than this take the products with both operands through LDS
 
 
+def moe_wide_pays(rows: int, experts: int, expert_size: int) -> bool:
+    """Whether so many (token, k) rows go to the products with both operands through LDS where those can take them: from two rows an
+    expert on, with workgroups for half of the chip.  The kernels for few rows / those, us, experts x model width x expert width:
+    32 x 2048 x 1024 at 68, 160, 400 and 1,024 rows 75 / 66, 90 / 76, 115 / 77, 245 / 82; 64 x 4096 x 1024 at 40, 68 and 160 rows
+    158 / 195, 223 / 230, 276 / 269; 128 x 2048 x 512 at 160 and 400 118 / 126, 152 / 148; 8 x 2048 x 1024 at 68 and 160 38 / 32, 55 /
+    32; 8 x 1024 x 512 at 68 and 160 18.0 / 19.9, 23.7 / 20.5; 4 x 512 x 256 at 400 15 / 20."""
+    if rows > MOE_WIDE_MIN_ROWS:
+        return True
+    workgroups = experts * -(-expert_size // 64)
+    return rows > 64 and rows >= 2 * experts and (workgroups >= 128 or (workgroups >= 64 and rows >= 160))
+
+
 def moe_wide_available(h: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor) -> bool:
     """bf16, widths that are whole stages of 64, and the gates' and ups' matrices one behind the other in memory
     (`w_up` is the second half of the tensor whose first half is `w_gate`: [2, E, F, d])."""
@@ -1500,10 +1512,10 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, w_gate: torch.Tensor, w_up: 
     if weight_inputs:
         _check(weights is not None and weights.dtype == torch.float32 and weights.shape == (T, top)
                and weights.is_contiguous(), "weights on the experts' inputs must be contiguous fp32 [T, top]")
-    if n > MOE_WIDE_MIN_ROWS and logits is None and moe_wide_available(h, w_gate, w_up, w_down):
+    if moe_wide_pays(n, E, F) and logits is None and moe_wide_available(h, w_gate, w_up, w_down):
         # prompt portions: the grouping here, the two products over tiles of up to 256 rows with both operands through LDS
         wide = load_library("gemm_experts")
-        rows = int(wide.sa_expert_tile_rows())
+        rows = int(wide.sa_expert_tile_rows(c_int(n), c_int(E), c_int(F)))
         _ret(lib.sa_moe_group(_ptr(ids), _ptr(ints), c_int(T), c_int(top), c_int(E), c_int(rows), c_void_p(0), c_int(0),
                               c_void_p(0), c_int(0), c_float(1.0), c_void_p(0), c_int(outputs), _stream()), "moe_group")
         o = 4
