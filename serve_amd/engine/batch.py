@@ -134,6 +134,10 @@ def plan_step(segments: Sequence[Segment], cache: CacheManager, vocab_size: int,
     """
     if not segments:
         raise ValueError("a step needs at least one segment")
+    # the ids of portions as arrays, converted once; looked at one by one below only if any is outside the vocabulary
+    portions = [np.asarray(s.tokens) for s in segments if len(s.tokens) > 1]
+    portion_ids = np.concatenate(portions) if len(portions) > 1 else portions[0] if portions else None
+    ids_ok = portion_ids is None or (int(portion_ids.min()) >= 0 and int(portion_ids.max()) < vocab_size)
     seen = set()
     for s in segments:
         if len(s.tokens) == 0:
@@ -147,6 +151,8 @@ def plan_step(segments: Sequence[Segment], cache: CacheManager, vocab_size: int,
             raise KeyError(f"request {s.req_id!r} is not admitted")
         if len(s.tokens) == 1:
             lo = hi = int(s.tokens[0])
+        elif ids_ok:
+            lo = hi = 0
         else:
             arr = np.asarray(s.tokens)
             lo, hi = int(arr.min()), int(arr.max())
@@ -234,29 +240,24 @@ def plan_step(segments: Sequence[Segment], cache: CacheManager, vocab_size: int,
             rows[dead_np] = 0                   # an inert segment reads page 0, whatever it holds
         rows_of.append(rows)
         host[lay.block_tables[g]: lay.block_tables[g] + n * MP].reshape(n, MP)[:] = rows[:, :MP]
-    # per token: the single-token segments together, the others one by one
+    # per token
     q_np = np.asarray(q_lens)
+    real = int(cu_np[n])
+    seg_np = np.repeat(np.arange(n), q_np)
+    pos = np.arange(real) + (before_np - cu_np[:n])[seg_np]
     one = np.nonzero(q_np == 1)[0]
     if one.size:
-        at = cu_np[one]
-        b1 = before_np[one]
-        host[lay.token_ids + at] = [segments[i].tokens[0] for i in one]
-        host[lay.positions + at] = b1
-        host[lay.seg_of_token + at] = one
-        for g in range(G):
-            host[lay.slots[g] + at] = np.where(dead_np[one], -1, rows_of[g][one, b1 // ps] * ps + b1 % ps)
-    for i in np.nonzero(q_np != 1)[0]:
-        s, b, a, c0 = segments[i], before[i], after[i], int(cu_np[i])
-        m = a - b
-        host[lay.token_ids + c0: lay.token_ids + c0 + m] = np.asarray(s.tokens, dtype=np.int32)
-        host[lay.positions + c0: lay.positions + c0 + m] = np.arange(b, a, dtype=np.int32)
-        host[lay.seg_of_token + c0: lay.seg_of_token + c0 + m] = i
-        pos = np.arange(b, a)
-        for g in range(G):
-            if inert[i]:
-                host[lay.slots[g] + c0: lay.slots[g] + c0 + m] = -1
-            else:
-                host[lay.slots[g] + c0: lay.slots[g] + c0 + m] = rows_of[g][i, pos // ps] * ps + pos % ps
+        host[lay.token_ids + cu_np[one]] = [segments[i].tokens[0] for i in one]
+    if portion_ids is not None:
+        host[lay.token_ids: lay.token_ids + real][(q_np != 1)[seg_np]] = portion_ids
+    host[lay.positions: lay.positions + real] = pos
+    host[lay.seg_of_token: lay.seg_of_token + real] = seg_np
+    page, place = pos // ps, pos % ps
+    for g in range(G):
+        slots = rows_of[g][seg_np, page] * ps + place
+        if any_inert:
+            slots[dead_np[seg_np]] = -1
+        host[lay.slots[g]: lay.slots[g] + real] = slots
     cu = int(cu_np[n])
     for j in range(pad):           # inert segments: one token, one visible key, nothing stored
         i = B_real + j
@@ -275,6 +276,13 @@ def plan_step(segments: Sequence[Segment], cache: CacheManager, vocab_size: int,
     return lay, host, facts
 
 
+def upload(host: np.ndarray, device: torch.device) -> torch.Tensor:
+    """A step's arrays on the device, by a copy that the host does not wait for: out of pinned memory, which the
+    allocator keeps until the copy is done (out of ordinary memory the host would wait for all steps before it)."""
+    t = torch.from_numpy(host)
+    return t.pin_memory().to(device, non_blocking=True) if device.type == "cuda" else t.to(device)
+
+
 def context_from(lay: StepLayout, dev_buf: torch.Tensor, facts: dict) -> StepContext:
     v = lay.views(dev_buf)
     return StepContext(num_tokens=lay.T, num_segments=lay.B, num_logit_rows=lay.R, **v, **facts)
@@ -284,5 +292,5 @@ def build_step(segments: Sequence[Segment], cache: CacheManager, vocab_size: int
                device: torch.device) -> StepContext:
     """Plan the step and copy its arrays to the device."""
     lay, host, facts = plan_step(segments, cache, vocab_size)
-    dev = torch.from_numpy(host).to(device)
+    dev = upload(host, device)
     return context_from(lay, dev, facts)

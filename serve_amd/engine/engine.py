@@ -128,9 +128,12 @@ class Engine:
         gen = []
         for i, (r, t) in enumerate(zip(requests, temps)):
             ids = r.input_ids.tolist() if isinstance(r.input_ids, torch.Tensor) else list(r.input_ids)
+            array = None                          # (portions of long prompts: slices of an array, not lists made into one)
+            if len(ids) >= 256 and isinstance(r.input_ids, torch.Tensor) and r.input_ids.dtype == torch.int64 and r.input_ids.dim() == 1:
+                array = r.input_ids.cpu().numpy()
             if r.input_length != len(ids):
                 raise ValueError(f"request {i}: input_length {r.input_length} != len(input_ids) {len(ids)}")
-            gen.append(GenerationRequest(req_id=i, prompt=ids, max_new_tokens=int(r.max_new_tokens),
+            gen.append(GenerationRequest(req_id=i, prompt=ids, max_new_tokens=int(r.max_new_tokens), prompt_array=array,
                                          temperature=float(t), keep_logits=keep_last, keep_all_logits=keep_all))
         sched = Scheduler(self.runner, self.sampler, self.cfg, eos_token_ids=self.stop_ids(stop_token_ids),
                           record_steps=step_log is not None)

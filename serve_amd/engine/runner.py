@@ -20,7 +20,7 @@ from ..cache.storage import CacheStorage, bytes_per_page, group_windows
 from ..config.engine import EngineConfig
 from ..models.model import Model
 from ..parts.base import Runtime
-from .batch import INERT, Segment, StepLayout, context_from, plan_step
+from .batch import INERT, Segment, StepLayout, context_from, plan_step, upload
 
 # padded batch sizes for which decode-only steps are captured into graphs
 GRAPH_BATCHES = (1, 2, 4, 8, 16, 32, 48, 64, 80, 96, 112, 128, 160, 192, 256)
@@ -91,6 +91,8 @@ class DecodeHandle:
         self.host_tokens, self.event, self.n = host_tokens, event, n
 
     def tokens(self) -> List[int]:
+        if self.n == 0:                           # (nothing was sampled: nothing to wait for)
+            return []
         with trace.span("read_back"):
             self.event.synchronize()
             return self.host_tokens[: self.n].tolist()
@@ -193,7 +195,7 @@ class ModelRunner:
                 with trace.span("plan_step"):
                     lay, host, facts = plan_step(segments, self.cache, self.vocab_size)
                 with trace.span("stage_copy"):
-                    ctx = context_from(lay, torch.from_numpy(host).to(self.rt.device), facts)
+                    ctx = context_from(lay, upload(host, self.rt.device), facts)
                 with trace.span("launch"):
                     logits = self.model.forward(ctx, self.storage.layers)
                 ctx_lens = ctx.ctx_lens
@@ -577,6 +579,21 @@ class ModelRunner:
     @torch.inference_mode()
     def step_launch(self, req_ids: Sequence, tokens: Sequence[Sequence[Optional[int]]], samples: Sequence[bool],
                     temperatures: Sequence[float], keys: Sequence[int]) -> DecodeHandle:
+        return self._step_launch(req_ids, tokens, samples, temperatures, keys, graphs=True)[0]
+
+    def pays_to_launch_with_logits(self, counts: Sequence[int]) -> bool:
+        """Whether a step of so many tokens a request is better launched ahead of the host, kernel by kernel, when its logits
+        are kept: not one that `step` replays from a graph."""
+        return self._launch_ahead and sum(counts) > SMALL_TOKEN_PADS[-1] and any(n != 1 for n in counts)
+
+    @torch.inference_mode()
+    def step_launch_logits(self, req_ids: Sequence, tokens: Sequence[Sequence[Optional[int]]], samples: Sequence[bool],
+                           temperatures: Sequence[float], keys: Sequence[int]):
+        """`step_launch`, kernel by kernel, and beside the handle the fp32 logits [R, V] that the tokens are drawn from,
+        which are the caller's."""
+        return self._step_launch(req_ids, tokens, samples, temperatures, keys, graphs=False)
+
+    def _step_launch(self, req_ids, tokens, samples, temperatures, keys, graphs: bool):
         """Launch any step (prompt portions beside single tokens) with sampling on the device, and
         return at once: the eager counterpart of `decode_launch`.  tokens[i] are request i's next
         tokens; a single token may be None for "the token that the previous launch sampled for
@@ -588,7 +605,7 @@ class ModelRunner:
                 raise ValueError("only a single token can be left to the device")
             segments = [Segment(r, toks if toks[0] is not None else [0], [len(toks) - 1] if smp else [])
                         for r, toks, smp in zip(req_ids, tokens, samples)]
-            shape = self._mixed_shape(segments)
+            shape = self._mixed_shape(segments) if graphs else None
             if shape is not None:
                 nd, key = shape
                 src_of_token = [self._row_of[r] if toks[0] is None else -1 for r, toks in zip(req_ids, tokens)]
@@ -603,7 +620,7 @@ class ModelRunner:
                 ev.record()
                 for s in segments:
                     self.cache.trim(s.req_id, self.cache.tokens_of(s.req_id))
-                return DecodeHandle(host_tokens, ev, R)
+                return DecodeHandle(host_tokens, ev, R), None
             with trace.span("plan_step"):
                 lay, host, facts = plan_step(segments, self.cache, self.vocab_size)
             T, R = lay.T, lay.R
@@ -621,7 +638,7 @@ class ModelRunner:
                     src[cu[i]] = self._row_of[r]
             buf[off_temps: off_temps + R].view(np.float32)[:] = np.asarray(temperatures, dtype=np.float32)
             buf[off_keys: off_keys + 2 * R].view(np.int64)[:] = np.asarray(keys, dtype=np.int64)
-            dev = torch.from_numpy(buf).to(self.rt.device)
+            dev = upload(buf, self.rt.device)
             ctx = context_from(lay, dev, facts)
             ctx.src_row = dev[off_src: off_src + T]
             ctx.prev_tokens = self.sampled
@@ -640,5 +657,5 @@ class ModelRunner:
             ev.record()
         for r, n in zip(req_ids, facts["ctx_lens"]):
             self.cache.trim(r, n)
-        return DecodeHandle(host_tokens, ev, R)
+        return DecodeHandle(host_tokens, ev, R), logits
 

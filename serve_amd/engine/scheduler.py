@@ -46,6 +46,7 @@ class GenerationRequest:
     preemptions: int = 0
     # progress: tokens of prompt + generated that are in the cache
     fed: int = 0
+    prompt_array: object = None          # the prompt as an array of integers (optional): portions are slices of it
 
     def all_tokens(self) -> List[int]:
         return self.prompt + self.generated
@@ -54,7 +55,7 @@ class GenerationRequest:
         """Tokens a..b-1 of prompt + generated, without joining the two lists."""
         n = len(self.prompt)
         if b <= n:
-            return self.prompt[a:b]
+            return self.prompt_array[a:b] if self.prompt_array is not None and b - a > 1 else self.prompt[a:b]
         if a >= n:
             return self.generated[a - n: b - n]
         return self.prompt[a:] + self.generated[: b - n]
@@ -290,8 +291,8 @@ class Scheduler:
         if ahead == "decode":
             self._launch_decode(plan)
             return True
-        if ahead == "any":
-            self._launch_step(plan)
+        if ahead in ("any", "logits"):
+            self._launch_step(plan, ahead == "logits")
             return True
         self._resolve()                       # the tokens of the step in flight are needed on the host
         segments = []
@@ -321,19 +322,23 @@ class Scheduler:
     def _pipelinable(self, plan: StepPlan) -> Optional[str]:
         """Whether the step can be launched before the tokens of the step before it have reached
         the host, which then are fed back on the device: its finishing must not depend on the
-        tokens (no stop tokens), nobody keeps its logits, and a request whose last token is still
+        tokens (no stop tokens), and a request whose last token is still
         on the device must have got it from the step in flight.  "decode": single tokens that all
         sample, replayed from a graph; "any": prompt portions too, launched kernel by kernel;
-        None: the host needs the tokens first."""
+        "logits": the same where somebody keeps the logits, for steps that are not replayed from a graph
+        otherwise; None: the host needs the tokens first."""
         if not self.async_decode:
             return None
-        if any(r.keep_logits or r.keep_all_logits for r in plan.requests):
+        keep = any(r.keep_logits or r.keep_all_logits for r in plan.requests)
+        if keep and not getattr(self.runner, "pays_to_launch_with_logits", lambda counts: False)(plan.counts):
             return None
         if self._inflight is not None:
             before = {id(r) for r in self._inflight[1]}
             for r in plan.requests:
                 if r.generated and r.generated[-1] is None and id(r) not in before:
                     return None
+        if keep:
+            return "logits"
         if (self.runner.can_decode_async(len(plan.requests))
                 and all(n == 1 and s for n, s in zip(plan.counts, plan.samples))):
             return "decode"
@@ -341,24 +346,29 @@ class Scheduler:
             return "any"
         return None
 
-    def _launch_step(self, plan: StepPlan) -> None:
+    def _launch_step(self, plan: StepPlan, with_logits: bool = False) -> None:
         """A step with prompt portions, launched ahead of the host like `_launch_decode`."""
         from ..sampling.sampler import row_keys
         reqs = plan.requests
         tokens = [r.tokens_between(r.fed, r.fed + n) for r, n in zip(reqs, plan.counts)]
         samplers = [r for r, s in zip(reqs, plan.samples) if s]
         keys = row_keys(self.sampler.seed, [r.req_id for r in samplers], [len(r.generated) for r in samplers])
-        handle = self.runner.step_launch([r.req_id for r in reqs], tokens, plan.samples,
-                                         [r.temperature for r in samplers], keys)
+        launch = self.runner.step_launch_logits if with_logits else self.runner.step_launch
+        handle = launch([r.req_id for r in reqs], tokens, plan.samples, [r.temperature for r in samplers], keys)
+        handle, logits = handle if with_logits else (handle, None)
         previous, self._inflight = self._inflight, (handle, samplers, [len(r.generated) for r in samplers])
         self._record(reqs, plan.counts, samplers)
         self.steps += 1
         with trace.span("update_requests"):
             for r, n in zip(reqs, plan.counts):
                 r.fed += n
-            for r in samplers:
+            for i, r in enumerate(samplers):
                 r.generated.append(None)          # filled in when the step's tokens are read back
+                if r.keep_all_logits:
+                    r.logit_rows.append(logits[i].clone())
                 if r.done():
+                    if r.keep_logits:
+                        r.last_logits = logits[i].clone()
                     self._finish(r)
         if previous is not None:
             self._read_back(previous)

@@ -477,3 +477,39 @@ def test_which_small_steps_are_padded_and_replayed():
     assert shape([(1024, 1, one)] * 8 + [(0, 20, [19])]) is None
     assert shape([(900, 1, one)] * 8 + [(0, 20, [19])], state=True) is None
     assert shape([(0, 4, [3])] * 5, state=True) is None
+
+
+def test_plan_of_portions_given_as_lists_and_as_arrays():
+    """The host arrays of a step of single tokens, portions and an inert segment, told token by token; ids outside the vocabulary are
+    refused wherever they stand."""
+    from serve_amd.engine.batch import INERT
+
+    def fresh():
+        c = CacheManager([None], [64], 4, 8, 16)
+        for r in range(3):
+            c.admit(r)
+        assert c.ensure(1, 7)
+        return c
+    ids = [list(range(5, 14)), [3], [9, 8, 7], [0, 0]]
+    for make in (list, np.asarray):
+        c = fresh()
+        segs = [Segment(0, make(ids[0]), [8]), Segment(1, [3], [0]), Segment(2, make(ids[2]), []), Segment(INERT, make(ids[3]), [])]
+        lay, host, facts = plan_step(segs, c, 100, pad_segments_to=5)
+        at, want = 0, {"token_ids": [], "positions": [], "seg_of_token": [], "slots": []}
+        for i, (s, begin) in enumerate(zip(segs, (0, 7, 0, 0))):
+            for k, t in enumerate(s.tokens):
+                want["token_ids"].append(int(t))
+                want["positions"].append(begin + k)
+                want["seg_of_token"].append(i)
+                table = [] if s.req_id is INERT else c.block_table(s.req_id)
+                want["slots"].append(-1 if s.req_id is INERT else table[(begin + k) // 4] * 4 + (begin + k) % 4)
+        for name, values in want.items():
+            off = lay.slots[0] if name == "slots" else getattr(lay, name)
+            assert host[off: off + len(values)].tolist() == values, name
+        assert facts["q_lens"] == [9, 1, 3, 2, 1] and host[lay.logit_rows: lay.logit_rows + 2].tolist() == [8, 9]
+        for bad in (-1, 100):
+            for place in (0, 2):
+                wrong = [list(x) for x in ids]
+                wrong[place][1] = bad
+                with pytest.raises(ValueError, match="outside the vocabulary"):
+                    plan_step([Segment(i, make(x), []) for i, x in enumerate(wrong[:3])], fresh(), 100)

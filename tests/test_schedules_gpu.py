@@ -651,3 +651,34 @@ def test_graphs_of_small_steps_keep_to_their_share(tmp_path):
     for n in counts[:7]:
         decode(n)
     assert [k for k in graphs if k[0] != "small"] == kept and len(small()) == 1
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_prompt_steps_that_keep_logits_run_ahead_of_the_host(tmp_path, dtype):
+    """Steps of more than 64 tokens with prompt portions are launched before the host has the tokens of those before, the last and
+    all logits among them: the same tokens and logits, bit for bit, as with the host in step."""
+    from serve_amd.engine.engine import Request
+    folder = util.make_folder(tmp_path, "A")
+    engine = make_engine(folder, dtype, page_size=4, num_pages=400, max_context=256, max_requests=8, max_tokens_per_step=80,
+                         prefill_chunk=72)
+    rng = random.Random(31)
+    prompts = [util.random_tokens(rng, n, 255) for n in (200, 3, 90, 1, 150, 40)]
+    reqs = [Request(torch.tensor(p), len(p), n) for p, n in zip(prompts, (1, 4, 3, 6, 2, 1))]
+    ahead = []
+    launch = engine.runner.step_launch_logits
+    engine.runner.step_launch_logits = lambda *a: ahead.append(len(a[0])) or launch(*a)
+    for keep in ("last", "all"):
+        for temperature in (0.0, 0.8):
+            ahead.clear()
+            out = engine.generate(reqs, temperature=temperature, return_logits=keep)
+            assert len(ahead) >= 4, "no step was launched ahead"
+            ahead.clear()
+            engine.cfg.async_decode = False
+            want = engine.generate(reqs, temperature=temperature, return_logits=keep)
+            engine.cfg.async_decode = True
+            assert not ahead
+            for a, b in zip(out, want):
+                assert a.error is None and a.generated_tokens.tolist() == b.generated_tokens.tolist()
+                assert torch.equal(a.logits, b.logits)
+    engine.runner.cache.check_invariants()
+    assert not engine.runner.cache.live_requests()
