@@ -19,12 +19,16 @@ __device__ __forceinline__ float bf16_bits_to_float(uint32_t bits16) {
   return __uint_as_float(bits16 << 16);
 }
 
-// round to nearest even; NaN stays NaN
+// Round to nearest even, NaN stays NaN: the conversion instruction, for one number and for two side by side (written out on the
+// bits it is eight instructions and a branch a number).
 __device__ __forceinline__ uint16_t float_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x0040u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+  return __builtin_bit_cast(uint16_t, (__bf16)f);
+}
+typedef float sa_float2_t __attribute__((ext_vector_type(2)));
+typedef __bf16 sa_bf16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t floats_to_bf16_bits(float first, float second) {
+  const sa_float2_t f = {first, second};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, sa_bf16x2_t));
 }
 
 __device__ __forceinline__ float to_float(float x) { return x; }
@@ -131,6 +135,28 @@ __device__ __forceinline__ float short_sigmoid(float z) {
   return __builtin_amdgcn_rcpf(1.f + short_exp(fminf(-z, 80.f)));
 }
 __device__ __forceinline__ float short_silu(float z) { return z * short_sigmoid(z); }
+
+// The same for any x, infinities and overflow among them (the correction is kept within -1 .. 1, which it exceeds nowhere
+// else), and with it gate_mul for results that are rounded to bf16: 10 instructions a silu and two at a quarter of the rate,
+// where expf and a division are 28 and two.  Within a few units in the last place of float32.
+__device__ __forceinline__ float any_exp(float x) {
+  const float L2E = 1.44269502162933349609375f, L2E_LO = 1.925963033500011e-8f;
+  const float t = x * L2E;
+  float r = fmaf(x, L2E, -t);
+  r = __builtin_amdgcn_fmed3f(fmaf(x, L2E_LO, r), -1.f, 1.f);
+  return __builtin_amdgcn_exp2f(t) * fmaf(r, 0.693147182464599609375f, 1.f);
+}
+template <int KIND>
+__device__ __forceinline__ float short_gate(float g, float u, float limit) {
+  float z = g;
+  if (KIND == SA_GATE_GELU_TANH) z = 1.5957691216057308f * (g + 0.044715f * g * g * g);   // (1 + tanh(s)) / 2 = sigmoid(2 s)
+  if (KIND == SA_GATE_CLAMPED_SWISH) {
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit) + 1.f;
+    z = 1.702f * g;
+  }
+  return g * __builtin_amdgcn_rcpf(1.f + any_exp(-z)) * u;
+}
 
 // the first key that a query at position p sees: of its own run of `chunk` positions (counted from position 0) where
 // chunk > 0, of the last `window` keys where window > 0, else the first of all

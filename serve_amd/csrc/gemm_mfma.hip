@@ -106,8 +106,8 @@ __device__ __forceinline__ void store4(float* p, const float (&v)[4], bool vec) 
 __device__ __forceinline__ void store4(bf16_t* p, const float (&v)[4], bool vec) {
   if (vec) {
     uint2 u;
-    u.x = (uint32_t)float_to_bf16_bits(v[0]) | ((uint32_t)float_to_bf16_bits(v[1]) << 16);
-    u.y = (uint32_t)float_to_bf16_bits(v[2]) | ((uint32_t)float_to_bf16_bits(v[3]) << 16);
+    u.x = floats_to_bf16_bits(v[0], v[1]);
+    u.y = floats_to_bf16_bits(v[2], v[3]);
     *reinterpret_cast<uint2*>(p) = u;
   } else {
 #pragma unroll

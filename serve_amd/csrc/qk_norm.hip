@@ -129,7 +129,7 @@ __device__ __forceinline__ void store8(bf16_t* p, const float (&v)[8]) {
   uint32_t w[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k)
-    w[k] = (uint32_t)float_to_bf16_bits(v[2 * k]) | ((uint32_t)float_to_bf16_bits(v[2 * k + 1]) << 16);
+    w[k] = floats_to_bf16_bits(v[2 * k], v[2 * k + 1]);
   *reinterpret_cast<uint4*>(p) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
@@ -330,7 +330,7 @@ __device__ __forceinline__ uint4 pack8(const float* f) {
   uint32_t w[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k)
-    w[k] = (uint32_t)float_to_bf16_bits(f[2 * k]) | ((uint32_t)float_to_bf16_bits(f[2 * k + 1]) << 16);
+    w[k] = floats_to_bf16_bits(f[2 * k], f[2 * k + 1]);
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 

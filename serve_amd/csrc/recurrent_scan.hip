@@ -946,8 +946,8 @@ __device__ __forceinline__ float4 rs_ld4(const bf16_t* p) {
 __device__ __forceinline__ void rs_st4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ __forceinline__ void rs_st4(bf16_t* p, float4 v) {
   uint2 u;
-  u.x = (uint32_t)float_to_bf16_bits(v.x) | ((uint32_t)float_to_bf16_bits(v.y) << 16);
-  u.y = (uint32_t)float_to_bf16_bits(v.z) | ((uint32_t)float_to_bf16_bits(v.w) << 16);
+  u.x = floats_to_bf16_bits(v.x, v.y);
+  u.y = floats_to_bf16_bits(v.z, v.w);
   *reinterpret_cast<uint2*>(p) = u;
 }
 

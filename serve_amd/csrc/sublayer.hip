@@ -97,8 +97,8 @@ __device__ __forceinline__ float4 ld4(const bf16_t* p) {
 __device__ __forceinline__ void st4(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 __device__ __forceinline__ void st4(bf16_t* p, float4 v) {
   uint2 u;
-  u.x = (uint32_t)float_to_bf16_bits(v.x) | ((uint32_t)float_to_bf16_bits(v.y) << 16);
-  u.y = (uint32_t)float_to_bf16_bits(v.z) | ((uint32_t)float_to_bf16_bits(v.w) << 16);
+  u.x = floats_to_bf16_bits(v.x, v.y);
+  u.y = floats_to_bf16_bits(v.z, v.w);
   *reinterpret_cast<uint2*>(p) = u;
 }
 
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(256) void activation_bf16x8_kernel(bf16_t* __restri
     for (int k = 0; k < 4; ++k) {
       const float z0 = bf16_bits_to_float(w[k] & 0xffffu), z1 = bf16_bits_to_float(w[k] >> 16);
       const float r0 = activate(z0, kind), r1 = activate(z1, kind);
-      w[k] = (uint32_t)float_to_bf16_bits(r0) | ((uint32_t)float_to_bf16_bits(r1) << 16);
+      w[k] = floats_to_bf16_bits(r0, r1);
     }
     *reinterpret_cast<uint4*>(a + gi * 8) = make_uint4(w[0], w[1], w[2], w[3]);
   }
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(256) void sigmoid_mul_bf16x8_kernel(bf16_t* __restr
     for (int k = 0; k < 4; ++k) {
       const float r0 = bf16_bits_to_float(aw[k] & 0xffffu) / (1.f + expf(-bf16_bits_to_float(gw[k] & 0xffffu)));
       const float r1 = bf16_bits_to_float(aw[k] >> 16) / (1.f + expf(-bf16_bits_to_float(gw[k] >> 16)));
-      w[k] = (uint32_t)float_to_bf16_bits(r0) | ((uint32_t)float_to_bf16_bits(r1) << 16);
+      w[k] = floats_to_bf16_bits(r0, r1);
     }
     *reinterpret_cast<uint4*>(a + gi * 8) = make_uint4(w[0], w[1], w[2], w[3]);
   }

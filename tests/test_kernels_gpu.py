@@ -723,6 +723,56 @@ def test_silu_mul(dtype):
     assert out[0].abs().max().item() == 0
 
 
+@pytest.mark.parametrize("kind,limit", [("silu", 0.0), ("gelu_tanh", 0.0), ("clamped_swish", 7.0)])
+def test_gates_of_every_bf16_number(kind, limit):
+    """The gates for bf16 results at all 65,536 numbers, infinities and NaN among them: within bf16's rounding of 64 bits, and not a
+    number where the plain formula is not."""
+    from serve_amd import ops
+    g = torch.arange(65536, dtype=torch.int32, device=DEV).to(torch.int16).view(torch.bfloat16)
+    u = torch.tensor([1.0, -3.0, 0.0, 2.0 ** -20, float("inf"), float("nan")], device=DEV).bfloat16()
+    gu = torch.cat([g.expand(6, -1), u[:, None].expand(-1, 65536)], 1).contiguous()
+    out = torch.empty((6, 65536), dtype=torch.bfloat16, device=DEV)
+    ops.gate_mul(gu, out, kind, limit)
+
+    def plain(x, y):
+        if kind == "gelu_tanh":
+            return 0.5 * x * (1 + torch.tanh(math.sqrt(2 / math.pi) * (x + 0.044715 * x ** 3))) * y
+        if kind == "clamped_swish":
+            x, y = x.clamp(max=limit), y.clamp(-limit, limit)
+            return x / (1 + torch.exp(-1.702 * x)) * (y + 1)
+        return x / (1 + torch.exp(-x)) * y
+    want = plain(g.double()[None], u.double()[:, None])
+    if kind == "gelu_tanh":                      # (without the cancellation of 1 + tanh)
+        want = g.double()[None] * torch.sigmoid(2 * math.sqrt(2 / math.pi) * (g.double() + 0.044715 * g.double() ** 3)) * u.double()[:, None]
+    nan = torch.isnan(plain(g.float()[None], u.float()[:, None]))
+    # clamping keeps a NaN in torch and may drop it in the kernel's minimum; beyond 80 below zero a gate is nothing, e^-80 of its size
+    sure = ~torch.isnan(g)[None] & ~torch.isnan(u)[:, None] if kind == "clamped_swish" else torch.ones_like(nan)
+    # (the plain formula overflows in float32 at the largest numbers: infinity times zero)
+    far = (g.abs().float() > 2.0 ** 40)[None] & ~torch.isinf(g)[None] & ~torch.isnan(g)[None]
+    # (where a gate is nothing, which of kernel and formula has come to zero first decides whether infinity times it is a number)
+    far = far | (torch.isinf(u)[:, None] & (plain(g.double(), torch.ones_like(g).double()).abs() < 1e-5)[None])
+    assert torch.equal(torch.isnan(out)[sure & ~far], nan[sure & ~far])
+    ok = ~nan & ~torch.isnan(out) & torch.isfinite(want) & (want.abs() < 3e38)
+    err = (out.double() - want).abs()
+    # half a unit of eight bits, and float32's few roundings; a sigmoid below the normal range (2^-126) may come out as zero
+    tiny = 2.0 ** -125 * (1 + g.double().abs()[None]) * (1 + u.double().abs()[:, None])
+    assert (err <= (2.0 ** -8 * (1 + 2.0 ** -10)) * want.abs() + tiny)[ok].all()
+
+
+def test_rounding_to_bf16_is_to_the_nearest_even():
+    """Products of two bf16 numbers have up to 16 bits: gates of 64 and more are their own silu, so the kernel's results are those
+    products rounded, for all numbers of one operand and every mantissa of the other."""
+    from serve_amd import ops
+    u = torch.arange(65536, dtype=torch.int32, device=DEV).to(torch.int16).view(torch.bfloat16)
+    for g in torch.arange(0x4280, 0x4300, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).tolist():
+        gu = torch.cat([torch.full((65536,), g, dtype=torch.bfloat16, device=DEV), u])[None].contiguous()
+        out = torch.empty((1, 65536), dtype=torch.bfloat16, device=DEV)
+        ops.silu_mul(gu, out)
+        want = (u.float() * g).bfloat16()
+        assert torch.equal(torch.isnan(out[0]), torch.isnan(want))
+        assert torch.equal(out[0].view(torch.int16)[~torch.isnan(want)], want.view(torch.int16)[~torch.isnan(want)])
+
+
 @pytest.mark.parametrize("V,shift", [(1000, 0), (1001, 0), (1000, 1), (6152, 0), (128256, 0), (70001, 0)])
 def test_sample_greedy_and_ties(V, shift):
     """One chunk and many; vocabularies of whole groups of four from an aligned address (read 16 bytes a lane,
