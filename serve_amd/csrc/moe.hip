@@ -54,6 +54,48 @@ __device__ __forceinline__ void route_token(const float* __restrict__ z, int* __
                                             int E, int top, int lane, int mode, float wscale,
                                             const float* __restrict__ corr) {
   const int over_all = mode == 1;
+  if (E <= SA_WAVE) {
+    // an output a lane: the largest through the register file, and of the lanes that hold it the first (the general form below
+    // goes through the outputs and six exchanges of value and place for each choice, and reads the weights back from memory:
+    // with it the kernel of product and routing takes 19 us for 1,000 tokens, 32 outputs, four chosen, so 12)
+    const float own = lane < E ? z[lane] : -INFINITY;
+    float v = own, big = 0.f, all = 1.f, mine = 0.f;
+    if (corr) {
+      big = wave_max(own);
+      all = wave_sum(lane < E ? expf(own - big) : 0.f);
+      mine = expf(own - big) / all;
+      v = lane < E ? mine + corr[lane] : -INFINITY;
+    }
+    bool left = lane < E;
+    float first = 0.f, sum = 0.f, weight = 0.f;              // (lane k keeps the k-th choice)
+    int choice = 0;
+    for (int k = 0; k < top; ++k) {
+      const float bv = wave_max(left ? v : -INFINITY);
+      const unsigned long long at = __ballot(left && v == bv);
+      int bi = at ? (int)__builtin_ctzll(at) : 0x7fffffff;   // (logits that are no numbers are not chosen)
+      if (k == 0) first = bv;
+      float p;
+      if (corr) {
+        bi = min(bi, E - 1);
+        p = __shfl(mine, bi, SA_WAVE);
+      } else {
+        p = mode == 2 ? 1.f / (1.f + expf(-bv)) : expf(bv - first);
+      }
+      sum += p;
+      if (lane == k) {
+        choice = bi;
+        weight = p;
+      }
+      if (lane == bi) left = false;
+    }
+    if (over_all && !corr) all = wave_sum(lane < E ? expf(own - first) : 0.f);
+    if (lane >= top) return;
+    ids[lane] = choice;
+    if (corr) wts[lane] = (weight / (sum + 1e-20f)) * wscale;
+    else if (mode == 2) wts[lane] = weight * wscale;
+    else wts[lane] = ((over_all ? weight / all : weight) / (over_all ? sum / all + 1e-20f : sum)) * wscale;
+    return;
+  }
   if (corr) {
     // shares of the softmax first: what is chosen is their sum with the correction
     float big = -INFINITY;
@@ -585,6 +627,96 @@ __global__ __launch_bounds__(256) void moe_combine_vec_kernel(const float* __res
 
 // the most tiles a step can have, at the smallest tile (16 rows): what the scratch arrays are sized for
 extern "C" int sa_moe_max_tiles(int rows, int E) { return (rows + 15) / 16 + E; }
+
+// ---------------------------------------------------------------------------------------------
+// The router's product and the routing in one kernel, bf16: a workgroup takes 16 tokens, its eight waves an eighth of the
+// columns each (tiles as in the products below: 16 of the router's rows by 16 tokens), the sums meet in LDS, go to `logits`
+// [T, N] and are routed from there, a wave a token in turn.  What bounds it is its chain: one trip or two for the operands, the
+// sums, `top` maxima.  1,000 tokens, 33 x 2,048, four of 32: the BLAS library's product 11 us and the routing 7.4 / this 12.
+// Whole feed-forward of 64 tokens, where the product of few rows had two workgroups, 118 / 112.
+// ---------------------------------------------------------------------------------------------
+#define MOE_ROUTER_MAX_ROWS 96         // of the router's matrix: what the sums have room for in LDS
+template <int NT>
+__global__ __launch_bounds__(512) void moe_router_kernel(const bf16_t* __restrict__ h, const bf16_t* __restrict__ W,
+                                                         float* __restrict__ logits, int* __restrict__ ids,
+                                                         float* __restrict__ wts, int T, int N, int K, int E, int top, int mode,
+                                                         float wscale, const float* __restrict__ corr) {
+  constexpr int KU = NT <= 3 ? 8 : 4;                       // steps of 32 columns loaded before their products
+  __shared__ float red[8][16 * NT][17];
+  __shared__ float z[16][16 * NT + 1];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+  const int t0 = blockIdx.x * 16;
+  const int steps = (K + 31) >> 5, per = (steps + 7) >> 3;
+  const int end = min(steps, (wave + 1) * per);
+  const bf16_t* arow = h + (size_t)min(t0 + c, T - 1) * K;  // (rows beyond T and N are read from the last and never used)
+  const bf16_t* wrow[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) wrow[nt] = W + (size_t)min(nt * 16 + c, N - 1) * K;
+  moe_floatx4_t acc[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) acc[nt] = (moe_floatx4_t){0.f, 0.f, 0.f, 0.f};
+  const moe_u32x4_t zero = {0u, 0u, 0u, 0u};
+  for (int s = wave * per; s < end; s += KU) {
+    MoeFrag af[KU], wf[KU][NT];
+#pragma unroll
+    for (int u = 0; u < KU; ++u) {
+      const int k = min((s + u) * 32 + g * 8, K - 8);
+      af[u].r = *reinterpret_cast<const moe_u32x4_t*>(arow + k);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) wf[u][nt].r = *reinterpret_cast<const moe_u32x4_t*>(wrow[nt] + k);
+    }
+    if (s + KU > end || (s + KU) * 32 > K) {                // beyond the columns the operand of h is zero
+#pragma unroll
+      for (int u = 0; u < KU; ++u) af[u].r = s + u < end && (s + u) * 32 + g * 8 < K ? af[u].r : zero;
+    }
+#pragma unroll
+    for (int u = 0; u < KU; ++u)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][nt].v, af[u].v, acc[nt], 0, 0, 0);
+  }
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wave][nt * 16 + 4 * g + r][c] = acc[nt][r];
+  __syncthreads();
+  for (int i = threadIdx.x; i < 256 * NT; i += 512) {
+    const int t = i / (16 * NT), n = i - t * (16 * NT);
+    float sum = red[0][n][t];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) sum += red[w][n][t];
+    z[t][n] = sum;
+    if (t0 + t < T && n < N) logits[(size_t)(t0 + t) * N + n] = sum;
+  }
+  __syncthreads();
+  for (int t = wave; t < 16 && t0 + t < T; t += 8)
+    route_token(z[t], ids + (size_t)(t0 + t) * top, wts + (size_t)(t0 + t) * top, E, top, lane, mode, wscale, corr);
+}
+
+extern "C" int sa_moe_router_max_rows() { return MOE_ROUTER_MAX_ROWS; }
+
+// h bf16 [T, K], W bf16 [N, K] (N up to sa_moe_router_max_rows(), of which the first E are the router's outputs), K % 8 == 0,
+// 16-byte aligned -> logits fp32 [T, N], ids, wts as sa_moe_route makes them.
+extern "C" int sa_moe_router(const void* h, const void* W, float* logits, int* ids, float* wts, int T, int N, int K, int E, int top,
+                             int mode, float wscale, const float* corr, hipStream_t stream) {
+  if (T <= 0) return 0;
+  if (N <= 0 || N > MOE_ROUTER_MAX_ROWS || K < 8 || (K & 7) || E <= 0 || E > N || top <= 0 || top > E || (corr && mode != 1) ||
+      ((((uintptr_t)h | (uintptr_t)W) & 15) != 0))
+    return SA_ERR_ARG;
+#define GO(NT)                                                                                                              \
+  hipLaunchKernelGGL(moe_router_kernel<NT>, dim3((T + 15) / 16), dim3(512), 0, stream, (const bf16_t*)h, (const bf16_t*)W, \
+                     logits, ids, wts, T, N, K, E, top, mode, wscale, corr)
+  switch ((N + 15) / 16) {
+    case 1: GO(1); break;
+    case 2: GO(2); break;
+    case 3: GO(3); break;
+    case 4: GO(4); break;
+    case 5: GO(5); break;
+    default: GO(6); break;
+  }
+#undef GO
+  SA_LAUNCH_CHECK();
+  return 0;
+}
 
 extern "C" int sa_moe_route(const float* logits, int ldz, int* ids, float* wts, int T, int E, int top,
                             int over_all, float wscale, const float* corr, hipStream_t stream) {

@@ -1448,6 +1448,30 @@ def moe_route(logits: torch.Tensor, experts: int, top: int, ids: torch.Tensor, w
                           c_int(top), c_int(_router_mode(over_all)), c_float(scale), _ptr(correction), _stream()), "moe_route")
 
 
+def moe_router_available(h: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether `moe_router` takes these: bf16, inner size a multiple of 8, up to 96 rows of the router's matrix."""
+    return (h.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and h.dim() == 2 and h.shape[0] > 0 and h.is_contiguous()
+            and w.is_contiguous() and h.shape[1] % 8 == 0 and h.shape[1] > 0
+            and 0 < w.shape[0] <= int(load_library("moe").sa_moe_router_max_rows()) and _aligned16(h, w))
+
+
+def moe_router(h: torch.Tensor, w: torch.Tensor, experts: int, logits: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
+               over_all=False, scale: float = 1.0, correction: Optional[torch.Tensor] = None) -> None:
+    """logits fp32 [T, N] = h @ w^T, and from its first `experts` columns `ids` and `weights` as `moe_route` makes them."""
+    _dev(h, w, logits, ids, weights, correction)
+    T, K = h.shape
+    N, top = w.shape[0], ids.shape[1]
+    _check_correction(correction, experts, over_all)
+    _check(w.shape[1] == K and moe_router_available(h, w), "moe_router takes bf16 rows of a multiple of 8, and up to 96 of the router's")
+    _check(logits.dtype == torch.float32 and logits.shape == (T, N) and logits.is_contiguous(), "router logits must be fp32 [T, N]")
+    _check(0 < top <= experts <= N, "top must be within the number of experts")
+    _check(ids.dtype == torch.int32 and ids.shape == (T, top) and ids.is_contiguous() and weights.dtype == torch.float32
+           and weights.shape == (T, top) and weights.is_contiguous(), "ids int32 [T, top], weights fp32 [T, top]")
+    lib = load_library("moe")
+    _ret(lib.sa_moe_router(_ptr(h), _ptr(w), _ptr(logits), _ptr(ids), _ptr(weights), c_int(T), c_int(N), c_int(K), c_int(experts),
+                           c_int(top), c_int(_router_mode(over_all)), c_float(scale), _ptr(correction), _stream()), "moe_router")
+
+
 def _check_correction(correction: Optional[torch.Tensor], outputs: int, over_all) -> None:
     if correction is not None:
         _f32vec(correction, outputs, "the router's correction")

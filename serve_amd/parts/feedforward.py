@@ -148,16 +148,22 @@ class RoutedExperts(Part):
         """[T, d]; with `rows_ok`, where `leaves_rows` says so, an `ops.ExpertRows` that the caller adds up."""
         T, d = h.shape
         dev = h.device
-        logits = linear(h, self.w_router, out_dtype=torch.float32)
         ids = torch.empty((T, self.top), dtype=torch.int32, device=dev)
         weights = torch.empty((T, self.top), dtype=torch.float32, device=dev)
+        routed = T > ops.MOE_ROUTE_INSIDE and ops.moe_router_available(h, self.w_router)
+        if routed:
+            logits = torch.empty((T, self.w_router.shape[0]), dtype=torch.float32, device=dev)
+            ops.moe_router(h, self.w_router, self.outputs, logits, ids, weights, self.over_all, self.router_scale, self.choice)
+        else:
+            logits = linear(h, self.w_router, out_dtype=torch.float32)
         yk = torch.empty((T * self.top, d), dtype=torch.float32, device=dev)
         if T <= ops.MOE_ROUTE_INSIDE:
             ops.moe_experts(h, ids, self.w_gate, self.w_up, self.w_down, yk, logits, weights, self.over_all,
                             self.router_scale, self.activation, self.limit, self.weight_inputs, self.choice,
                             self.outputs)    # routes, too
         else:
-            ops.moe_route(logits, self.outputs, self.top, ids, weights, self.over_all, self.router_scale, self.choice)
+            if not routed:
+                ops.moe_route(logits, self.outputs, self.top, ids, weights, self.over_all, self.router_scale, self.choice)
             ops.moe_experts(h, ids, self.w_gate, self.w_up, self.w_down, yk, weights=weights, gate=self.activation,
                             limit=self.limit, weight_inputs=self.weight_inputs, outputs=self.outputs)
         if rows_ok and self.leaves_rows:

@@ -573,6 +573,30 @@ def test_steps_with_prompt_portions_replayed_from_graphs(tmp_path, dtype):
     assert compared > 3 * count
 
 
+@pytest.mark.parametrize("T,N,K,E,top", [(1, 1, 8, 1, 1), (15, 17, 40, 17, 2), (16, 16, 256, 16, 1), (17, 33, 2048, 32, 4), (33, 48, 1000, 40, 4),
+                                         (100, 65, 4096, 64, 6), (47, 80, 2056, 80, 4), (1000, 96, 264, 90, 8)])
+@pytest.mark.parametrize("mode", ["chosen", "all", "sigmoid"])
+def test_router_product_with_the_routing(T, N, K, E, top, mode):
+    """One kernel for the router's logits and what is chosen by them: the logits against 64 bits, the choice as the routing kernel
+    makes it from the same logits; rows of the matrix, tokens and columns that are no whole tiles or steps."""
+    from serve_amd import ops
+    g = torch.Generator("cuda").manual_seed(T + N + K)
+    h = torch.randn((T, K), device="cuda", generator=g).bfloat16()
+    w = (torch.randn((N, K), device="cuda", generator=g) * K ** -0.5).bfloat16()
+    corr = torch.randn((E,), device="cuda", generator=g) * 0.02 if mode == "all" else None
+    assert ops.moe_router_available(h, w)
+    logits = torch.full((T, N), float("nan"), dtype=torch.float32, device="cuda")
+    ids, weights = torch.full((T, top), -1, dtype=torch.int32, device="cuda"), torch.full((T, top), float("nan"), device="cuda")
+    ops.moe_router(h, w, E, logits, ids, weights, mode, 1.5, corr)
+    size = h.double().abs() @ w.double().abs().T
+    # a rounding of a running sum, at most `size`, for every 32 columns and the eight sums that are joined (and the truncation inside
+    # a step: counted as another)
+    assert ((logits.double() - h.double() @ w.double().T).abs() <= size * (2 * (K / 32 + 1) + 8) * 2.0 ** -24).all()
+    want_ids, want = torch.empty_like(ids), torch.empty_like(weights)
+    ops.moe_route(logits, E, top, want_ids, want, mode, 1.5, corr)
+    assert torch.equal(ids, want_ids) and torch.allclose(weights, want, rtol=1e-6, atol=0)
+
+
 # (256 compute units)  128 weight rows a workgroup in both products; 256 in the first, in both, and in the second, over one stage and more
 @pytest.mark.parametrize("d,F,E", [(64, 64, 14), (128, 2048, 14), (1152, 3264, 15), (3392, 192, 14)])
 def test_experts_products_at_the_edges_of_tiles(d, F, E):
