@@ -271,10 +271,11 @@ extern "C" int sa_add_rmsnorm(float* x, const void* delta, int delta_dtype, int 
 // `parts` > 1 (fp32): the rows are partial sums of a product, `part_stride` elements apart, which are added in order; the
 // finished queries go to the first part's rows.
 //
-// What bounds it: a chain of trips (position, sums, angle, store) and the exact sine and cosine.  A thread therefore takes one
-// pair or one value, in gridDim.y workgroups a token, and loads up to eight sums at once; threads that went through a token's
-// pairs and then through its values took, 24 tokens of 40 heads of 64 in four parts, 8.2 us where this takes 5.0, and 1,050
-// tokens 15.2 where this takes 12.
+// What bounds it: a chain of trips (position, sums, angle, store) and the exact sine and cosine.  In a step of few tokens a
+// thread therefore takes one pair or one value, in gridDim.y workgroups a token, and loads up to eight sums at once: threads that
+// went through a token's pairs and then through its values took, 24 tokens of 40 heads of 64 in four parts, 8.2 us where this
+// takes 5.1.  Many tokens fill the chip by themselves, with up to four workgroups each: 1,164 tokens 16.6 / 16.2 / 15.7 / 17.2 us with
+// one, two, four and seven.
 template <typename TA, typename TC>
 __global__ void rope_kv_write_kernel(TA* __restrict__ qkv, const int* __restrict__ positions,
                                      const float* __restrict__ inv_freq, const int* __restrict__ slot,
@@ -443,7 +444,8 @@ extern "C" int sa_rope_kv_write(void* qkv, int act_dtype, const int* positions, 
     return SA_ERR_ARG;
   const long long total = (long long)(Hq + Hk) * (rot_dim / 2) + (long long)(parts > 1 ? Hq + Hk : Hk) * (D - rot_dim) + (long long)Hk * D;
   const long long groups = (total + 255) / 256;
-  dim3 grid(T, (unsigned)(groups < 1 ? 1 : (groups > 65535 ? 65535 : groups))), block(256);
+  const long long most = T <= 128 ? 65535 : 4;
+  dim3 grid(T, (unsigned)(groups < 1 ? 1 : (groups > most ? most : groups))), block(256);
   int tpb = T >= 1024 ? 8 : (T >= 512 ? 4 : (T >= 256 ? 2 : 1));
   while (tpb > 1 && (size_t)tpb * ((size_t)Hk * D + 8) * 2 > 65536) tpb >>= 1;   // the values' tile has to fit LDS
   const size_t tile_bytes = (size_t)tpb * ((size_t)Hk * D + 8) * 2;
