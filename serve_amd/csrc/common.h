@@ -157,6 +157,11 @@ __device__ __forceinline__ float short_gate(float g, float u, float limit) {
   }
   return g * __builtin_amdgcn_rcpf(1.f + any_exp(-z)) * u;
 }
+__device__ __forceinline__ float short_gate(float g, float u, int kind, float limit) {
+  if (kind == SA_GATE_SILU) return short_gate<SA_GATE_SILU>(g, u, limit);
+  if (kind == SA_GATE_GELU_TANH) return short_gate<SA_GATE_GELU_TANH>(g, u, limit);
+  return short_gate<SA_GATE_CLAMPED_SWISH>(g, u, limit);
+}
 
 // the first key that a query at position p sees: of its own run of `chunk` positions (counted from position 0) where
 // chunk > 0, of the last `window` keys where window > 0, else the first of all

@@ -185,8 +185,7 @@ __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, i
       for (int i = 0; i < 4; ++i) {
         if constexpr (FIRST) {
           const float gt = acc[mt][nt][i] * in_w, up = acc[mt][nt + CT / 2][i] * in_w;
-          // (the plain gate with the fast exponential, as in the dense feed-forward's products)
-          o[i] = p.gate_kind == SA_GATE_SILU ? (gt / (1.f + __expf(-gt))) * up : gate_mul(gt, up, p.gate_kind, p.gate_limit);
+          o[i] = short_gate(gt, up, p.gate_kind, p.gate_limit);
         } else {
           o[i] = acc[mt][nt][i];
         }
