@@ -352,7 +352,9 @@ class Scheduler:
         reqs = plan.requests
         tokens = [r.tokens_between(r.fed, r.fed + n) for r, n in zip(reqs, plan.counts)]
         samplers = [r for r, s in zip(reqs, plan.samples) if s]
-        keys = row_keys(self.sampler.seed, [r.req_id for r in samplers], [len(r.generated) for r in samplers])
+        keys = [0] * len(samplers)               # (greedy rows draw nothing)
+        if any(r.temperature > 0 for r in samplers):
+            keys = row_keys(self.sampler.seed, [r.req_id for r in samplers], [len(r.generated) for r in samplers])
         launch = self.runner.step_launch_logits if with_logits else self.runner.step_launch
         handle = launch([r.req_id for r in reqs], tokens, plan.samples, [r.temperature for r in samplers], keys)
         handle, logits = handle if with_logits else (handle, None)
