@@ -136,31 +136,15 @@ __device__ __forceinline__ float short_sigmoid(float z) {
 }
 __device__ __forceinline__ float short_silu(float z) { return z * short_sigmoid(z); }
 
-// The same for any x, infinities and overflow among them (the correction is kept within -1 .. 1, which it exceeds nowhere
-// else), and with it gate_mul for results that are rounded to bf16: 10 instructions a silu and two at a quarter of the rate,
-// where expf and a division are 28 and two.  Within a few units in the last place of float32.
-__device__ __forceinline__ float any_exp(float x) {
-  const float L2E = 1.44269502162933349609375f, L2E_LO = 1.925963033500011e-8f;
-  const float t = x * L2E;
-  float r = fmaf(x, L2E, -t);
-  r = __builtin_amdgcn_fmed3f(fmaf(x, L2E_LO, r), -1.f, 1.f);
-  return __builtin_amdgcn_exp2f(t) * fmaf(r, 0.693147182464599609375f, 1.f);
-}
+// gate_mul for results that are rounded to bf16: the same, but for gelu_tanh, where (1 + tanh(s)) / 2 is written as
+// sigmoid(2 s): 1 + tanh(s) cancels, and beyond five below zero it holds fewer bits than bf16 does.
 template <int KIND>
-__device__ __forceinline__ float short_gate(float g, float u, float limit) {
-  float z = g;
-  if (KIND == SA_GATE_GELU_TANH) z = 1.5957691216057308f * (g + 0.044715f * g * g * g);   // (1 + tanh(s)) / 2 = sigmoid(2 s)
-  if (KIND == SA_GATE_CLAMPED_SWISH) {
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit) + 1.f;
-    z = 1.702f * g;
-  }
-  return g * __builtin_amdgcn_rcpf(1.f + any_exp(-z)) * u;
+__device__ __forceinline__ float gate_mul_for_bf16(float g, float u, float limit) {
+  if (KIND != SA_GATE_GELU_TANH) return gate_mul(g, u, KIND, limit);
+  return (g / (1.f + expf(-1.5957691216057308f * (g + 0.044715f * g * g * g)))) * u;
 }
-__device__ __forceinline__ float short_gate(float g, float u, int kind, float limit) {
-  if (kind == SA_GATE_SILU) return short_gate<SA_GATE_SILU>(g, u, limit);
-  if (kind == SA_GATE_GELU_TANH) return short_gate<SA_GATE_GELU_TANH>(g, u, limit);
-  return short_gate<SA_GATE_CLAMPED_SWISH>(g, u, limit);
+__device__ __forceinline__ float gate_mul_for_bf16(float g, float u, int kind, float limit) {
+  return kind == SA_GATE_GELU_TANH ? gate_mul_for_bf16<SA_GATE_GELU_TANH>(g, u, limit) : gate_mul(g, u, kind, limit);
 }
 
 // the first key that a query at position p sees: of its own run of `chunk` positions (counted from position 0) where

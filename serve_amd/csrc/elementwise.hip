@@ -485,9 +485,10 @@ __global__ void silu_mul_kernel(const TA* __restrict__ gu, TA* __restrict__ a, i
   }
 }
 
-// The same, eight bf16 values per thread in 16-byte vectors (I % 8 == 0).  With gate_mul and conversions written out on the bits
-// the vector units were what it waited for; with short gates and the conversion instruction it is memory: 2,000 rows of
-// 2 x 14,336, clamped, 36 -> 28 us, 2,048 of 2 x 8,192 20.9 -> 18.2 (5.5 TB/s).
+// The same, eight bf16 values per thread in 16-byte vectors (I % 8 == 0).  With conversions written out on the bits the vector
+// units were what it waited for; with the conversion instruction, and the kind of gate known when it is compiled, it is memory:
+// 2,000 rows of 2 x 14,336, clamped, 36 -> 31 us, 2,048 of 2 x 8,192, silu, 20.2 -> 17.7 (5.7 TB/s).  The hardware's reciprocal in
+// place of the division would be 28 and 17.2, and twice as far from 64 bits before the rounding: not taken.
 template <int KIND>
 __global__ __launch_bounds__(256) void silu_mul_bf16x8_kernel(const bf16_t* __restrict__ gu, bf16_t* __restrict__ a,
                                                                int T, int I, float limit) {
@@ -503,8 +504,8 @@ __global__ __launch_bounds__(256) void silu_mul_bf16x8_kernel(const bf16_t* __re
     for (int k = 0; k < 4; ++k) {
       const float g0 = bf16_bits_to_float(gw[k] & 0xffffu), g1 = bf16_bits_to_float(gw[k] >> 16);
       const float u0 = bf16_bits_to_float(uw[k] & 0xffffu), u1 = bf16_bits_to_float(uw[k] >> 16);
-      const float o0 = short_gate<KIND>(g0, u0, limit);
-      const float o1 = short_gate<KIND>(g1, u1, limit);
+      const float o0 = gate_mul_for_bf16<KIND>(g0, u0, limit);
+      const float o1 = gate_mul_for_bf16<KIND>(g1, u1, limit);
       ow[k] = floats_to_bf16_bits(o0, o1);
     }
     *reinterpret_cast<uint4*>(a + (size_t)t * I + i) = make_uint4(ow[0], ow[1], ow[2], ow[3]);

@@ -185,7 +185,7 @@ __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, i
       for (int i = 0; i < 4; ++i) {
         if constexpr (FIRST) {
           const float gt = acc[mt][nt][i] * in_w, up = acc[mt][nt + CT / 2][i] * in_w;
-          o[i] = short_gate(gt, up, p.gate_kind, p.gate_limit);
+          o[i] = gate_mul_for_bf16(gt, up, p.gate_kind, p.gate_limit);
         } else {
           o[i] = acc[mt][nt][i];
         }

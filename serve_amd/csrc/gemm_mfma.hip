@@ -56,6 +56,13 @@ struct QkvRopeArgs {
   float magnitude;
 };
 
+// silu(g) u with the fast exponential, as the plain SwiGLU feed-forward has always been computed (its error grows with -g, to
+// nine units in the last place of float32 over normal inputs); any other gate through gate_mul_for_bf16
+__device__ __forceinline__ float gated(float gt, float up, const QkvRopeArgs& qa) {
+  if (qa.gate_kind == SA_GATE_SILU) return (gt / (1.f + __expf(-gt))) * up;
+  return gate_mul_for_bf16(gt, up, qa.gate_kind, qa.gate_limit);
+}
+
 // What the rotating epilogue needs besides the sums: read when a kernel starts, so that the trip to
 // memory for them runs beside the product and not after it.
 template <int MT>
@@ -130,7 +137,7 @@ __device__ __forceinline__ void store_tiles(floatx4_t (&acc)[RT][MT], TC* __rest
       for (int r = 0; r < 4; ++r) {
         const float gt = acc[0][mt][r];
         const float up = acc[1][mt][r];
-        o[r] = short_gate(gt, up, qa.gate_kind, qa.gate_limit);
+        o[r] = gated(gt, up, qa);
       }
       if (n + 3 < N) {
         store4(C + (size_t)m * ldc + n, o, (N & 3) == 0);
@@ -748,7 +755,7 @@ __global__ __launch_bounds__(512) void gemm_wide_kernel(const bf16_t* __restrict
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         if (SWIGLU) {
-          o[r] = short_gate(acc[mt][nt][r], acc[mt][SWIGLU ? nt + NT / 2 : nt][r], qa.gate_kind, qa.gate_limit);
+          o[r] = gated(acc[mt][nt][r], acc[mt][SWIGLU ? nt + NT / 2 : nt][r], qa);
         } else {
           o[r] = acc[mt][nt][r];
         }

@@ -500,7 +500,7 @@ __global__ __launch_bounds__(256) void moe_mfma_kernel(const bf16_t* __restrict_
 #pragma unroll
         for (int r = 0; r < 4; ++r)
           if (n + r < N)
-            dst[r] = from_float<bf16_t>(short_gate(acc[wr][mt][r] * w, acc[RT - WR + wr][mt][r] * w, gate_kind, gate_limit));
+            dst[r] = from_float<bf16_t>(gate_mul_for_bf16(acc[wr][mt][r] * w, acc[RT - WR + wr][mt][r] * w, gate_kind, gate_limit));
       } else {
         float* dst = yk + (size_t)perm[row0 + m] * N + n;
 #pragma unroll

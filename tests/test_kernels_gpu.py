@@ -759,6 +759,50 @@ def test_gates_of_every_bf16_number(kind, limit):
     assert (err <= (2.0 ** -8 * (1 + 2.0 ** -10)) * want.abs() + tiny)[ok].all()
 
 
+@pytest.mark.parametrize("entry", ["rows", "few", "wide", "experts few", "experts"])
+@pytest.mark.parametrize("kind,limit", [("silu", 0.0), ("gelu_tanh", 0.0), ("clamped_swish", 7.0)])
+def test_gates_keep_what_float32_holds(kind, limit, entry):
+    """Sigmoids from 2^-126 down to where e^-z overflows in float32 (z = -88.72) are no zeros: their gates are normal bf16 numbers
+    (of gelu no argument in bf16 falls there: those down from -9, where 1 + tanh(s) has no bits left).  In the pass over rows and in the epilogues of every product that gates, from operands whose sums are exact."""
+    from serve_amd import ops
+    g = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).double()
+    z = {"silu": g, "gelu_tanh": 2 * math.sqrt(2 / math.pi) * (g + 0.044715 * g ** 3), "clamped_swish": 1.702 * g}[kind]
+    g = g[(z < (-60 if kind == "gelu_tanh" else -87.35)) & (z > -88.7)]
+    assert 0 < g.numel() <= 32
+    g = torch.cat([g, torch.tensor([-20.0, -3.0, 5.0], dtype=torch.float64)]).repeat(64)[:64]
+    u = torch.where(torch.arange(64) % 2 == 0, 1.5, -3.0).double()
+    if kind == "gelu_tanh":
+        want = g * torch.sigmoid(2 * math.sqrt(2 / math.pi) * (g + 0.044715 * g ** 3)) * u
+    elif kind == "clamped_swish":
+        want = g * torch.sigmoid(1.702 * g) * (u + 1)
+    else:
+        want = g * torch.sigmoid(g) * u
+    wgu = torch.zeros((2, 64, 64))
+    wgu[0, :, 0], wgu[1, :, 0] = g.float(), u.float()
+    wgu = wgu.bfloat16().to(DEV)
+    if entry == "rows":
+        out = torch.empty((1, 64), dtype=torch.bfloat16, device=DEV)
+        ops.gate_mul(wgu[:, :, 0].reshape(1, 128).contiguous(), out, kind, limit)
+    elif entry in ("few", "wide"):
+        a = torch.zeros((3 if entry == "few" else 64, 64), device=DEV).bfloat16()
+        a[:, 0] = 1
+        out = torch.empty((a.shape[0], 64), dtype=torch.bfloat16, device=DEV)
+        ops.swiglu_bf16(a, wgu.reshape(128, 64), out, kind, limit)
+    else:
+        T, E = (40, 4) if entry == "experts few" else (160, 64)
+        assert ops.moe_wide_pays(T, E, 64) == (entry == "experts")
+        h = torch.zeros((T, 64), device=DEV).bfloat16()
+        h[:, 0] = 1
+        w = wgu[:, None].expand(2, E, 64, 64).contiguous()
+        down = torch.eye(64, device=DEV).bfloat16().expand(E, 64, 64).contiguous()
+        out = torch.empty((T, 64), dtype=torch.float32, device=DEV)
+        ops.moe_experts(h, (torch.arange(T, dtype=torch.int32, device=DEV) % E)[:, None].contiguous(), w[0], w[1], down, out,
+                        gate=kind, limit=limit)
+    # half a unit of bf16's eight bits; e^-z is off by the roundings of z, 88 times 2^-24 each, far below (and a gate below the
+    # range of float32 is nothing: 1e-40)
+    assert ((out.cpu().double() - want).abs() <= 2.0 ** -8 * (1 + 2.0 ** -7) * want.abs() + 1e-40).all()
+
+
 def test_rounding_to_bf16_is_to_the_nearest_even():
     """Products of two bf16 numbers have up to 16 bits: gates of 64 and more are their own silu, so the kernel's results are those
     products rounded, for all numbers of one operand and every mantissa of the other."""
