@@ -127,10 +127,17 @@ class Engine:
             raise ValueError("one temperature per request is needed")
         gen = []
         for i, (r, t) in enumerate(zip(requests, temps)):
-            ids = r.input_ids.tolist() if isinstance(r.input_ids, torch.Tensor) else list(r.input_ids)
-            array = None                          # (portions of long prompts: slices of an array, not lists made into one)
-            if len(ids) >= 256 and isinstance(r.input_ids, torch.Tensor) and r.input_ids.dtype == torch.int64 and r.input_ids.dim() == 1:
-                array = r.input_ids.cpu().numpy()
+            array = None
+            if not isinstance(r.input_ids, torch.Tensor):
+                ids = list(r.input_ids)
+            elif r.input_ids.dtype == torch.int64 and r.input_ids.dim() == 1:
+                # A copy of the caller's ids, which may change during the call.  Kept as an array beside the list made from it:
+                # portions are slices of it, which the planner takes as they are (from the caller's ids to the planner's, us, as
+                # a list only / so: 8 ids 1.1 / 2.3, 17 ids 2.8 / 2.4, 256 ids 13 / 8, 2,048 ids 101 / 24)
+                array = r.input_ids.numpy().copy() if r.input_ids.device.type == "cpu" else r.input_ids.cpu().numpy()
+                ids = array.tolist()
+            else:
+                ids = r.input_ids.tolist()
             if r.input_length != len(ids):
                 raise ValueError(f"request {i}: input_length {r.input_length} != len(input_ids) {len(ids)}")
             gen.append(GenerationRequest(req_id=i, prompt=ids, max_new_tokens=int(r.max_new_tokens), prompt_array=array,

@@ -8,6 +8,7 @@ import random
 
 import numpy as np
 import pytest
+import torch
 
 from serve_amd.cache.manager import FREED, CacheError, CacheManager, PagePool
 from serve_amd.config.engine import EngineConfig
@@ -513,3 +514,30 @@ def test_plan_of_portions_given_as_lists_and_as_arrays():
                 wrong[place][1] = bad
                 with pytest.raises(ValueError, match="outside the vocabulary"):
                     plan_step([Segment(i, make(x), []) for i, x in enumerate(wrong[:3])], fresh(), 100)
+
+
+@pytest.mark.parametrize("length", [3, 300])
+def test_prompts_are_what_they_were_when_generate_was_called(length):
+    """A caller that refills its ids while `generate` runs changes nothing: all portions of a prompt are the ids it was given."""
+    from types import SimpleNamespace
+    from serve_amd.engine.engine import Engine, Request
+    ids = torch.tensor([(7 * i + 3) % VOCAB for i in range(length)])
+    given = ids.tolist()
+
+    class Refilled(FakeRunner):
+        rt = SimpleNamespace(device=torch.device("cpu"))
+
+        def step(self, segments, borrow=False):
+            logits = super().step(segments)
+            ids.fill_(1)
+            return logits
+
+    runner = Refilled(num_pages=128, page_size=4, max_context=512)
+    cfg = EngineConfig(max_tokens_per_step=64, prefill_chunk=64, max_context=512, page_size=4, num_pages=128)
+    engine = Engine(None, runner, cfg)
+    engine.sampler = FakeSampler()
+    fed = []
+    runner.release = lambda rid: (fed.append(list(runner.history[rid])), FakeRunner.release(runner, rid))
+    out = engine.generate([Request(ids, length, 2)])
+    assert ids.tolist() == [1] * length
+    assert fed[0][:length] == given and out[0].generated_tokens.tolist() == alone(given, 2)
