@@ -665,9 +665,14 @@ __global__ __launch_bounds__(512) void moe_router_kernel(const bf16_t* __restric
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) wf[u][nt].r = *reinterpret_cast<const moe_u32x4_t*>(wrow[nt] + k);
     }
-    if (s + KU > end || (s + KU) * 32 > K) {                // beyond the columns the operand of h is zero
+    if (s + KU > end || (s + KU) * 32 > K) {                // beyond the columns both operands are zero (what was read there is
+#pragma unroll                                              // another column's, which may be an infinity)
+      for (int u = 0; u < KU; ++u) {
+        const bool in = s + u < end && (s + u) * 32 + g * 8 < K;
+        af[u].r = in ? af[u].r : zero;
 #pragma unroll
-      for (int u = 0; u < KU; ++u) af[u].r = s + u < end && (s + u) * 32 + g * 8 < K ? af[u].r : zero;
+        for (int nt = 0; nt < NT; ++nt) wf[u][nt].r = in ? wf[u][nt].r : zero;
+      }
     }
 #pragma unroll
     for (int u = 0; u < KU; ++u)

@@ -597,6 +597,32 @@ def test_router_product_with_the_routing(T, N, K, E, top, mode):
     assert torch.equal(ids, want_ids) and torch.allclose(weights, want, rtol=1e-6, atol=0)
 
 
+@pytest.mark.parametrize("K", [8, 264, 1000, 2048, 2056, 4104])     # parts of steps, of a wave's share and of what is loaded at once
+def test_router_logits_of_numbers_without_bounds(K):
+    """An infinity in a row of the router's matrix makes that row's logits infinite, and no NaN comes of columns that were read and
+    do not count; infinities and NaN in a token stay with the token."""
+    from serve_amd import ops
+    g = torch.Generator("cuda").manual_seed(K)
+    h = torch.randn((40, K), device="cuda", generator=g).bfloat16()
+    w = (torch.randn((33, K), device="cuda", generator=g) * K ** -0.5).bfloat16()
+    inf = float("inf")
+    h[h == 0] = 1
+    for n, k in ((0, K - 1), (3, K // 2), (5, 0), (9, K - 8), (17, (3 * K) // 4), (32, K - 1)):
+        w[n, k] = inf if n % 2 else -inf
+    h[11, K - 1], h[12, 0], h[30, K // 2] = inf, -inf, float("nan")
+    w[w == 0] = 1e-3
+    logits = torch.zeros((40, 33), dtype=torch.float32, device="cuda")
+    ids, weights = torch.zeros((40, 2), dtype=torch.int32, device="cuda"), torch.zeros((40, 2), device="cuda")
+    ops.moe_router(h, w, 32, logits, ids, weights)
+    want = (h.double().cpu()[:, None] * w.double().cpu()[None]).sum(-1)        # (a product and a sum of its own for each: no library)
+    got = logits.double().cpu()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.isinf(want).sum() > 100
+    assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+    ok = torch.isfinite(want)
+    size = (h.double().cpu()[:, None] * w.double().cpu()[None]).abs().sum(-1)
+    assert torch.isfinite(got[ok]).all() and ((got - want).abs() <= size * (2 * (K / 32 + 1) + 8) * 2.0 ** -24)[ok].all()   # (as above)
+
+
 # (256 compute units)  128 weight rows a workgroup in both products; 256 in the first, in both, and in the second, over one stage and more
 @pytest.mark.parametrize("d,F,E", [(64, 64, 14), (128, 2048, 14), (1152, 3264, 15), (3392, 192, 14)])
 def test_experts_products_at_the_edges_of_tiles(d, F, E):
