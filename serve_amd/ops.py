@@ -1455,6 +1455,24 @@ def moe_router_available(h: torch.Tensor, w: torch.Tensor) -> bool:
             and 0 < w.shape[0] <= int(load_library("moe").sa_moe_router_max_rows()) and _aligned16(h, w))
 
 
+def moe_router_pays(tokens: int, rows: int, size: int, outputs: int) -> bool:
+    """Whether `moe_router` is faster than a product and `moe_route`, for `tokens` of `size` numbers, `rows` rows of the router's
+    matrix and `outputs` of them to choose from.  It is a chain of loads, 2,048 columns at a time with up to 48 rows and 1,024 beyond,
+    which 16 tokens are too few to hide; from 65 outputs on it routes by the general form; and of more tokens than 4,096 each 16 read
+    the matrix again.  Whole feed-forward, this against those, us (rows x size at tokens): 9 x 2048 at 64, 256 and 4,096 -2.5, -3.9,
+    -3.4; 9 x 1024 -0.3, -1.2, -1.4; 9 x 4096 -3.6, -1.6, -5.1; 9 x 2048 at 32 -0.5, 16 x 1024 at 48 +0.7, 8 x 6144 at 256 +2.0; 16 x 3072
+    +0.4; 33 x 2048 at 48, 64, 100, 1,000, 4,096 and 6,144 +0.2, -0.2, -2.8, -0.8, -3.4, +1.4; 33 x 1024 at 64, 100, 256 and 1,000 +1.7,
+    +0.3, -1.4, -1.5; 33 x 4096 at 256 +4.8; 48 x 2048 at 256 +1.0; 65 x 1024 at 64, 256 and 4,096 +0.7, -2.1, -3.6; 65 x 2048 at 256
+    +2.7; 90 x 2048 at 256 +14."""
+    if not 64 <= tokens <= 4096 or outputs > 64:
+        return False
+    if rows <= 16:
+        return size <= 2048 or size == 4096
+    if rows <= 40:
+        return size <= 2048 and (size > 1024 or tokens >= 96)
+    return rows > 48 and size <= 1024 and tokens >= 256
+
+
 def moe_router(h: torch.Tensor, w: torch.Tensor, experts: int, logits: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor,
                over_all=False, scale: float = 1.0, correction: Optional[torch.Tensor] = None) -> None:
     """logits fp32 [T, N] = h @ w^T, and from its first `experts` columns `ids` and `weights` as `moe_route` makes them."""

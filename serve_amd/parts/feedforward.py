@@ -150,7 +150,8 @@ class RoutedExperts(Part):
         dev = h.device
         ids = torch.empty((T, self.top), dtype=torch.int32, device=dev)
         weights = torch.empty((T, self.top), dtype=torch.float32, device=dev)
-        routed = T > ops.MOE_ROUTE_INSIDE and ops.moe_router_available(h, self.w_router)
+        routed = (T > ops.MOE_ROUTE_INSIDE and ops.moe_router_pays(T, self.w_router.shape[0], d, self.outputs)
+                  and ops.moe_router_available(h, self.w_router))
         if routed:
             logits = torch.empty((T, self.w_router.shape[0]), dtype=torch.float32, device=dev)
             ops.moe_router(h, self.w_router, self.outputs, logits, ids, weights, self.over_all, self.router_scale, self.choice)

@@ -597,6 +597,33 @@ def test_router_product_with_the_routing(T, N, K, E, top, mode):
     assert torch.equal(ids, want_ids) and torch.allclose(weights, want, rtol=1e-6, atol=0)
 
 
+@pytest.mark.parametrize("T,d,E,fused", [(63, 2048, 8, False), (64, 2048, 8, True), (64, 4096, 8, True), (64, 3072, 8, False), (95, 1024, 32, False),
+                                         (96, 1024, 32, True), (64, 2048, 32, True), (256, 1024, 63, True), (255, 1024, 64, False),
+                                         (300, 1088, 64, False), (300, 256, 65, False), (4096, 64, 8, True), (4097, 64, 8, False)])
+def test_when_the_router_takes_product_and_routing_together(monkeypatch, T, d, E, fused):
+    """Both ways of the rule, at its edges: the same feed-forward."""
+    from serve_amd import ops
+    from serve_amd.parts.base import Runtime
+    from serve_amd.registry import get_part
+    part = get_part("feed_forward", "routed_experts")(hidden_size=d, experts=E, top=2, expert_size=64, shared_size=64)
+    g = torch.Generator("cuda").manual_seed(T + d)
+    part.load({r.name: (torch.randn(tuple(r.shape), device="cuda", generator=g) * 0.05).bfloat16() for r in part.param_requests()},
+              Runtime(torch.device("cuda:0"), torch.bfloat16, max_context=64))
+    h = torch.randn((T, d), device="cuda", generator=g).bfloat16()
+    calls = []
+    router = ops.moe_router
+    monkeypatch.setattr(ops, "moe_router", lambda *a: (calls.append(1), router(*a)))
+    y = part.forward(h, None)
+    assert bool(calls) == fused
+    monkeypatch.setattr(ops, "moe_router_pays", lambda *a: not fused)
+    want = part.forward(h, None)
+    assert len(calls) == 1
+    # The logits are float32 sums in another order, so the weights of the rows differ by float32 roundings and the bf16 rows not at
+    # all; a token whose second and third logits are as near as that may choose another expert
+    same = ((y - want).norm(dim=1) <= 1e-4 * want.norm(dim=1))
+    assert same.float().mean() > 0.995
+
+
 @pytest.mark.parametrize("K", [8, 264, 1000, 2048, 2056, 4104])     # parts of steps, of a wave's share and of what is loaded at once
 def test_router_logits_of_numbers_without_bounds(K):
     """An infinity in a row of the router's matrix makes that row's logits infinite, and no NaN comes of columns that were read and
