@@ -12,6 +12,8 @@
 // activations).  Of the two, 72 us are the weights' stream (5.6 TB/s; without loads 41 us, without loads and products 23).
 #include "common.h"
 
+#include <type_traits>
+
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4_t __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x4_t __attribute__((ext_vector_type(4)));
@@ -170,38 +172,44 @@ __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, i
   SA_WAIT_VMCNT(0);                                // (loads into LDS beyond the last stage)
 
   // lane l holds C[m = row tile's row l % 16][n = 4 (l / 16) .. + 3] of every tile pair
+  // (the kind of gate is chosen once: a branch at every number is another 4 of 181 us with the whole feed-forward of 1,000 tokens)
+  auto store = [&](auto kind) __attribute__((always_inline)) {
 #pragma unroll
-  for (int mt = 0; mt < RT; ++mt) {
-    const int m = (rg * RT + mt) * 16 + c;
-    if (m >= M) continue;
-    const int r = row0 + m;
-    const int at = FIRST && !p.in_wts ? 0 : p.perm[r];
-    const float in_w = FIRST && p.in_wts ? p.in_wts[at] : 1.f;   // (a weight on the input: gate and up are linear in it)
+    for (int mt = 0; mt < RT; ++mt) {
+      const int m = (rg * RT + mt) * 16 + c;
+      if (m >= M) continue;
+      const int r = row0 + m;
+      const int at = FIRST && !p.in_wts ? 0 : p.perm[r];
+      const float in_w = FIRST && p.in_wts ? p.in_wts[at] : 1.f;   // (a weight on the input: gate and up are linear in it)
 #pragma unroll
-    for (int nt = 0; nt < (FIRST ? CT / 2 : CT); ++nt) {
-      const int n = col0 + cg * (COLS / 4) + nt * 16 + 4 * g;
-      float o[4];
+      for (int nt = 0; nt < (FIRST ? CT / 2 : CT); ++nt) {
+        const int n = col0 + cg * (COLS / 4) + nt * 16 + 4 * g;
+        float o[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if constexpr (FIRST) {
-          const float gt = acc[mt][nt][i] * in_w, up = acc[mt][nt + CT / 2][i] * in_w;
-          o[i] = gate_mul_for_bf16(gt, up, p.gate_kind, p.gate_limit);
-        } else {
-          o[i] = acc[mt][nt][i];
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (FIRST) {
+            const float gt = acc[mt][nt][i] * in_w, up = acc[mt][nt + CT / 2][i] * in_w;
+            o[i] = gate_mul_for_bf16<decltype(kind)::value>(gt, up, p.gate_limit);
+          } else {
+            o[i] = acc[mt][nt][i];
+          }
         }
-      }
-      if (n < N) {                                 // (N is a multiple of 64)
-        if constexpr (FIRST) {
-          union { bf16_t h[4]; uint2 u; } q;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) q.h[i] = from_float<bf16_t>(o[i]);
-          *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.C) + (size_t)r * N + n) = q.u;
-        } else {
-          *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.C) + (size_t)at * N + n) = make_float4(o[0], o[1], o[2], o[3]);
+        if (n < N) {                                 // (N is a multiple of 64)
+          if constexpr (FIRST) {
+            uint2 q;
+            q.x = floats_to_bf16_bits(o[0], o[1]);
+            q.y = floats_to_bf16_bits(o[2], o[3]);
+            *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(p.C) + (size_t)r * N + n) = q;
+          } else {
+            *reinterpret_cast<float4*>(reinterpret_cast<float*>(p.C) + (size_t)at * N + n) = make_float4(o[0], o[1], o[2], o[3]);
+          }
         }
       }
     }
-  }
+  };
+  if (!FIRST || p.gate_kind == SA_GATE_SILU) store(std::integral_constant<int, SA_GATE_SILU>{});
+  else if (p.gate_kind == SA_GATE_GELU_TANH) store(std::integral_constant<int, SA_GATE_GELU_TANH>{});
+  else store(std::integral_constant<int, SA_GATE_CLAMPED_SWISH>{});
 }
 
 template <int CT, bool FIRST>
