@@ -1504,12 +1504,25 @@ def moe_wide_pays(rows: int, experts: int, expert_size: int) -> bool:
     """Whether so many (token, k) rows go to the products with both operands through LDS where those can take them: from two rows an
     expert on, with workgroups for half of the chip.  The kernels for few rows / those, us, experts x model width x expert width:
     32 x 2048 x 1024 at 68, 160, 400 and 1,024 rows 75 / 66, 90 / 76, 115 / 77, 245 / 82; 64 x 4096 x 1024 at 40, 68 and 160 rows
-    158 / 195, 223 / 230, 276 / 269; 128 x 2048 x 512 at 160 and 400 118 / 126, 152 / 148; 8 x 2048 x 1024 at 68 and 160 38 / 32, 55 /
-    32; 8 x 1024 x 512 at 68 and 160 18.0 / 19.9, 23.7 / 20.5; 4 x 512 x 256 at 400 15 / 20."""
+    158 / 195, 223 / 230, 272 / 259; 8 x 2048 x 1024 at 68 and 160 38 / 32, 55 / 32; 8 x 1024 x 512 at 68 and 160 18.0 / 19.9,
+    23.7 / 20.5; 4 x 512 x 256 at 400 15 / 20.
+
+    Where the workgroups of the gate and up product, one a compute unit, are somewhat more than a round of the chip, the second round
+    is for a few of them: more rows an expert then, by how empty it is.  At 2, 4, 6, 8 and 12 rows an expert: 72 x 1024 x 512 (1.12
+    rounds) 48 / 47, 55 / 66, 58 / 66, 61 / 66, 70 / 67; 40 x 2048 x 1024 (1.25) 91 / 110, 106 / 112, 113 / 113, 119 / 113, 135 / 113;
+    90 x 1024 x 512 (1.41) 56 / 67, 66 / 70, 71 / 71, 74 / 71, 104 / 72; 48 x 2048 x 1024 (1.5) 99 / 112, 125 / 119, 135 / 119, 140 /
+    121, 161 / 121; 128 x 2048 x 512 (2) 135 / 136, 161 / 152, 175 / 153, 210 / 155, 285 / 160.  Over 31 shapes of 8 to 256 experts
+    at 1.5 to 12 rows an expert the choice costs 0.7 % on the mean (with two rows an expert for all 3.2 %, and up to 30)."""
     if rows > MOE_WIDE_MIN_ROWS:
         return True
     workgroups = experts * -(-expert_size // 64)
-    return rows > 64 and rows >= 2 * experts and (workgroups >= 128 or (workgroups >= 64 and rows >= 160))
+    if rows <= 64 or not (workgroups >= 128 or (workgroups >= 64 and rows >= 160)):
+        return False
+    units = compute_units()
+    wide = experts * -(-expert_size // 128)                   # (workgroups of 128 gates and their ups where they fill the chip)
+    groups = max(units, wide if 4 * wide >= 3 * units else workgroups)
+    empty = -(-groups // units) * units / groups - 1          # of whole rounds, as a share of what is not
+    return rows >= experts * (2 + 6 * empty)
 
 
 def moe_wide_available(h: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor) -> bool:

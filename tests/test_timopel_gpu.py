@@ -650,6 +650,43 @@ def test_router_logits_of_numbers_without_bounds(K):
     assert torch.isfinite(got[ok]).all() and ((got - want).abs() <= size * (2 * (K / 32 + 1) + 8) * 2.0 ** -24)[ok].all()   # (as above)
 
 
+# (256 compute units)  both sides of each line of the rule: the smallest number of rows, half of the chip, two rows an expert, a
+# second round of workgroups that is nearly empty
+@pytest.mark.parametrize("T,top,E,d,F,tiles", [(16, 4, 32, 128, 256, False), (17, 4, 32, 128, 256, True), (65, 1, 32, 64, 256, True),
+                                               (40, 4, 32, 192, 256, True), (256, 4, 32, 128, 256, True), (159, 1, 8, 64, 512, False),
+                                               (160, 1, 8, 64, 512, True), (127, 1, 64, 64, 128, False), (128, 1, 64, 64, 128, True),
+                                               (119, 2, 36, 64, 512, False), (121, 2, 36, 64, 512, True), (1024, 1, 4, 64, 192, False)])
+@pytest.mark.parametrize("identity", [0, 3])
+def test_experts_of_65_to_1024_rows(T, top, E, d, F, tiles, identity):
+    """Which kernels a step of few rows takes, and what they give: experts with many rows, with one and with none, and identity
+    outputs, whose rows are left alone."""
+    from serve_amd import ops
+    assert ops.moe_wide_pays(T * top, E, F) == tiles
+    gc = torch.Generator("cuda").manual_seed(T + E + identity)
+    # (the last expert without rows, the one before with one, the first with more than its share)
+    order = torch.rand((T, E + identity), device="cuda", generator=gc)
+    order[:, 0] += 0.3
+    order[:, E - 2: E] = -1
+    order[0, E - 2] = 2
+    ids = order.topk(top, -1).indices.int().contiguous()
+    h = torch.randn((T, d), device="cuda", generator=gc).bfloat16()
+    wgu = (torch.randn((2, E, F, d), device="cuda", generator=gc) * d ** -0.5).bfloat16()
+    wd = (torch.randn((E, d, F), device="cuda", generator=gc) * F ** -0.5).bfloat16()
+    assert ops.moe_wide_available(h, wgu[0], wgu[1], wd)
+    yk = torch.full((T * top, d), float("nan"), dtype=torch.float32, device="cuda")
+    ops.moe_experts(h, ids, wgu[0], wgu[1], wd, yk, outputs=E + identity)
+    flat = ids.view(-1)
+    assert torch.isnan(yk[flat >= E]).all() and not (flat == E - 1).any() and (flat == E - 2).sum() == 1
+    for e in range(E):
+        r = (flat == e).nonzero()[:, 0]
+        x = h[r // top].double()
+        z = x @ wgu[0, e].double().T
+        act = z * torch.sigmoid(z) * (x @ wgu[1, e].double().T)
+        # (as below: the gated values are rounded to bf16's eight bits)
+        bound = 1.1 * 2.0 ** -8 * (act.abs() @ wd[e].double().abs().T)
+        assert torch.isfinite(yk[r]).all() and ((yk[r].double() - act @ wd[e].double().T).abs() <= bound).all(), e
+
+
 # (256 compute units)  128 weight rows a workgroup in both products; 256 in the first, in both, and in the second, over one stage and more
 @pytest.mark.parametrize("d,F,E", [(64, 64, 14), (128, 2048, 14), (1152, 3264, 15), (3392, 192, 14)])
 def test_experts_products_at_the_edges_of_tiles(d, F, E):
