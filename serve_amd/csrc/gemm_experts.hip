@@ -261,16 +261,31 @@ static int launch(ExpertArgs p, int max_tiles, hipStream_t stream) {
   return 0;
 }
 
+// 256 weight rows a workgroup where that still gives most compute units one (every expert chosen), else 128: of E experts with
+// `pieces` times 256 weight rows in a product
+static bool wide_columns(int E, int pieces) { return (long long)E * pieces * 4 >= 3ll * compute_units(); }
+
 // The most rows of a tile (a multiple of 16), for `rows` (token, k) rows of E experts of width F: 256, so that an expert's matrices
-// are read once; 192 where the mean is so near 256 that some experts would have one tile and others two; 128 where there would be
-// too few tiles for the chip.  Both products with tiles of 128 / 192 / 256 rows, us: 32 experts of 2,048 x 1,024 at 3,600 rows
-// 171 / 110 / 109, at 6,000 164 / 191 / 138, at 8,000 232 / 170 / 229, at 10,000 233 / 194 / 193; 16 of them at 4,000 rows
-// 124 / 98 / 144; 64 of 4,096 x 1,536 at 8,800 rows 831 / 599 / 599, at 16,000 1,147 / 936 / 887; 8 of 2,048 x 1,024 at 1,400 rows
-// 49 / 69 / 69.
+// are read once; 128 where there would be too few tiles for the chip.  Near 256 rows an expert some have one tile and others two, and
+// with 192 all have two half as long.  That is better where the second tiles would begin another round of workgroups of 256 rows all
+// the same, and worse where the last round has room for them: of the mean 230 about none, of 256 half of the experts have two.  Beyond
+// two rounds it is the better one from about 262 rows on.
+//
+// Both products with tiles of 128 / 192 / 256 rows, us: 32 experts of 2,048 x 1,024 at 3,600 rows 171 / 110 / 109, at 6,000 164 / 191 /
+// 138, at 10,000 233 / 194 / 193; 8 of them at 1,400 rows 49 / 69 / 69.  With 192 / 256 at 235, 250, 275 and 295 rows an expert: 16 of
+// 2,048 x 1,024 (workgroups of the first product: a round) 101 / 147, 102 / 129, 108 / 131, 115 / 118; 32 of them (a round) 175 / 232, 173 /
+// 226, 174 / 210, 187 / 188; 24 (0.75 of a round) 159 / 126, 160 / 187, 162 / 193, 162 / 163; 48 (1.5) 260 / 253, 261 / 310, 267 / 297, 267 /
+// 267; 16 of 3,072 x 1,536 (0.75) 236 / 168, 235 / 173, 229 / 236, 230 / 229; 128 of 2,048 x 768 (3) 545 / 519, 554 / 567, 553 / 578, 573 /
+// 580; 64 of 4,096 x 1,536 (3) at 250 936 / 887.
 extern "C" int sa_expert_tile_rows(int rows, int E, int F) {
   const long long tiles = (rows + 255ll) / 256 > E ? (rows + 255ll) / 256 : E;
-  if (tiles * ((F + 63) / 64) * 4 < 3ll * compute_units()) return 128;
-  return rows > 230ll * E && rows < 300ll * E ? 192 : 256;
+  const int cus = compute_units();
+  if (tiles * ((F + 63) / 64) * 4 < 3ll * cus) return 128;
+  if (rows <= 230ll * E || rows >= 300ll * E) return 256;
+  const long long gx = wide_columns(E, (F + 127) / 128) ? (F + 127) / 128 : (F + 63) / 64;
+  const long long rounds = (E * gx + cus - 1) / cus, room = (rounds * cus - E * gx) / gx;
+  if (rounds > 2) return rows >= 262ll * E ? 192 : 256;
+  return room * 56 < rows - 228ll * E ? 192 : 256;
 }
 
 // Lists from sa_moe_group with tiles of sa_expert_tile_rows(...) rows at most (max_tiles: the grid's worst case, rows /
@@ -286,10 +301,7 @@ extern "C" int sa_expert_products(const void* h, const void* Wgu, const void* Wd
   if (gate_kind < 0 || gate_kind >= SA_GATE_KINDS || (long long)E * F > 0x7fffffffLL) return SA_ERR_ARG;
   ExpertArgs p = {(const bf16_t*)h, (const bf16_t*)Wgu, act, F, d, E * F, 0, E, top, gate_kind, gate_limit,
                   perm, tile_expert, tile_row0, num_tiles, in_wts};
-  // 256 weight rows a workgroup where that still gives most compute units one (every expert chosen), else 128
-  const int cus = compute_units();
-  const int rc = (long long)E * ((F + 127) / 128) * 4 >= 3ll * cus ? launch<4, true>(p, max_tiles, stream)
-                                                                    : launch<2, true>(p, max_tiles, stream);
+  const int rc = wide_columns(E, (F + 127) / 128) ? launch<4, true>(p, max_tiles, stream) : launch<2, true>(p, max_tiles, stream);
   if (rc != 0) return rc;
   p.A = (const bf16_t*)act;
   p.W = (const bf16_t*)Wd;
@@ -297,6 +309,5 @@ extern "C" int sa_expert_products(const void* h, const void* Wgu, const void* Wd
   p.N = d;
   p.K = F;
   p.in_wts = nullptr;
-  return (long long)E * ((d + 255) / 256) * 4 >= 3ll * cus ? launch<4, false>(p, max_tiles, stream)
-                                                              : launch<2, false>(p, max_tiles, stream);
+  return wide_columns(E, (d + 255) / 256) ? launch<4, false>(p, max_tiles, stream) : launch<2, false>(p, max_tiles, stream);
 }

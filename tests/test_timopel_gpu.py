@@ -716,6 +716,45 @@ def test_experts_products_at_the_edges_of_tiles(d, F, E):
             assert torch.isfinite(yk[t]).all() and ((yk[t].double() - act @ wd[e].double().T).abs() <= bound).all(), (e, counts[e])
 
 
+@pytest.mark.parametrize("rows,E,F,tile", [(8000, 32, 1024, 192), (7360, 32, 1024, 256), (7361, 32, 1024, 192), (9600, 32, 1024, 256),
+                                           (5640, 24, 1024, 256), (6600, 24, 1024, 192), (3760, 16, 1536, 256), (4400, 16, 1536, 192),
+                                           (16000, 64, 1536, 256), (17600, 64, 1536, 192), (1400, 8, 1024, 128)])
+def test_the_rows_of_experts_tiles(rows, E, F, tile):
+    """(256 compute units)  192 rows near 256 an expert, where second tiles have no room in the last round of workgroups."""
+    from ctypes import c_int
+
+    from serve_amd.csrc.build import load_library
+    assert load_library("gemm_experts").sa_expert_tile_rows(c_int(rows), c_int(E), c_int(F)) == tile
+
+
+def test_experts_products_with_tiles_of_192_rows():
+    """Experts with as many rows as one, two and three of these tiles take, with one more, with few and with none."""
+    from ctypes import c_int
+
+    from serve_amd import ops
+    from serve_amd.csrc.build import load_library
+    d, F, E = 64, 512, 32
+    counts = [192, 193, 385, 0, 576, 577, 1, 17] * 4
+    T = sum(counts)
+    assert load_library("gemm_experts").sa_expert_tile_rows(c_int(T), c_int(E), c_int(F)) == 192
+    g = torch.Generator().manual_seed(T)
+    ids = torch.repeat_interleave(torch.arange(E), torch.tensor(counts))[torch.randperm(T, generator=g)].int()[:, None].cuda()
+    gc = torch.Generator("cuda").manual_seed(T)
+    h = torch.randn((T, d), device="cuda", generator=gc).bfloat16()
+    wgu = (torch.randn((2, E, F, d), device="cuda", generator=gc) * d ** -0.5).bfloat16()
+    wd = (torch.randn((E, d, F), device="cuda", generator=gc) * F ** -0.5).bfloat16()
+    assert ops.moe_wide_pays(T, E, F) and ops.moe_wide_available(h, wgu[0], wgu[1], wd)
+    yk = torch.full((T, d), float("nan"), dtype=torch.float32, device="cuda")
+    ops.moe_experts(h, ids, wgu[0], wgu[1], wd, yk)
+    for e in range(E):
+        t = (ids[:, 0] == e).nonzero()[:, 0]
+        x = h[t].double()
+        z = x @ wgu[0, e].double().T
+        act = z * torch.sigmoid(z) * (x @ wgu[1, e].double().T)
+        bound = 1.1 * 2.0 ** -8 * (act.abs() @ wd[e].double().abs().T)       # (as above)
+        assert torch.isfinite(yk[t]).all() and ((yk[t].double() - act @ wd[e].double().T).abs() <= bound).all(), (e, counts[e])
+
+
 @pytest.mark.parametrize("gate,limit", [("silu", 0.0), ("clamped_swish", 0.8)])
 @pytest.mark.parametrize("T,d,F,E,top", [(700, 128, 192, 5, 2), (300, 64, 64, 9, 4), (2048, 256, 128, 6, 1)])
 def test_experts_of_many_rows_with_both_operands_through_lds(T, d, F, E, top, gate, limit):
