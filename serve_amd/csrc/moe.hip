@@ -66,13 +66,13 @@ __device__ __forceinline__ void route_token(const float* __restrict__ z, int* __
       mine = expf(own - big) / all;
       v = lane < E ? mine + corr[lane] : -INFINITY;
     }
-    bool left = lane < E;
+    bool left = lane < E && v == v;                          // (logits that are no numbers are not chosen)
     float first = 0.f, sum = 0.f, weight = 0.f;              // (lane k keeps the k-th choice)
     int choice = 0;
     for (int k = 0; k < top; ++k) {
       const float bv = wave_max(left ? v : -INFINITY);
       const unsigned long long at = __ballot(left && v == bv);
-      int bi = at ? (int)__builtin_ctzll(at) : 0x7fffffff;   // (logits that are no numbers are not chosen)
+      int bi = at ? (int)__builtin_ctzll(at) : 0x7fffffff;   // (none left: outside the table, as below)
       if (k == 0) first = bv;
       float p;
       if (corr) {

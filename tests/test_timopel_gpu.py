@@ -597,6 +597,59 @@ def test_router_product_with_the_routing(T, N, K, E, top, mode):
     assert torch.equal(ids, want_ids) and torch.allclose(weights, want, rtol=1e-6, atol=0)
 
 
+@pytest.mark.parametrize("mode", ["chosen", "all", "sigmoid", "corrected"])
+@pytest.mark.parametrize("E,top", [(1, 1), (2, 2), (63, 5), (64, 8), (65, 8), (130, 3)])        # an output a lane, and more than a wave has
+def test_routing_of_ties_and_of_what_is_no_number(E, top, mode):
+    """Of equal logits the first is chosen (zeros of either sign are equal), infinities are logits like others, and what is no number
+    is not chosen: where nothing else is left the place is given to no expert."""
+    from serve_amd import ops
+    inf, nan = float("inf"), float("nan")
+    g = torch.Generator().manual_seed(E)
+    rows = [torch.zeros(E), torch.randint(-2, 3, (E,), generator=g).float(), torch.randint(0, 2, (E,), generator=g).float() * -0.0,
+            torch.full((E,), -inf), torch.where(torch.rand(E, generator=g) < 0.9, -inf, 1.0), torch.full((E,), -1e4)]
+    ends = torch.randn(E, generator=g)
+    ends[0] = ends[-1] = 9.0                                             # first and last equal, above the others
+    rows.append(ends)
+    if mode != "corrected":                                              # (there a share of NaN makes all of them NaN)
+        rows += [torch.full((E,), nan), torch.where(torch.arange(E) % 7 == 3, 2.0, nan), torch.where(torch.arange(E) == E // 2, nan, 1.0)]
+    z = torch.stack(rows).cuda()
+    T = z.shape[0]
+    corr = torch.randint(0, 3, (E,), generator=g).float() / 4 if mode == "corrected" else None
+    over = "all" if mode == "corrected" else mode
+    ids, w = torch.full((T, top), -1, dtype=torch.int32, device="cuda"), torch.zeros((T, top), device="cuda")
+    ops.moe_route(z, E, top, ids, w, over, 1.5, None if corr is None else corr.cuda())
+    ids, w = ids.cpu(), w.cpu().double()
+    for t, row in enumerate(z.double().cpu()):
+        numbers = [e for e in range(E) if row[e] == row[e]]
+        if corr is not None:
+            shares = torch.softmax(row, 0)
+            if not torch.isfinite(shares).all():
+                assert ((ids[t] >= 0) & (ids[t] < E)).all()             # stays within the table
+                continue
+            score = (torch.softmax(row.float(), 0) + corr).tolist()
+            chosen = ids[t].tolist()
+            assert len(set(chosen)) == top
+            # (shares are rounded: scores as near as that are in either order, equal logits with equal corrections in theirs)
+            left = min((score[e] for e in chosen))
+            assert all(score[e] <= left + 1e-6 for e in range(E) if e not in chosen)
+            for a, b in zip(chosen, chosen[1:]):
+                assert score[a] >= score[b] - 1e-6 and (row[a] != row[b] or corr[a] != corr[b] or a < b)
+            want = shares[ids[t].long()]
+            assert torch.allclose(w[t], 1.5 * want / (want.sum() + 1e-20), rtol=1e-5, atol=1e-7)
+            continue
+        order = sorted(numbers, key=lambda e: (-row[e].item(), e))[:top]
+        assert ids[t, : len(order)].tolist() == order
+        assert ((ids[t, len(order):] < 0) | (ids[t, len(order):] >= E)).all()
+        value = torch.cat([row[order], torch.full((top - len(order),), -inf, dtype=torch.float64)])
+        if mode == "sigmoid":
+            want = torch.sigmoid(value) * 1.5
+        else:
+            want = torch.softmax(value, 0) * 1.5                         # (of the chosen: the sum over all cancels)
+            if mode == "all" and not torch.isfinite(row).all() and torch.isnan(row).any():
+                want = torch.full_like(want, nan)                        # (the sum over all is none)
+        assert torch.allclose(w[t], want, rtol=1e-5, atol=1e-7, equal_nan=True), (t, w[t], want)
+
+
 @pytest.mark.parametrize("T,d,E,fused", [(63, 2048, 8, False), (64, 2048, 8, True), (64, 4096, 8, True), (64, 3072, 8, False), (95, 1024, 32, False),
                                          (96, 1024, 32, True), (64, 2048, 32, True), (256, 1024, 63, True), (255, 1024, 64, False),
                                          (300, 1088, 64, False), (300, 256, 65, False), (4096, 64, 8, True), (4097, 64, 8, False)])
