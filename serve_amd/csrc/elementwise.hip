@@ -271,17 +271,75 @@ extern "C" int sa_add_rmsnorm(float* x, const void* delta, int delta_dtype, int 
 // `parts` > 1 (fp32): the rows are partial sums of a product, `part_stride` elements apart, which are added in order; the
 // finished queries go to the first part's rows.
 //
-// What bounds it: a chain of trips (position, sums, angle, store) and the exact sine and cosine.  In a step of few tokens a
-// thread therefore takes one pair or one value, in gridDim.y workgroups a token, and loads up to eight sums at once: threads that
-// went through a token's pairs and then through its values took, 24 tokens of 40 heads of 64 in four parts, 8.2 us where this
-// takes 5.1.  Many tokens fill the chip by themselves, with up to four workgroups each: 1,164 tokens 16.6 / 16.2 / 15.7 / 17.2 us with
-// one, two, four and seven.
+// What bounds it: a chain of trips (position, sums, angle, store) and the exact sine and cosine, and of many tokens the work an
+// item.  A thread takes one pair or one value, in gridDim.y workgroups a token, and loads up to eight sums at once
+// (rope_kv_write_items_kernel).  Of more than 640 tokens, which fill the chip by themselves, without parts a workgroup goes through
+// one token (rope_kv_write_kernel): less to find out for every item.  A workgroup a token (1,024 threads up to 128 tokens) / an
+// item a thread, us, float32, heads of queries and keys x size: 32 + 8 x 64 at 1, 24, 128, 512, 768, 1,164 and 2,048 tokens 3.8 /
+// 3.2, 4.2 / 3.7, 4.8 / 4.4, 8.4 / 8.0, 9.8 / 10.1, 12.6 / 13.3, 17.1 / 20.1; 64 + 8 x 128 at 160, 512, 768 and 2,048 12.9 / 7.5, 19.5 /
+// 15.9, 23.6 / 21.9, 40.4 / 50.6; bf16, 16 + 16 x 64, adjacent pairs, at 160, 512 and 2,048 6.4 / 4.6, 8.3 / 7.9, 16.0 / 21.0; 32 + 8 x
+// 64 in four parts at 24, 512 and 1,164 5.6 / 3.9, 15.9 / 8.5, 21.2 / 17.3.
 template <typename TA, typename TC>
 __global__ void rope_kv_write_kernel(TA* __restrict__ qkv, const int* __restrict__ positions,
                                      const float* __restrict__ inv_freq, const int* __restrict__ slot,
                                      TC* __restrict__ k_pages, TC* __restrict__ v_pages, int Hq, int Hk,
-                                     int D, int rot_dim, int adjacent, int page_size, int write_kv, int parts,
-                                     size_t part_stride) {
+                                     int D, int rot_dim, int adjacent, int page_size, int write_kv) {
+  const int t = blockIdx.x;
+  TA* row = qkv + (size_t)t * (size_t)(Hq + 2 * Hk) * D;
+  const float pos = (float)positions[t];
+  const int s = write_kv ? slot[t] : -1;
+  const int page = s >= 0 ? s / page_size : 0;
+  const int off = s >= 0 ? s % page_size : 0;
+  const int half = rot_dim / 2;
+
+  // rotated pairs of q heads and k heads
+  const int npairs = (Hq + Hk) * half;
+  for (int idx = threadIdx.x; idx < npairs; idx += blockDim.x) {
+    const int h = idx / half;
+    const int j = idx - h * half;
+    const int i0 = adjacent ? 2 * j : j;
+    const int i1 = adjacent ? 2 * j + 1 : j + half;
+    float sn, cs;
+    if (sizeof(TA) == 2) sincos_reduced(pos * inv_freq[j], &sn, &cs);   // bf16 keeps 8 bits of it
+    else sincosf(pos * inv_freq[j], &sn, &cs);
+    TA* hp = row + (size_t)h * D;
+    const float a = to_float(hp[i0]);
+    const float b = to_float(hp[i1]);
+    const float o0 = a * cs - b * sn;
+    const float o1 = b * cs + a * sn;
+    if (h < Hq) {
+      hp[i0] = from_float<TA>(o0);
+      hp[i1] = from_float<TA>(o1);
+    } else if (s >= 0) {
+      TC* kp = k_pages + (((size_t)page * Hk + (h - Hq)) * page_size + off) * D;
+      kp[i0] = from_float<TC>(o0);
+      kp[i1] = from_float<TC>(o1);
+    }
+  }
+  if (s < 0) return;
+  // k dims that are not rotated
+  const int rest = D - rot_dim;
+  for (int idx = threadIdx.x; idx < Hk * rest; idx += blockDim.x) {
+    const int h = idx / rest;
+    const int i = rot_dim + (idx - h * rest);
+    TC* kp = k_pages + (((size_t)page * Hk + h) * page_size + off) * D;
+    kp[i] = from_float<TC>(to_float(row[(size_t)(Hq + h) * D + i]));
+  }
+  // v, stored transposed inside the page
+  for (int idx = threadIdx.x; idx < Hk * D; idx += blockDim.x) {
+    const int h = idx / D;
+    const int i = idx - h * D;
+    TC* vp = v_pages + (((size_t)page * Hk + h) * D + i) * page_size + off;
+    *vp = from_float<TC>(to_float(row[(size_t)(Hq + Hk + h) * D + i]));
+  }
+}
+
+template <typename TA, typename TC>
+__global__ void rope_kv_write_items_kernel(TA* __restrict__ qkv, const int* __restrict__ positions,
+                                           const float* __restrict__ inv_freq, const int* __restrict__ slot,
+                                           TC* __restrict__ k_pages, TC* __restrict__ v_pages, int Hq, int Hk,
+                                           int D, int rot_dim, int adjacent, int page_size, int write_kv, int parts,
+                                           size_t part_stride, int first) {
   const int t = blockIdx.x;
   TA* row = qkv + (size_t)t * (size_t)(Hq + 2 * Hk) * D;
   const int half = rot_dim / 2, rest = D - rot_dim;
@@ -302,53 +360,50 @@ __global__ void rope_kv_write_kernel(TA* __restrict__ qkv, const int* __restrict
   };
   // the rotated pairs of q heads and k heads, the q dims that are not rotated (sums in parts only), such k dims, the values
   const int pairs = (Hq + Hk) * half, q_rest = parts > 1 ? Hq * rest : 0, k_rest = Hk * rest;
-  const int total = pairs + q_rest + k_rest + Hk * D;
-  for (int item = blockIdx.y * blockDim.x + threadIdx.x; item < total; item += gridDim.y * blockDim.x) {
-    int idx = item;
-    if (idx < pairs) {
-      const int h = idx / half;
-      const int j = idx - h * half;
-      const int i0 = adjacent ? 2 * j : j;
-      const int i1 = adjacent ? 2 * j + 1 : j + half;
-      const float a = at((size_t)h * D + i0);
-      const float b = at((size_t)h * D + i1);
-      const float pos = (float)positions[t];
-      const int s = write_kv && h >= Hq ? slot[t] : -1;
-      float sn, cs;
-      if (sizeof(TA) == 2) sincos_reduced(pos * inv_freq[j], &sn, &cs);   // bf16 keeps 8 bits of it
-      else sincosf(pos * inv_freq[j], &sn, &cs);
-      const float o0 = a * cs - b * sn;
-      const float o1 = b * cs + a * sn;
-      if (h < Hq) {
-        TA* hp = row + (size_t)h * D;
-        hp[i0] = from_float<TA>(o0);
-        hp[i1] = from_float<TA>(o1);
-      } else if (s >= 0) {
-        TC* kp = k_pages + (((size_t)(s / page_size) * Hk + (h - Hq)) * page_size + s % page_size) * D;
-        kp[i0] = from_float<TC>(o0);
-        kp[i1] = from_float<TC>(o1);
-      }
-      continue;
+  int idx = first + blockIdx.y * blockDim.x + threadIdx.x;
+  if (idx < pairs) {
+    const int h = idx / half;
+    const int j = idx - h * half;
+    const int i0 = adjacent ? 2 * j : j;
+    const int i1 = adjacent ? 2 * j + 1 : j + half;
+    const float a = at((size_t)h * D + i0);
+    const float b = at((size_t)h * D + i1);
+    const float pos = (float)positions[t];
+    const int s = write_kv && h >= Hq ? slot[t] : -1;
+    float sn, cs;
+    if (sizeof(TA) == 2) sincos_reduced(pos * inv_freq[j], &sn, &cs);   // bf16 keeps 8 bits of it
+    else sincosf(pos * inv_freq[j], &sn, &cs);
+    const float o0 = a * cs - b * sn;
+    const float o1 = b * cs + a * sn;
+    if (h < Hq) {
+      TA* hp = row + (size_t)h * D;
+      hp[i0] = from_float<TA>(o0);
+      hp[i1] = from_float<TA>(o1);
+    } else if (s >= 0) {
+      TC* kp = k_pages + (((size_t)(s / page_size) * Hk + (h - Hq)) * page_size + s % page_size) * D;
+      kp[i0] = from_float<TC>(o0);
+      kp[i1] = from_float<TC>(o1);
     }
-    idx -= pairs;
-    if (idx < q_rest) {
-      const size_t i = (size_t)(idx / rest) * D + rot_dim + idx % rest;
-      row[i] = from_float<TA>(at(i));
-      continue;
-    }
-    idx -= q_rest;
-    if (!write_kv) return;
-    const bool key = idx < k_rest;
-    if (!key) idx -= k_rest;
-    const int h = idx / (key ? rest : D);
-    const int i = key ? rot_dim + idx % rest : idx - h * D;
-    const float v = at((size_t)(Hq + (key ? 0 : Hk) + h) * D + i);
-    const int s = slot[t];
-    if (s < 0) return;                   // (the same for every thread and item that comes here)
-    const size_t head = (size_t)(s / page_size) * Hk + h;
-    if (key) k_pages[(head * page_size + s % page_size) * D + i] = from_float<TC>(v);
-    else v_pages[(head * D + i) * page_size + s % page_size] = from_float<TC>(v);      // (stored transposed inside the page)
+    return;
   }
+  idx -= pairs;
+  if (idx < q_rest) {
+    const size_t i = (size_t)(idx / rest) * D + rot_dim + idx % rest;
+    row[i] = from_float<TA>(at(i));
+    return;
+  }
+  idx -= q_rest;
+  if (!write_kv || idx >= k_rest + Hk * D) return;
+  const bool key = idx < k_rest;
+  if (!key) idx -= k_rest;
+  const int h = idx / (key ? rest : D);
+  const int i = key ? rot_dim + idx % rest : idx - h * D;
+  const float v = at((size_t)(Hq + (key ? 0 : Hk) + h) * D + i);
+  const int s = slot[t];
+  if (s < 0) return;
+  const size_t head = (size_t)(s / page_size) * Hk + h;
+  if (key) k_pages[(head * page_size + s % page_size) * D + i] = from_float<TC>(v);
+  else v_pages[(head * D + i) * page_size + s % page_size] = from_float<TC>(v);      // (stored transposed inside the page)
 }
 
 // The same for bf16 with (j, j + D/2) pairs over the whole head (rot_dim == D, D % 16 == 0), 16-byte
@@ -443,9 +498,6 @@ extern "C" int sa_rope_kv_write(void* qkv, int act_dtype, const int* positions, 
       (parts > 1 && act_dtype != SA_F32))
     return SA_ERR_ARG;
   const long long total = (long long)(Hq + Hk) * (rot_dim / 2) + (long long)(parts > 1 ? Hq + Hk : Hk) * (D - rot_dim) + (long long)Hk * D;
-  const long long groups = (total + 255) / 256;
-  const long long most = T <= 128 ? 65535 : 4;
-  dim3 grid(T, (unsigned)(groups < 1 ? 1 : (groups > most ? most : groups))), block(256);
   int tpb = T >= 1024 ? 8 : (T >= 512 ? 4 : (T >= 256 ? 2 : 1));
   while (tpb > 1 && (size_t)tpb * ((size_t)Hk * D + 8) * 2 > 65536) tpb >>= 1;   // the values' tile has to fit LDS
   const size_t tile_bytes = (size_t)tpb * ((size_t)Hk * D + 8) * 2;
@@ -459,10 +511,21 @@ extern "C" int sa_rope_kv_write(void* qkv, int act_dtype, const int* positions, 
     SA_LAUNCH_CHECK();
     return 0;
   }
-#define GO(TA, TC)                                                                               \
-  hipLaunchKernelGGL((rope_kv_write_kernel<TA, TC>), grid, block, 0, stream, (TA*)qkv, positions, \
-                     inv_freq, slot, (TC*)k_pages, (TC*)v_pages, Hq, Hk, D, rot_dim, adjacent,   \
-                     page_size, write_kv, parts, (size_t)T * (Hq + 2 * Hk) * D)
+  if (total > 0x7fffffffll) return SA_ERR_ARG;
+#define GO(TA, TC)                                                                                                            \
+  do {                                                                                                                        \
+    if (T > 640 && parts == 1) {                                                                                              \
+      hipLaunchKernelGGL((rope_kv_write_kernel<TA, TC>), dim3(T), dim3(256), 0, stream, (TA*)qkv, positions, inv_freq, slot,   \
+                         (TC*)k_pages, (TC*)v_pages, Hq, Hk, D, rot_dim, adjacent, page_size, write_kv);                       \
+    } else {                                                                                                                  \
+      for (long long first = 0; first < total; first += 65535ll * 256) {       /* (a launch takes 65,535 workgroups a token) */ \
+        const long long groups = (total - first + 255) / 256;                                                                  \
+        hipLaunchKernelGGL((rope_kv_write_items_kernel<TA, TC>), dim3(T, (unsigned)(groups < 65535 ? groups : 65535)),          \
+                           dim3(256), 0, stream, (TA*)qkv, positions, inv_freq, slot, (TC*)k_pages, (TC*)v_pages, Hq, Hk, D,    \
+                           rot_dim, adjacent, page_size, write_kv, parts, (size_t)T * (Hq + 2 * Hk) * D, (int)first);           \
+      }                                                                                                                       \
+    }                                                                                                                         \
+  } while (0)
   if (act_dtype == SA_F32 && cache_dtype == SA_F32) GO(float, float);
   else if (act_dtype == SA_BF16 && cache_dtype == SA_BF16) GO(bf16_t, bf16_t);
   else return SA_ERR_UNSUPPORTED;

@@ -427,6 +427,46 @@ def test_rope_kv_write(dtype, Hq, Hk, D, rot, adjacent, ps):
     assert v_pages.permute(0, 3, 1, 2)[mask].abs().max().item() == 0
 
 
+@pytest.mark.parametrize("T", [1, 129, 640, 641, 900])
+@pytest.mark.parametrize("dtype,Hq,Hk,D,rot,adjacent,parts", [
+    ("float32", 4, 2, 16, 16, False, 1), ("float32", 3, 1, 48, 32, True, 1), ("float32", 5, 0, 24, 24, False, 1),
+    ("float32", 3, 2, 40, 0, False, 1), ("float32", 3, 1, 48, 32, True, 3), ("float32", 7, 2, 20, 12, False, 9),
+    ("bfloat16", 4, 2, 32, 32, True, 1), ("bfloat16", 6, 3, 80, 48, False, 1)])
+def test_rope_kv_write_in_its_general_form(dtype, Hq, Hk, D, rot, adjacent, parts, T):
+    """On both sides of the number of tokens from which a workgroup takes a whole token: heads rotated in part, in adjacent pairs and
+    not at all, queries alone, sums in parts, and tokens without a cache slot."""
+    from serve_amd import ops
+    ps = 8
+    P = T // ps + 2
+    qkv = rnd((parts, T, (Hq + 2 * Hk) * D), DT[dtype], 26)
+    x = qkv.double().sum(0).view(T, Hq + 2 * Hk, D)
+    size = qkv.double().abs().sum(0).view(T, Hq + 2 * Hk, D)
+    if parts == 1:
+        qkv = qkv[0].contiguous()
+    pos = (torch.arange(T, device=DEV) * 3 + 1).to(torch.int32)
+    inv_freq = (1.0 / (10000.0 ** (torch.arange(0, rot, 2).float() / max(rot, 1)))).to(DEV)
+    slots = torch.randperm(P * ps, generator=torch.Generator().manual_seed(T))[:T].to(torch.int32).to(DEV)
+    slots[T // 2] = -1
+    k_pages = torch.zeros((P, Hk, ps, D), dtype=DT[dtype], device=DEV)
+    v_pages = torch.zeros((P, Hk, D, ps), dtype=DT[dtype], device=DEV)
+    cache = (slots, k_pages, v_pages) if Hk else (None, None, None)
+    ops.rope_kv_write(qkv, pos, inv_freq, *cache, Hq, Hk, D, rot, adjacent, ps)
+    q = (qkv[0] if parts > 1 else qkv).double().view(T, -1, D)[:, :Hq]
+    # float32: a rounding for every part, sine, cosine, two products and their sum, of numbers no larger than `size` times sqrt(2)
+    t = dict(atol=(parts + 6) * 2.0 ** -24 * 1.5 * size.max().item(), rtol=0) if dtype == "float32" else tol(dtype)
+    torch.testing.assert_close(q, rope_ref(x[:, :Hq], pos, inv_freq, rot, adjacent), **t)
+    if not Hk:
+        return
+    stored = slots >= 0
+    page, off = (slots // ps).long()[stored], (slots % ps).long()[stored]
+    torch.testing.assert_close(k_pages.double()[page, :, off, :], rope_ref(x[:, Hq: Hq + Hk], pos, inv_freq, rot, adjacent)[stored], **t)
+    torch.testing.assert_close(v_pages.double()[page, :, :, off], x[stored][:, Hq + Hk:], **t)
+    mask = torch.ones((P, ps), dtype=torch.bool, device=DEV)
+    mask[page, off] = False
+    assert k_pages.permute(0, 2, 1, 3)[mask].abs().max().item() == 0
+    assert v_pages.permute(0, 3, 1, 2)[mask].abs().max().item() == 0
+
+
 @pytest.mark.parametrize("T", [300, 600, 1100])
 @pytest.mark.parametrize("Hq,Hk,D,ps", [(32, 8, 64, 16), (6, 2, 128, 16), (5, 5, 48, 12), (36, 36, 128, 16)])
 def test_rope_kv_write_of_many_tokens(T, Hq, Hk, D, ps):
