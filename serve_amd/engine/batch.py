@@ -280,7 +280,12 @@ def upload(host: np.ndarray, device: torch.device) -> torch.Tensor:
     """A step's arrays on the device, by a copy that the host does not wait for: out of pinned memory, which the
     allocator keeps until the copy is done (out of ordinary memory the host would wait for all steps before it)."""
     t = torch.from_numpy(host)
-    return t.pin_memory().to(device, non_blocking=True) if device.type == "cuda" else t.to(device)
+    if device.type != "cuda":
+        return t.to(device)
+    if torch.cuda.is_current_stream_capturing():
+        # (a replay would read the pinned memory again, which is another step's by then)
+        raise RuntimeError("a step's arrays cannot be copied to the device while the stream is captured into a graph")
+    return t.pin_memory().to(device, non_blocking=True)
 
 
 def context_from(lay: StepLayout, dev_buf: torch.Tensor, facts: dict) -> StepContext:

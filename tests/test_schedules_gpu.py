@@ -682,3 +682,24 @@ def test_prompt_steps_that_keep_logits_run_ahead_of_the_host(tmp_path, dtype):
                 assert torch.equal(a.logits, b.logits)
     engine.runner.cache.check_invariants()
     assert not engine.runner.cache.live_requests()
+
+
+@torch.inference_mode()      # (as the engine's own captures: torch's generator keeps tensors of the first)
+def test_steps_arrays_are_not_captured():
+    """A program that captures a step which is run kernel by kernel is told that it cannot: the copy of the step's arrays would be
+    replayed from memory that the step no longer holds."""
+    import numpy as np
+
+    from serve_amd.engine.batch import upload
+    host = np.arange(64, dtype=np.int32)
+    device = torch.device("cuda:0")
+    assert upload(host, device).tolist() == host.tolist()
+    x = torch.zeros(64, device=device)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x += 1
+        with pytest.raises(RuntimeError, match="captured"):
+            upload(host, device)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert x.tolist() == [1.0] * 64 and upload(host, device).tolist() == host.tolist()
