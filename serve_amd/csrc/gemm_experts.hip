@@ -1,5 +1,5 @@
-// The two products of routed experts for prompt portions, bf16 with float32 sums, over tiles of one expert's rows from lists
-// that csrc/moe.hip has built on the device.
+// The two products of routed experts from 65 (token, k) rows on (steps of decoding requests and prompt portions alike), bf16
+// with float32 sums, over tiles of one expert's rows from lists that csrc/moe.hip has built on the device.
 //
 // What bounds them: reading the experts' matrices once (32 experts of 2,048 x 1,024: 403 MB).  So an expert's rows are one
 // tile up to 256 of them (beyond that, tiles of equal size), and a workgroup takes 256 weight rows: with 32 experts that is
@@ -7,7 +7,7 @@
 // takes a run of (tile, weight rows), so the workgroups that read the same activations share an L2, which then holds one
 // expert's at a time.
 //
-// Measured, 1,000 tokens, 4 of 32 experts of 2,048 x 1,024, us: gate/up 88 -> 62 and down 67 -> 43 against tiles of 128 rows
+// Measured, 1,000 tokens, 4 of 32 experts of 2,048 x 1,024, us: gate/up 88 -> 64 and down 67 -> 41 against tiles of 128 rows
 // by 128 weight rows in the order of the grid (an expert with 130 rows read its matrices twice, and every die all of the
 // activations).  Of the two, 72 us are the weights' stream (5.6 TB/s; without loads 41 us, without loads and products 23).
 #include "common.h"
@@ -234,6 +234,9 @@ __global__ __launch_bounds__(512, 2) void expert_product_kernel(ExpertArgs p) {
   // what else is in the step.
   const int u = e * p.gx + t - tile * p.gx, part = max(1, p.E * p.gx >> 3);
   const int first = u % part + (nstages >= 8 ? nstages >> 3 : 1) * (u / part);
+  // The bodies: a tile's products are made for all rows of its body.  32 experts of 2,048 x 1,024 with the same number of rows each,
+  // both products, us: 136 rows 110 with a body for 160 and 121 without, 160 rows 115 and 126.  Bodies for 96 and 224 rows would give
+  // less (72 rows 103 -> 101, 96 rows 108 -> 105, 200 rows 143 -> 136, 224 rows 145 -> 140), a third more code: left out.
   if (M <= 32) expert_tile<CT, 1, FIRST>(p, expert_lds, e, row0, M, col0, first);
   else if (M <= 64) expert_tile<CT, 2, FIRST>(p, expert_lds, e, row0, M, col0, first);
   else if (M <= 128) expert_tile<CT, 4, FIRST>(p, expert_lds, e, row0, M, col0, first);

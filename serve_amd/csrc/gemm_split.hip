@@ -461,10 +461,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
 // and 4-7, 8-11, 16-19, 28-31, and rows of 256 bytes and more then touch every bank once.
 // gridDim.z parts of K, each with sums [M, N] of its own.
 //
-// Measured, the float32 matrix instruction / this kernel in us (weights not in a cache): K 2048, 16,384 rows of W 43 / 30 at
+// Measured, the float32 matrix instruction / this kernel in us (weights not in a cache): K 2048, 16,384 rows of W 43 / 33 at
 // 24 rows of A, 65 / 41 at 64, 121 / 67 at 128; 3,072 rows of W in four parts 20 / 10, 2,048 in eight 8.7 / 8.3; K 8192, 2,048
 // rows in eight parts 24 / 19; 128,256 rows 315 / 219 at 24, 489 / 332 at 64, 965 / 550 at 128.  A step at 24 rows reads
-// its 134 MB at 4.2 TB/s; from 64 rows on the splits of A, which every workgroup makes again, weigh as much.  Distance to
+// its 134 MB at 4.1 TB/s; from 64 rows on the splits of A, which every workgroup makes again, weigh as much.  Distance to
 // 64 bits (rms, of the result's size), normal operands: K 2048 2.9e-7 / 1.1e-7 at 24 rows and 1.35e-7 at 100, K 8192 3.9e-7 /
 // 1.4e-7 at 64 and 100; operands in 1 .. 2: 0.97e-7 / 0.48e-7 and 0.68e-7, 0.88e-7 / 0.56e-7.
 // From five rows, with K in parts: level with the kernel of few rows of csrc/gemm.hip over 3,072 and 2,048 rows of W at K 2048
@@ -535,10 +535,12 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
     src[d] = row < 32 * NT ? W + (size_t)min(n0 + row, N - 1) * K : A + (size_t)min(m0 + row - 32 * NT, M - 1) * K;
     col[d] = seg * 4;
   }
-  // Workgroups begin at different stages, which depend on the rows of W only: neighbours on a die one apart, dies an eighth of
-  // the walk.  Rows lie a power of two apart, so that the same columns of many rows are in one channel of a die's L2 and a few
+  // Workgroups begin at different stages: neighbours on a die one apart, dies an eighth of the walk.  Where depends on a workgroup's
+  // rows of W and on the tiles and parts that the launch has chosen (so on the number of rows of A as far as these do), not on its
+  // rows of A.  Rows lie a power of two apart, so that the same columns of many rows are in one channel of a die's L2 and a few
   // of the memory: 24 rows, four steps of the 1B shape 7.80 ms where all begin at the first column, 7.38 so, and 8.35 where a
-  // die's workgroups begin eight stages apart (as with the number of the workgroup modulo the stages).
+  // die's workgroups begin eight stages apart (as with the number of the workgroup modulo the stages).  One product, 24 rows, us:
+  // 16,384 x 2,048 33.9 -> 32.8, 28,672 x 4,096 107.7 -> 100.1, 128,256 x 2,048 217 -> 201; from 33 rows on within 2 %.
   const int ahead = n > 0 ? (int)(((blockIdx.x >> 3) + (blockIdx.x & 7) * (n >= 8 ? n >> 3 : 1)) % (unsigned)n) : 0;
   auto stage_of = [&](int s) __attribute__((always_inline)) {
     const int t = min(s, n - 1) + ahead;

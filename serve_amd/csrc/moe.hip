@@ -632,8 +632,9 @@ extern "C" int sa_moe_max_tiles(int rows, int E) { return (rows + 15) / 16 + E; 
 // The router's product and the routing in one kernel, bf16: a workgroup takes 16 tokens, its eight waves an eighth of the
 // columns each (tiles as in the products below: 16 of the router's rows by 16 tokens), the sums meet in LDS, go to `logits`
 // [T, N] and are routed from there, a wave a token in turn.  What bounds it is its chain: one trip or two for the operands, the
-// sums, `top` maxima.  1,000 tokens, 33 x 2,048, four of 32: the BLAS library's product 11 us and the routing 7.4 / this 12.
-// Whole feed-forward of 64 tokens, where the product of few rows had two workgroups, 118 / 112.
+// sums, `top` maxima: one after the other where a wave's share of the columns is more than KU steps, so which sizes take it is a
+// rule of its host side.  Feed-forward of 32 experts of 2,048 x 1,024 (33 rows), four chosen, with a product and the routing kernel /
+// with this, us: 64 tokens 113.2 / 111.5, 100 tokens 123.6 / 117.8, 1,000 tokens 182.0 / 178.6 (of which this is 12).
 // ---------------------------------------------------------------------------------------------
 #define MOE_ROUTER_MAX_ROWS 96         // of the router's matrix: what the sums have room for in LDS
 template <int NT>

@@ -556,8 +556,8 @@ def test_differential_heads(dtype, H, Dv, Dp, T):
                                                (700, 8, 4, 2, 64, 64), (16, 3, 0, 3, 96, 24), (300, 70, 20, 4, 32, 16),
                                                (16, 1, 1, 2, 32, 8), (900, 6, 2, 4, 128, 64), (9, 10, 2, 9, 64, 16)])
 def test_experts_with_corrected_choice_and_identity_experts(dtype, T, E, ident, top, d, F):
-    """Every path of the experts' kernels (routing inside the grouping kernel for few tokens, tiles of 16, 64 and 128 rows
-    on the matrix cores, the vector kernels) with choices by corrected shares and outputs that are the token itself."""
+    """Every path of the experts' kernels (routing inside the grouping kernel for few tokens, tiles of 16 to 64 rows and of up
+    to 256 on the matrix cores, the vector kernels) with choices by corrected shares and outputs that are the token itself."""
     from serve_amd import ops
     n = E + ident
     g = torch.Generator().manual_seed(T + E)
