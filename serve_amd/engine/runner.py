@@ -579,6 +579,12 @@ class ModelRunner:
     @torch.inference_mode()
     def step_launch(self, req_ids: Sequence, tokens: Sequence[Sequence[Optional[int]]], samples: Sequence[bool],
                     temperatures: Sequence[float], keys: Sequence[int]) -> DecodeHandle:
+        """Launch any step (prompt portions beside single tokens) with sampling on the device, and
+        return at once: the eager counterpart of `decode_launch`.  tokens[i] are request i's next
+        tokens; a single token may be None for "the token that the previous launch sampled for
+        this request".  samples[i]: whether a token is drawn from the logits at request i's last
+        place; `temperatures` and `keys` belong to those requests, in order, and so do the tokens
+        of the handle."""
         return self._step_launch(req_ids, tokens, samples, temperatures, keys, graphs=True)[0]
 
     def pays_to_launch_with_logits(self, counts: Sequence[int]) -> bool:
@@ -594,12 +600,7 @@ class ModelRunner:
         return self._step_launch(req_ids, tokens, samples, temperatures, keys, graphs=False)
 
     def _step_launch(self, req_ids, tokens, samples, temperatures, keys, graphs: bool):
-        """Launch any step (prompt portions beside single tokens) with sampling on the device, and
-        return at once: the eager counterpart of `decode_launch`.  tokens[i] are request i's next
-        tokens; a single token may be None for "the token that the previous launch sampled for
-        this request".  samples[i]: whether a token is drawn from the logits at request i's last
-        place; `temperatures` and `keys` belong to those requests, in order, and so do the tokens
-        of the handle."""
+        """`step_launch` (through a graph where `graphs` allows it and the shape has one) and the step's logits (of a graph: None)."""
         with torch.cuda.device(self.rt.device):
             if any(toks[0] is None and len(toks) != 1 for toks in tokens):
                 raise ValueError("only a single token can be left to the device")
