@@ -33,6 +33,7 @@ typedef const __attribute__((address_space(1))) void* gptr_t;
 
 // FIRST: act[r] = gate(Wg_e x, Wu_e x) with x = A[perm[r] / top], W [2, E, N, K] (gates, then ups, `up_offset` rows apart).
 // else:  C[perm[r]] = W_e A[r], W [E, N, K].  r: grouped rows of this tile.
+// perm null (the shared expert): every row in its place, and C in bf16 either way.
 struct ExpertArgs {
   const bf16_t* A;
   const bf16_t* W;
@@ -52,7 +53,7 @@ struct ExpertArgs {
 // 16-byte LDS read serves together touch every bank once.  Weights come from memory and activations mostly from the die's L2,
 // which needs fewer stages ahead: two rings, the weights' filled by waves 0 to 3 and the activations' by waves 4 to 7, since a
 // wave's loads land in order and would otherwise wait for each other.
-template <int CT, int RT, bool FIRST>
+template <int CT, int RT, bool FIRST, bool SHARED = false>
 __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, int e, int row0, int M, int col0,
                                             int first) {
   constexpr int BM = 32 * RT, BN = 64 * CT;
@@ -95,7 +96,7 @@ __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, i
       const int row = (lw * RT + d) * 8 + (lane >> 3);
       const int seg = (lane & 7) ^ ((row >> 1) & 7);
       const int r = row0 + min(row, M - 1);
-      src[d] = p.A + (size_t)(FIRST ? p.perm[r] / p.top : r) * K + seg * 8;
+      src[d] = p.A + (size_t)(FIRST && !SHARED ? p.perm[r] / p.top : r) * K + seg * 8;
     }
   }
   const lds_ptr_t as = (lds_ptr_t)lds, ws = as + NA * (A_BYTES / 16);
@@ -179,8 +180,8 @@ __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, i
       const int m = (rg * RT + mt) * 16 + c;
       if (m >= M) continue;
       const int r = row0 + m;
-      const int at = FIRST && !p.in_wts ? 0 : p.perm[r];
-      const float in_w = FIRST && p.in_wts ? p.in_wts[at] : 1.f;   // (a weight on the input: gate and up are linear in it)
+      const int at = SHARED || (FIRST && !p.in_wts) ? 0 : p.perm[r];
+      const float in_w = FIRST && !SHARED && p.in_wts ? p.in_wts[at] : 1.f;   // (a weight on the input: gate and up are linear in it)
 #pragma unroll
       for (int nt = 0; nt < (FIRST ? CT / 2 : CT); ++nt) {
         const int n = col0 + cg * (COLS / 4) + nt * 16 + 4 * g;
@@ -195,7 +196,7 @@ __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, i
           }
         }
         if (n < N) {                                 // (N is a multiple of 64)
-          if constexpr (FIRST) {
+          if constexpr (FIRST || SHARED) {
             uint2 q;
             q.x = floats_to_bf16_bits(o[0], o[1]);
             q.y = floats_to_bf16_bits(o[2], o[3]);
@@ -212,13 +213,55 @@ __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, i
   else store(std::integral_constant<int, SA_GATE_CLAMPED_SWISH>{});
 }
 
+// The shared expert's part of a product, in the same launch: of all M rows, tiles of `rows` by 128 weight rows (SHARED_CT), which
+// fill what the experts leave of the chip.  Up to SHARED_AHEAD rows they stand before the experts' workgroups in the grid, whose
+// stream of weights then begins beside them; of more rows each takes so long that they come behind.  The whole feed-forward, us, the
+// shared expert as two products of its own / ahead / behind: 32 experts of 2,048 x 1,024 and a shared one of 2,048 at 129, 256, 400,
+// 512, 700, 1,000 and 2,048 tokens 127 / 116 / 132, 142 / 125 / 137, 139 / 125 / 140, 156 / 151 / 153, 168 / 159 / 159, 177 / 170 / 166,
+// 259 / 263 / 258; 8 of them and a shared one of 1,024 at 40, 128, 256 and 1,000 53 / 42 / 42, 64 / 52 / 51, 87 / 55 / 54, 122 / 95 / 95.
+// What bounds them is the way into a compute unit (a tile reads 1 MB); tiles of 256 weight rows, or of 256 rows, leave half of the chip
+// idle: 198 and 228 us at 1,000 tokens.
+struct SharedArgs {
+  ExpertArgs p;             // (A null: none)
+  int M, rows, tiles;       // tiles of rows
+  int grid;                 // workgroups (a multiple of 8)
+};
+#define SHARED_CT 2
+#define SHARED_AHEAD 640
+
+template <bool FIRST>
+__device__ __forceinline__ void shared_expert_tile(const SharedArgs& s, u32x4_t* lds, int block) {
+  const int work = s.tiles * s.p.gx;
+  const int die = block & 7, place = block >> 3;           // a die takes a run of weight rows, for all rows each
+  const int share = work >> 3, more = work & 7;
+  if (place >= share + (die < more ? 1 : 0)) return;
+  const int t = die * share + min(die, more) + place;
+  const int col = t / s.tiles, row0 = (t - col * s.tiles) * s.rows;
+  const int M = min(s.rows, s.M - row0);
+  const int eighth = max(1, s.p.K >> 9);
+  const int first = col / 8 + eighth * (col % 8);          // (where to begin depends on the weight rows alone, as below)
+  const int col0 = col * (FIRST ? 32 : 64) * SHARED_CT;
+  if (M <= 32) expert_tile<SHARED_CT, 1, FIRST, true>(s.p, lds, 0, row0, M, col0, first);
+  else if (M <= 64) expert_tile<SHARED_CT, 2, FIRST, true>(s.p, lds, 0, row0, M, col0, first);
+  else expert_tile<SHARED_CT, 4, FIRST, true>(s.p, lds, 0, row0, M, col0, first);
+}
+
 template <int CT, bool FIRST>
-__global__ __launch_bounds__(512, 2) void expert_product_kernel(ExpertArgs p) {
+__global__ __launch_bounds__(512, 2) void expert_product_kernel(ExpertArgs p, SharedArgs s) {
   extern __shared__ __attribute__((aligned(16))) u32x4_t expert_lds[];
+  int block = blockIdx.x;
+  if (s.p.A) {
+    const int begin = s.M <= SHARED_AHEAD ? 0 : (int)gridDim.x - s.grid;
+    if (block >= begin && block < begin + s.grid) {
+      shared_expert_tile<FIRST>(s, expert_lds, block - begin);
+      return;
+    }
+    if (begin == 0) block -= s.grid;
+  }
   // neighbouring workgroups run on different dies: a die takes a run of the work, the weight rows of one tile together
   const int tiles = *p.num_tiles;
   const int work = tiles * p.gx;
-  const int die = blockIdx.x & 7, place = blockIdx.x >> 3;
+  const int die = block & 7, place = block >> 3;
   const int share = work >> 3, more = work & 7;
   if (place >= share + (die < more ? 1 : 0)) return;       // (the grid is the worst case)
   const int t = die * share + min(die, more) + place;
@@ -245,11 +288,26 @@ __global__ __launch_bounds__(512, 2) void expert_product_kernel(ExpertArgs p) {
   else expert_tile<CT, 8, FIRST>(p, expert_lds, e, row0, M, col0, first);
 }
 
+// rows of a tile of the shared expert: equal shares of at most 128, in sixteens
+static int shared_rows(int M) {
+  const int tiles = (M + 127) / 128;
+  return ((M + tiles - 1) / tiles + 15) / 16 * 16;
+}
+
 template <int CT, bool FIRST>
-static int launch(ExpertArgs p, int max_tiles, hipStream_t stream) {
+static int launch(ExpertArgs p, SharedArgs s, int max_tiles, hipStream_t stream) {
   p.gx = (p.N + (FIRST ? 32 : 64) * CT - 1) / ((FIRST ? 32 : 64) * CT);
-  const long long grid = ((long long)p.gx * max_tiles + 7) / 8 * 8;
-  if (max_tiles < 1 || grid > 0x7fffffffLL) return SA_ERR_ARG;
+  long long grid = ((long long)p.gx * max_tiles + 7) / 8 * 8;
+  if (max_tiles < 1 || grid > 0x3fffffffLL) return SA_ERR_ARG;
+  if (s.p.A) {
+    s.p.gx = (s.p.N + (FIRST ? 32 : 64) * SHARED_CT - 1) / ((FIRST ? 32 : 64) * SHARED_CT);
+    s.rows = shared_rows(s.M);
+    s.tiles = (s.M + s.rows - 1) / s.rows;
+    const long long more = ((long long)s.p.gx * s.tiles + 7) / 8 * 8;
+    if (more > 0x3fffffffLL) return SA_ERR_ARG;
+    s.grid = (int)more;
+    grid += more;
+  }
   auto kernel = expert_product_kernel<CT, FIRST>;
   static bool allowed[64] = {};                    // (per device: more than 64 KB of LDS has to be asked for)
   int dev = 0;
@@ -259,7 +317,7 @@ static int launch(ExpertArgs p, int max_tiles, hipStream_t stream) {
     if (e != hipSuccess) return (int)e;
     allowed[dev] = true;
   }
-  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), EX_LDS, stream, p);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(512), EX_LDS, stream, p, s);
   SA_LAUNCH_CHECK();
   return 0;
 }
@@ -296,15 +354,28 @@ extern "C" int sa_expert_tile_rows(int rows, int E, int F) {
 //   gate/up: h [T, d] gathered by perm / top, Wgu [2, E, F, d] -> act [rows, F] = gate(gate, up)
 //            (in_wts, fp32 [T top] or null: both sums times the row's weight first, for weights on the experts' inputs)
 //   down:    act [rows, F], Wd [E, d, F] -> yk [T top, d] fp32 at row perm[r]
+// Sgu not null: in the same two launches a shared expert for all T rows, its gates and ups Sgu [2 S, d], Sd [d, S], the same kind of
+// gate with its own limit: s_act [T, S], s_out [T, d], both bf16 (S a multiple of 64).
 extern "C" int sa_expert_products(const void* h, const void* Wgu, const void* Wd, void* act, float* yk, int E, int d, int F,
                                   int max_tiles, const int* perm, const int* tile_expert, const int* tile_row0,
                                   const int* num_tiles, int top, int gate_kind, float gate_limit, const float* in_wts,
+                                  const void* Sgu, const void* Sd, void* s_act, void* s_out, int T, int S, float s_limit,
                                   hipStream_t stream) {
   if (E <= 0 || d <= 0 || F <= 0 || (d & 63) || (F & 63) || top <= 0) return SA_ERR_ARG;
   if (gate_kind < 0 || gate_kind >= SA_GATE_KINDS || (long long)E * F > 0x7fffffffLL) return SA_ERR_ARG;
   ExpertArgs p = {(const bf16_t*)h, (const bf16_t*)Wgu, act, F, d, E * F, 0, E, top, gate_kind, gate_limit,
                   perm, tile_expert, tile_row0, num_tiles, in_wts};
-  const int rc = wide_columns(E, (F + 127) / 128) ? launch<4, true>(p, max_tiles, stream) : launch<2, true>(p, max_tiles, stream);
+  SharedArgs s = {};
+  if (Sgu) {
+    if (!Sd || !s_act || !s_out || T <= 0 || S <= 0 || (S & 63)) return SA_ERR_ARG;
+    s.p = p;
+    s.p.W = (const bf16_t*)Sgu;
+    s.p.C = s_act;
+    s.p.N = s.p.up_offset = S;
+    s.p.gate_limit = s_limit;
+    s.M = T;
+  }
+  const int rc = wide_columns(E, (F + 127) / 128) ? launch<4, true>(p, s, max_tiles, stream) : launch<2, true>(p, s, max_tiles, stream);
   if (rc != 0) return rc;
   p.A = (const bf16_t*)act;
   p.W = (const bf16_t*)Wd;
@@ -312,5 +383,12 @@ extern "C" int sa_expert_products(const void* h, const void* Wgu, const void* Wd
   p.N = d;
   p.K = F;
   p.in_wts = nullptr;
-  return wide_columns(E, (d + 255) / 256) ? launch<4, false>(p, max_tiles, stream) : launch<2, false>(p, max_tiles, stream);
+  if (Sgu) {
+    s.p.A = (const bf16_t*)s_act;
+    s.p.W = (const bf16_t*)Sd;
+    s.p.C = s_out;
+    s.p.N = d;
+    s.p.K = S;
+  }
+  return wide_columns(E, (d + 255) / 256) ? launch<4, false>(p, s, max_tiles, stream) : launch<2, false>(p, s, max_tiles, stream);
 }

@@ -1533,11 +1533,45 @@ def moe_wide_available(h: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor
             and w_up.data_ptr() == w_gate.data_ptr() + w_gate.numel() * w_gate.element_size())
 
 
+class SharedExpert:
+    """A shared expert's matrices for `moe_experts`, which leaves its rows [T, d] in `out`."""
+
+    def __init__(self, w_gate_up: torch.Tensor, w_down: torch.Tensor, limit: float = 0.0):
+        self.w_gate_up, self.w_down, self.limit = w_gate_up, w_down, float(limit)
+        self.out: Optional[torch.Tensor] = None
+
+
+def moe_shared_available(h: torch.Tensor, w_gate_up: torch.Tensor, w_down: torch.Tensor) -> bool:
+    """bf16 and contiguous, an inner width that is whole stages of 64."""
+    return (h.dtype == w_gate_up.dtype == w_down.dtype == torch.bfloat16 and w_down.dim() == 2 and w_down.shape[1] % 64 == 0
+            and w_down.shape[0] == h.shape[1] and w_gate_up.is_contiguous() and w_down.is_contiguous()
+            and _aligned16(h, w_gate_up, w_down))
+
+
+def moe_shared_inside(h: torch.Tensor, top: int, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
+                      shared_gate_up: torch.Tensor, shared_down: torch.Tensor) -> bool:
+    """Whether `moe_experts` computes the shared expert of these in its own launches, whose tiles of it fill what the experts leave of
+    the chip.  Up to 128 tokens the products of few rows are as fast by themselves where the experts have workgroups for half of the
+    chip (32 x 2048 x 1024 with a shared one of 2,048 at 24, 64 and 128 tokens 104, 114 and 124 us, in the experts' launches 103, 119
+    and 125; 8 of them with one of 1,024 at 64 53 / 41).  Large ones run faster in the library (16 x 4096 x 1024 with a shared one of
+    4,096 at 300, 512, 700 and 1,000 tokens 170 / 155, 193 / 184, 216 / 226, 244 / 252; the first shape at 2,048 and 4,096 259 / 258
+    and 443 / 452)."""
+    E, F, _ = w_gate.shape
+    T, d = h.shape
+    if T <= MOE_ROUTE_INSIDE or T * d * shared_down.shape[-1] > 9e9:
+        return False
+    if T <= SKINNY_MAX_ROWS and 2 * E * -(-F // 128) > compute_units():
+        return False
+    return (moe_wide_pays(T * top, E, F) and moe_wide_available(h, w_gate, w_up, w_down)
+            and moe_shared_available(h, shared_gate_up, shared_down))
+
+
 def moe_experts(h: torch.Tensor, ids: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor,
                 yk: torch.Tensor, logits: Optional[torch.Tensor] = None,
                 weights: Optional[torch.Tensor] = None, over_all=False, scale: float = 1.0,
                 gate: str = "silu", limit: float = 0.0, weight_inputs: bool = False,
-                correction: Optional[torch.Tensor] = None, outputs: Optional[int] = None) -> torch.Tensor:
+                correction: Optional[torch.Tensor] = None, outputs: Optional[int] = None,
+                shared: Optional["SharedExpert"] = None) -> torch.Tensor:
     """yk[t * top + k] = expert ids[t, k] applied to h[t]: down(gate(gate h, up h)), fp32 [T top, d], with
     one of GATES (silu(g) u unless said otherwise).
     w_gate, w_up [E, F, d], w_down [E, d, F] in h's dtype.  With `logits` (fp32 [T, >= E], at most
@@ -1545,7 +1579,8 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, w_gate: torch.Tensor, w_up: 
     `weight_inputs`: expert ids[t, k] is applied to weights[t, k] * h[t] (the weight enters where the gate is applied,
     gate and up being linear), for designs whose weights multiply the experts' inputs and not their outputs.
     `outputs`: how many outputs the router has (None: E); ids of E and above are identity experts, whose rows of yk are
-    left alone (`moe_combine` and `stream_mix` take the token's own row for them).  `correction`: see `moe_route`."""
+    left alone (`moe_combine` and `stream_mix` take the token's own row for them).  `correction`: see `moe_route`.
+    `shared` (where `moe_shared_inside` says so): a shared expert of all tokens, computed in the same launches into `shared.out`."""
     _dev(h, ids, w_gate, w_up, w_down, yk, logits, weights, correction)
     T, d = h.shape
     top = ids.shape[1]
@@ -1577,11 +1612,22 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, w_gate: torch.Tensor, w_up: 
         perm = ints.data_ptr() + o * (2 * E + 1)
         tile_expert = perm + o * n
         tile_row0, num_tiles = tile_expert + o * tiles, tile_expert + o * 2 * tiles
+        sgu = sd = s_act = s_out = None
+        S, s_limit = 0, 0.0
+        if shared is not None:
+            sgu, sd, S, s_limit = shared.w_gate_up, shared.w_down, shared.w_down.shape[1], shared.limit
+            _dev(h, sgu, sd)
+            _check(moe_shared_available(h, sgu, sd) and sgu.shape == (2 * S, d), "the shared expert's matrices must be bf16 [2 S, d], [d, S]")
+            _check(gate != "clamped_swish" or s_limit > 0.0, "the clamped gate needs a positive limit")
+            s_act = torch.empty((T, S), dtype=h.dtype, device=h.device)
+            s_out = shared.out = torch.empty((T, d), dtype=h.dtype, device=h.device)
         _ret(wide.sa_expert_products(_ptr(h), _ptr(w_gate), _ptr(w_down), _ptr(act), _ptr(yk), c_int(E), c_int(d), c_int(F),
                               c_int(-(-n // rows) + E), c_void_p(perm), c_void_p(tile_expert),
                               c_void_p(tile_row0), c_void_p(num_tiles), c_int(top), c_int(GATES[gate]), c_float(limit),
-                              _ptr(weights if weight_inputs else None), _stream()), "expert_products")
+                              _ptr(weights if weight_inputs else None), _ptr(sgu), _ptr(sd), _ptr(s_act), _ptr(s_out),
+                              c_int(T), c_int(S), c_float(s_limit), _stream()), "expert_products")
         return yk
+    _check(shared is None, "these experts' products take no shared expert")
     ldz = 0
     if logits is not None:
         _check(T <= MOE_ROUTE_INSIDE and logits.dtype == torch.float32 and logits.dim() == 2 and logits.shape[0] == T

@@ -158,6 +158,7 @@ class RoutedExperts(Part):
         else:
             logits = linear(h, self.w_router, out_dtype=torch.float32)
         yk = torch.empty((T * self.top, d), dtype=torch.float32, device=dev)
+        shared = None
         if T <= ops.MOE_ROUTE_INSIDE:
             ops.moe_experts(h, ids, self.w_gate, self.w_up, self.w_down, yk, logits, weights, self.over_all,
                             self.router_scale, self.activation, self.limit, self.weight_inputs, self.choice,
@@ -165,11 +166,17 @@ class RoutedExperts(Part):
         else:
             if not routed:
                 ops.moe_route(logits, self.outputs, self.top, ids, weights, self.over_all, self.router_scale, self.choice)
+            inside = None
+            if self.shared is not None and ops.moe_shared_inside(h, self.top, self.w_gate, self.w_up, self.w_down,
+                                                                 self.shared.w_gate_up, self.shared.w_down):
+                inside = ops.SharedExpert(self.shared.w_gate_up, self.shared.w_down, self.shared.limit)
             ops.moe_experts(h, ids, self.w_gate, self.w_up, self.w_down, yk, weights=weights, gate=self.activation,
-                            limit=self.limit, weight_inputs=self.weight_inputs, outputs=self.outputs)
+                            limit=self.limit, weight_inputs=self.weight_inputs, outputs=self.outputs, shared=inside)
+            shared = inside.out if inside is not None else None
         if rows_ok and self.leaves_rows:
             return ops.ExpertRows(yk, weights, ids, self.experts, h)
-        shared = self.shared.forward(h, ctx) if self.shared is not None else None
+        if shared is None and self.shared is not None:
+            shared = self.shared.forward(h, ctx)
         y = torch.empty((T, d), dtype=torch.float32, device=dev)
         return ops.moe_combine(yk, None if self.weight_inputs else weights, shared,
                                logits if self.shared_gate else None, self.outputs, y,

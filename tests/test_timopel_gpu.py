@@ -808,6 +808,37 @@ def test_experts_products_with_tiles_of_192_rows():
         assert torch.isfinite(yk[t]).all() and ((yk[t].double() - act @ wd[e].double().T).abs() <= bound).all(), (e, counts[e])
 
 
+# tiles of 16 rows and more, one and several of them; fewer weight rows than a workgroup takes and no whole share; ahead and behind
+@pytest.mark.parametrize("gate,limit,shared_limit", [("silu", 0.0, 0.0), ("clamped_swish", 0.8, 1.7)])
+@pytest.mark.parametrize("T,d,S", [(65, 64, 64), (96, 192, 320), (129, 128, 192), (257, 64, 2048), (640, 320, 192), (641, 64, 64), (1153, 192, 576)])
+def test_a_shared_expert_in_the_experts_launches(T, d, S, gate, limit, shared_limit):
+    from serve_amd import ops
+    E, F, top = 64, 128, 2
+    g = torch.Generator("cuda").manual_seed(T + d + S)
+    h = torch.randn((T, d), device="cuda", generator=g).bfloat16()
+    wgu = (torch.randn((2, E, F, d), device="cuda", generator=g) * d ** -0.5).bfloat16()
+    wd = (torch.randn((E, d, F), device="cuda", generator=g) * F ** -0.5).bfloat16()
+    sgu = (torch.randn((2 * S, d), device="cuda", generator=g) * d ** -0.5).bfloat16()
+    sd = (torch.randn((d, S), device="cuda", generator=g) * S ** -0.5).bfloat16()
+    ids = torch.stack([torch.randperm(E, device="cuda", generator=g)[:top] for _ in range(T)]).int().contiguous()
+    assert ops.moe_wide_pays(T * top, E, F) and ops.moe_shared_available(h, sgu, sd)
+    alone, both = (torch.full((T * top, d), float("nan"), device="cuda") for _ in range(2))
+    ops.moe_experts(h, ids, wgu[0], wgu[1], wd, alone, gate=gate, limit=limit)
+    shared = ops.SharedExpert(sgu, sd, shared_limit)
+    ops.moe_experts(h, ids, wgu[0], wgu[1], wd, both, gate=gate, limit=limit, shared=shared)
+    assert torch.equal(alone, both), "the experts' own rows have changed"
+    z, u = h.double() @ sgu[:S].double().T, h.double() @ sgu[S:].double().T
+    if gate == "silu":
+        act = z * torch.sigmoid(z) * u
+    else:
+        z, u = z.clamp(max=shared_limit), u.clamp(-shared_limit, shared_limit)
+        act = z * torch.sigmoid(1.702 * z) * (u + 1.0)
+    want = act @ sd.double().T
+    # the gated values and the result are rounded to bf16's eight bits; the rest is float32
+    bound = 1.1 * 2.0 ** -8 * (act.abs() @ sd.double().abs().T + want.abs())
+    assert shared.out.shape == (T, d) and ((shared.out.double() - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("gate,limit", [("silu", 0.0), ("clamped_swish", 0.8)])
 @pytest.mark.parametrize("T,d,F,E,top", [(700, 128, 192, 5, 2), (300, 64, 64, 9, 4), (2048, 256, 128, 6, 1)])
 def test_experts_of_many_rows_with_both_operands_through_lds(T, d, F, E, top, gate, limit):
