@@ -28,6 +28,8 @@
 //                 (two 8-byte loads when the page size is a multiple of 4 only).
 #include "common.h"
 
+#include <type_traits>
+
 #ifndef HEAD_DIM
 #error "compile with -DHEAD_DIM=<head size>"
 #endif
@@ -518,6 +520,13 @@ __global__ __launch_bounds__(64 * WG_SPLITS) void paged_attention_mfma_wg_kernel
 // p = 0.  A branch around the matrix products themselves would make the compiler copy O at every
 // stage.
 //
+// PM 2 (heads of 64, and of 128 with eight waves; pages of 8 keys, a power of two, up to what a round of the workgroup's loads
+// holds): a thread's eight loads of a stage and their lookups were 90 vector instructions of its 460, for addresses of their own;
+// every wave's load lies in one page here, so its address is a scalar and a constant of the lane.  The same bits; 32 heads on 8,
+// us, PM 1 / PM 2: heads of 64, 256 tokens 9.5 / 9.1, 24 ragged prompts up to 256 22.8 / 21.4, 1,000 tokens 19.7 / 18.6, 2,048 36.9 / 35.1,
+// 2,048 over 4,096 keys 78.3 / 74.4, over 12,288 245 / 234 (0.77 -> 0.81 PFLOP/s), 4,096 113 / 108; heads of 128, from 1,000 tokens on:
+// 29.5 / 28.2, 57.0 / 54.7, 129 / 125, 418 / 400, 183 / 176.
+//
 // LDS of a stage: K as [key][16-byte slot] with rows of 128 bytes (256 above head size 64), slot
 // s of key row r stored at s ^ ((r & 3) | ((r >> 1) & 4)): the eight lanes that read together
 // (c = 0..7 -> rows 0..3, 8..11 of a block, one slot) then fall into eight different 16-byte bank
@@ -552,6 +561,9 @@ struct PromptShape {
   static constexpr int MERGE_FLOATS = DT * 8 + 4;          // per lane: O, m and l of two column tiles
   static constexpr int MERGE_BYTES = (KW - 1) * TW * MERGE_FLOATS * 64 * 4;   // the merge reuses the stages' memory
   static constexpr int LDS_BYTES = RING_BYTES > MERGE_BYTES ? RING_BYTES : MERGE_BYTES;
+  static constexpr int LOAD_KEYS = THREADS * 8 / HD;       // keys from one of a thread's loads to its next
+  // whether a thread's places in LDS then differ by a constant (whole groups of four runs of eight keys, whole loads)
+  static constexpr bool PAGE_LOADS = HD % 64 == 0 && LOAD_KEYS % 32 == 0 && CHUNKS % THREADS == 0;
   static_assert(TW * KW == WAVES && (WAVES == 8 || WAVES == 4), "eight waves, or four");
 };
 
@@ -566,6 +578,9 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prompt_attention_kernel(
   using S = PromptShape<KW, WAVES>;
   constexpr int TW = S::TW, KB = S::KB, NT = 2, PT = S::PER_THREAD;
   constexpr int VL = PM == 0 ? 2 : 1;                      // loads per 16 bytes of V^T
+  constexpr bool PAGE_LOADS = PM == 2;                     // each of a wave's loads lies in one page
+  constexpr int LOAD_KEYS = S::LOAD_KEYS;
+  static_assert(!PAGE_LOADS || S::PAGE_LOADS, "see PromptShape");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -590,7 +605,7 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prompt_attention_kernel(
   const int ctx_before = ctx - q_len;
   const int* bt = block_table + (size_t)seg * max_pages;
   const uint32_t page_bytes = (uint32_t)Hk * page_size * HD * 2;   // of a page of K, and of V (checked by the host)
-  const int last_page = PM == 1 ? (ctx - 1) >> page_shift : (ctx - 1) / page_size;
+  const int last_page = PM != 0 ? (ctx - 1) >> page_shift : (ctx - 1) / page_size;
   const char* k_base = reinterpret_cast<const char*>(k_pages);
   const char* v_base = reinterpret_cast<const char*>(v_pages);
 
@@ -601,8 +616,24 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prompt_attention_kernel(
   // read from the last page, at their own place in it, and are never visible.
   int k_key[PT], k_seg[PT], k_off[PT], k_lds[PT], v_run[PT], v_dim[PT], v_off[PT], v_lds[PT];
   bool fetches[PT];
+  // PAGE_LOADS: a thread's loads differ by LOAD_KEYS keys and by nothing else, and load i of a wave, of keys and values alike,
+  // lies in one page, which lane i of the wave looks up: an address is a scalar and a constant of the thread.
+  uint32_t pl_koff = 0, pl_voff = 0;
+  int pl_klds = 0, pl_vlds = 0, pl_run = 0, pl_key = 0;
+  if constexpr (PAGE_LOADS) {
+    const int rs = page_shift - 3;
+    const int key = tid / (HD / 8), slot = tid - key * (HD / 8);
+    const int piece = (tid >> rs) / HD, within = tid - ((piece * HD) << rs);
+    const int dim = within >> rs;
+    pl_run = (piece << rs) + (within & ((1 << rs) - 1));
+    pl_koff = (((hk * page_size + (key & (page_size - 1))) * HD) + slot * 8) * 2;
+    pl_voff = ((hk * HD + dim) * page_size + ((pl_run * 8) & (page_size - 1))) * 2;
+    pl_klds = key * S::K_ROW + ((slot ^ ((key & 3) | ((key >> 1) & 4))) << 4);
+    pl_vlds = (((pl_run >> 2) * HD + dim) * 4 + ((pl_run & 3) ^ ((dim >> 1) & 3))) << 4;
+    pl_key = wave * 512 / HD + min(lane, PT - 1) * LOAD_KEYS;
+  }
 #pragma unroll
-  for (int i = 0; i < PT; ++i) {
+  for (int i = 0; i < (PAGE_LOADS ? 0 : PT); ++i) {
     const int raw = tid + i * S::THREADS;
     fetches[i] = raw < S::CHUNKS;
     const int ch = min(raw, S::CHUNKS - 1);
@@ -629,11 +660,16 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prompt_attention_kernel(
   // page ids of a stage's keys, and of its values, fetched one step before the keys and values are
   auto lookup_k = [&](int sb, int (&pk)[PT]) __attribute__((always_inline)) {
     const int key0 = sb * S::KEYS;
+    if constexpr (PAGE_LOADS) {
+      pk[0] = bt[min((key0 + pl_key) >> page_shift, last_page)];
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < PT; ++i)
       pk[i] = PM == 1 ? bt[min((key0 + k_key[i]) >> page_shift, last_page)] : bt[min((key0 + k_key[i]) / page_size, last_page)];
   };
   auto lookup_v = [&](int sb, int (&pv)[PT * VL]) __attribute__((always_inline)) {
+    if constexpr (PAGE_LOADS) return;
     const int key0 = sb * S::KEYS;
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
@@ -647,8 +683,17 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prompt_attention_kernel(
   };
   // The loads carry no conditions: a stage beyond the last is read from the last page and never used.
   // With a power-of-two page size, (stage begin mod page) is 0 unless a page holds several stages.
+  uint64_t pl_page[PT];                                      // PAGE_LOADS: where the pages of the keys issued last begin
   auto issue_k = [&](int sb, const int (&pk)[PT], u32x4_t (&r)[PT]) __attribute__((always_inline)) {
     const int key0 = sb * S::KEYS;
+    if constexpr (PAGE_LOADS) {
+#pragma unroll
+      for (int i = 0; i < PT; ++i) {
+        pl_page[i] = (uint64_t)(uint32_t)max(__builtin_amdgcn_readlane(pk[0], i), 0) * page_bytes;
+        r[i] = *reinterpret_cast<const u32x4_t*>(k_base + pl_page[i] + pl_koff);
+      }
+      return;
+    }
     if (PM == 1) {
       const char* kb = k_base + (size_t)(key0 & (page_size - 1)) * (HD * 2);
 #pragma unroll
@@ -664,6 +709,11 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prompt_attention_kernel(
     }
   };
   auto issue_v = [&](int sb, const int (&pv)[PT * VL], u32x4_t (&r)[PT]) __attribute__((always_inline)) {
+    if constexpr (PAGE_LOADS) {                              // (of the same stage)
+#pragma unroll
+      for (int i = 0; i < PT; ++i) r[i] = *reinterpret_cast<const u32x4_t*>(v_base + pl_page[i] + pl_voff);
+      return;
+    }
     const int key0 = sb * S::KEYS;
     if (PM == 1) {
       const char* vb = v_base + (size_t)(key0 & (page_size - 1)) * 2;
@@ -694,7 +744,8 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prompt_attention_kernel(
     unsigned char* st = smem + buf * S::K_BYTES;
 #pragma unroll
     for (int i = 0; i < PT; ++i)
-      if (S::CHUNKS % S::THREADS == 0 || fetches[i]) *reinterpret_cast<u32x4_t*>(st + k_lds[i]) = r[i];
+      if (S::CHUNKS % S::THREADS == 0 || fetches[i])
+        *reinterpret_cast<u32x4_t*>(st + (PAGE_LOADS ? pl_klds + i * S::THREADS * 16 : k_lds[i])) = r[i];
   };
   auto stash_v = [&](int sb, int buf, const u32x4_t (&r)[PT]) __attribute__((always_inline)) {
     unsigned char* st = smem + 2 * S::K_BYTES + buf * S::V_BYTES;
@@ -704,14 +755,15 @@ __global__ __launch_bounds__(64 * WAVES, 2) void prompt_attention_kernel(
     for (int i = 0; i < PT; ++i) {
       u32x4_t v = r[i];
       if (at_edge) {
-        const int first = key0 + v_run[i] * 8;
+        const int first = key0 + (PAGE_LOADS ? pl_run * 8 + i * LOAD_KEYS : v_run[i] * 8);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int k0 = first + 2 * e, k1 = k0 + 1;
           v[e] &= (k0 < ctx && k0 >= lo_visible ? 0x0000ffffu : 0u) | (k1 < ctx && k1 >= lo_visible ? 0xffff0000u : 0u);
         }
       }
-      if (S::CHUNKS % S::THREADS == 0 || fetches[i]) *reinterpret_cast<u32x4_t*>(st + v_lds[i]) = v;
+      if (S::CHUNKS % S::THREADS == 0 || fetches[i])
+        *reinterpret_cast<u32x4_t*>(st + (PAGE_LOADS ? pl_vlds + i * S::THREADS * 16 : v_lds[i])) = v;
     }
   };
 
@@ -1197,18 +1249,24 @@ extern "C" int sa_paged_attention_mfma(const void* q, int q_stride, void* out, c
     if (items * Hk > 0x7fffffffLL || (long long)Hk * page_size * HD * 2 > 0x7fffffffLL) return SA_ERR_ARG;
     dim3 grid((unsigned)(items * Hk), B * num_splits);
     const int pm = page_shift >= 3 ? 1 : 0;
-    int rc;
-#define GO(KW, PM, WAVES)                                                                                \
-  rc = launch_prompt<KW, PM, WAVES>(grid, stream, (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_pages, \
+    auto go = [&](auto kw_, auto waves_) {
+      constexpr int KW = decltype(kw_)::value, WAVES = decltype(waves_)::value;
+      using Shape = PromptShape<KW, WAVES>;
+#define GO(PM)                                                                                           \
+  return launch_prompt<KW, PM, WAVES>(grid, stream, (const bf16_t*)q, q_stride, (bf16_t*)out, (const bf16_t*)k_pages, \
                              (const bf16_t*)v_pages, block_table, max_pages, cu_q, ctx_len, Hq, Hk, page_size, \
                              page_shift, scale_log2e, window, chunk, num_splits, pair, part_o, part_ml, sinks)
-    if (light && pm == 1) GO(1, 1, 4);
-    else if (light) GO(1, 0, 4);
-    else if (kw == 2 && pm == 1) GO(2, 1, 8);
-    else if (kw == 2) GO(2, 0, 8);
-    else if (pm == 1) GO(4, 1, 8);
-    else GO(4, 0, 8);
+      if constexpr (Shape::PAGE_LOADS) {
+        if (pm == 1 && page_size <= Shape::LOAD_KEYS) GO(2);
+      }
+      if (pm == 1) GO(1);
+      GO(0);
 #undef GO
+    };
+    using std::integral_constant;
+    const int rc = light ? go(integral_constant<int, 1>{}, integral_constant<int, 4>{})
+                 : kw == 2 ? go(integral_constant<int, 2>{}, integral_constant<int, 8>{})
+                           : go(integral_constant<int, 4>{}, integral_constant<int, 8>{});
     if (rc != 0) return rc;
   }
   SA_LAUNCH_CHECK();

@@ -1009,6 +1009,17 @@ def test_prompt_attention_of_short_contexts_as_the_engine_calls_it(Hq, Hk, D, ps
         attention_case("bfloat16", Hq, Hk, D, ps, segs, seed=531 + D + top, kernel="dispatch", window=50, poison=True)
 
 
+@pytest.mark.parametrize("Hq,Hk,D,ps", [(8, 2, 64, 8), (8, 2, 64, 32), (8, 2, 64, 64), (8, 2, 64, 128), (4, 4, 128, 8), (4, 4, 128, 32),
+                                        (4, 4, 128, 64)])
+def test_prompt_attention_on_both_sides_of_the_largest_page_of_a_load(Hq, Hk, D, ps):
+    """The largest pages for which a wave's loads differ by a constant (heads of 64: 64 keys with eight waves and 32 with four;
+    of 128: 32), the next ones, and the smallest."""
+    attention_case("bfloat16", Hq, Hk, D, ps, [(0, 37), (100, 28), (0, 129), (250, 7), (0, 300)], seed=570 + D, kernel="mfma", poison=True)
+    attention_case("bfloat16", Hq, Hk, D, ps, [(0, 700), (900, 130), (300, 21)], seed=571 + D, kernel="mfma", poison=True)
+    attention_case("bfloat16", Hq, Hk, D, ps, [(700, 20), (300, 90)], seed=572 + D, kernel="mfma", window=290, poison=True)
+    attention_case("bfloat16", Hq, Hk, D, ps, [(0, 200), (33, 65)], seed=573 + D, kernel="dispatch", poison=True)
+
+
 @pytest.mark.parametrize("Hq,Hk,D,ps", [(8, 2, 64, 16), (4, 1, 128, 32), (3, 3, 80, 20)])
 def test_prompt_attention_long_prompts_windows_and_split_keys(Hq, Hk, D, ps):
     """Many row groups per segment (a workgroup takes group w and group last - w; an odd count leaves
