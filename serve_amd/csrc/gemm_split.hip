@@ -170,8 +170,9 @@ __device__ __forceinline__ bool small_operands(uint32_t ka, uint32_t kw) {
   return a < 0x1p-103f || w < 0x1p-103f || a * w < 0x1p-94f;
 }
 
-// C[m, n], just stored by this lane, once more if it is not finite or at most `limit`.
-__device__ __noinline__ void redo(const float* A, const float* W, float* C, int m, int n, int N, int K, int k_begin, int k_end,
+// C[m, n], just stored by this lane, once more if it is not finite or at most `limit`.  (Inlined: a call needs a stack, which
+// every launch then sets up; 24 rows, 2,048 of W at K 8192 in eight parts 18.5 -> 18.3 us.)
+__device__ __forceinline__ void redo(const float* A, const float* W, float* C, int m, int n, int N, int K, int k_begin, int k_end,
                                   float limit) {
   float* cp = C + (size_t)m * N + n;
   const float size = fabsf(*cp);
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
 // rows of W and MT tiles of 32 rows of A (gridDim.y runs of them; which, see few_rows).  A stage is 128 / NT columns of both (a row of it is 512 / NT bytes),
 // loaded straight into LDS, a kilobyte an instruction, in a ring of NB stages: no registers hold what is on its way.
 // Wave = (tile of W wt, run of 16 columns kc): it reads its fragments (lane l: row l % 32, eight columns from 8 (l / 32)),
-// splits them and multiplies; the waves of a tile add their sums through LDS at the end, in order.  Segment s (16 bytes)
+// splits them and multiplies; the sums of a tile's waves are added through LDS at the end, in order.  Segment s (16 bytes)
 // of row r lies at slot s ^ (r & 15): a 16-byte LDS read serves 16 lanes a cycle, in the groups 0-3, 12-15, 20-23, 24-27
 // and 4-7, 8-11, 16-19, 28-31, and rows of 256 bytes and more then touch every bank once.
 // gridDim.z parts of K, each with sums [M, N] of its own.
@@ -513,7 +514,6 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   constexpr int ND = ROWS / RPI / 8;                         // instructions a wave and stage
   static_assert(ROWS % (RPI * 8) == 0, "every wave issues the same number of loads");
   constexpr int KH = 8 / NT;                                 // waves a tile of W
-  static_assert(NB * STAGE >= (KH - 1) * NT * MT * 16 * 64 * 4, "the sums are handed over in the ring's memory");
   extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -636,75 +636,66 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
     sizes[wave] = most_a;
     sizes[8 + wave] = most_w;
   }
-  float* sums = reinterpret_cast<float*>(ring);              // [KH - 1][NT][MT][16][64]
-  if (kc > 0) {
+  // Every wave hands over its sums, and then adds up those of eight rows of W with all of A's, 16 bytes a lane.  (With a tile
+  // of W added and stored by one of its waves, number by number, the others idle, us: 24 rows, K 2048 in four parts,
+  // 3,072 rows of W 11.7 / 11.1 so; 100 rows, 16,384 of W 75.5 / 70.6; 128 rows, 128,256 of W 575 / 544.)
+  f32x4_t* sums = reinterpret_cast<f32x4_t*>(ring);          // [KH][NT][MT][4][64]
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) sums[((((kc - 1) * NT + wt) * MT + mt) * 16 + e) * 64 + lane] = acc[mt][e];
-  }
+    for (int q = 0; q < 4; ++q)
+      sums[((wave * MT + mt) * 4 + q) * 64 + lane] =
+          (f32x4_t){acc[mt][4 * q], acc[mt][4 * q + 1], acc[mt][4 * q + 2], acc[mt][4 * q + 3]};
   __syncthreads();
-  if (kc > 0) return;
+  if (wave >= 4 * NT) return;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     most_a = fmaxf(most_a, sizes[i]);
     most_w = fmaxf(most_w, sizes[8 + i]);
   }
   const float limit = redo_limit(most_a, most_w, K);
+  const int nw = n0 + wave * 8;                              // (lane l: rows 4 (l / 32) .. + 3 of these)
   bool any_small = false, odd = false;
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int m = m0 + mt * 32 + r;
+    f32x4_t v = sums[((wave >> 2) * MT + mt) * 256 + (wave & 3) * 64 + lane];
 #pragma unroll
-    for (int e4 = 0; e4 < 4; ++e4) {
-      float v[4];
+    for (int o = 1; o < KH; ++o) v += sums[((o * NT + (wave >> 2)) * MT + mt) * 256 + (wave & 3) * 64 + lane];
+    const int cn = nw + h * 4;
+    if (m >= M) continue;
+    float* cp = C + (size_t)m * N + cn;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int e = e4 * 4 + c;
-        float sum = acc[mt][e];
+    for (int c = 0; c < 4; ++c) {
+      any_small |= cn + c < N && fabsf(v[c]) <= limit;
+      odd |= cn + c < N && !(fabsf(v[c]) < INFINITY);
+    }
+    if (cn + 3 < N && (((uintptr_t)cp) & 15) == 0) {
+      *reinterpret_cast<f32x4_t*>(cp) = v;
+    } else {
 #pragma unroll
-        for (int o = 1; o < KH; ++o) sum += sums[((((o - 1) * NT + wt) * MT + mt) * 16 + e) * 64 + lane];
-        v[c] = sum;
-      }
-      const int cn = n0 + wt * 32 + e4 * 8 + h * 4;
-      if (m >= M) continue;
-      float* cp = C + (size_t)m * N + cn;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        any_small |= cn + c < N && fabsf(v[c]) <= limit;
-        odd |= cn + c < N && !(fabsf(v[c]) < INFINITY);
-      }
-      if (cn + 3 < N && (((uintptr_t)cp) & 15) == 0) {
-        *reinterpret_cast<f32x4_t*>(cp) = (f32x4_t){v[0], v[1], v[2], v[3]};
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (cn + c < N) cp[c] = v[c];
-      }
+      for (int c = 0; c < 4; ++c)
+        if (cn + c < N) cp[c] = v[c];
     }
   }
   if (!__any(any_small) && !__any(odd)) return;
   const int k_begin = s_begin * COLS, k_end = min(K, (s_begin + n) * COLS);
-  const int nw = n0 + wt * 32;
-  auto row_of = [&](int x) { return m0 + (x >> 4) * 32 + r; };
-  auto col_of = [&](int x) { return nw + ((x & 15) >> 2) * 8 + h * 4 + (x & 3); };
-  auto in_row = [&](int m) { return ((m - m0) & 31) == r ? 0xffffull << ((m - m0) >> 5) * 16 : 0ull; };
-  auto in_col = [&](int n) {
-    const int q = n - nw;
-    return ((q >> 2) & 1) == h ? 0x0001000100010001ull << ((q >> 3) * 4 + (q & 3)) : 0ull;
-  };
+  auto row_of = [&](int x) { return m0 + (x >> 2) * 32 + r; };
+  auto col_of = [&](int x) { return nw + h * 4 + (x & 3); };
+  auto in_row = [&](int m) { return ((m - m0) & 31) == r ? 0xfull << ((m - m0) >> 5) * 4 : 0ull; };
+  auto in_col = [&](int n) { return ((n - nw) >> 2) == h ? 0x1111ull << ((n - nw) & 3) : 0ull; };
   unsigned long long small = 0;                              // which of them, from what this lane has just stored
 #pragma unroll 16
-  for (int x = 0; x < MT * 16; ++x) {
+  for (int x = 0; x < MT * 4; ++x) {
     const int m = row_of(x), cn = col_of(x);
     const float v = C[(size_t)min(m, M - 1) * N + min(cn, N - 1)];
     small |= m < M && cn < N && fabsf(v) <= limit ? 1ull << x : 0ull;
   }
   const bool left = settle(A, W, C, small, N, K, k_begin, k_end, limit, row_of, col_of, in_row, in_col);
   const float below = left && small_operands(least_key(A, m0, 32 * MT, M, K, k_begin, k_end),
-                                             least_key(W, nw, 32, N, K, k_begin, k_end)) ? limit : -1.f;
+                                             least_key(W, nw, 8, min(nw + 8, N), K, k_begin, k_end)) ? limit : -1.f;
   if (!odd && !(small != 0 && below >= 0.f)) return;
-  for (int x = 0; x < MT * 16; ++x) {
+  for (int x = 0; x < MT * 4; ++x) {
     const int m = row_of(x), cn = col_of(x);
     if (m < M && cn < N) redo(A, W, C, m, cn, N, K, k_begin, k_end, below);
   }
@@ -713,7 +704,8 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
 template <int MT, int NT, int NB>
 static int launch_f32_wide(const void* A, const void* W, void* C, int M, int N, int K, int parts, size_t part_stride,
                            hipStream_t stream) {
-  constexpr int lds = NB * 32 * (NT + MT) * 512 / NT;
+  constexpr int ring = NB * 32 * (NT + MT) * 512 / NT, sums = 8 * MT * 4096;
+  constexpr int lds = ring > sums ? ring : sums;
   static bool sized[64] = {};                      // (per device: more than 64 KB of LDS has to be asked for)
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
