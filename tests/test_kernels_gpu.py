@@ -212,6 +212,32 @@ def test_gemm_f32_of_short_rows(monkeypatch, M, N, K):
     assert torch.equal(torch.isnan(out), torch.isnan(want)) and torch.equal(torch.isinf(out), torch.isinf(want))
 
 
+# (256 compute units)  more than 256 workgroups of 32 rows of W, at most 256 of 64, slices of more than 1,024 columns: two tiles
+# of W a wave; past each of these lines one
+@pytest.mark.parametrize("M,N,K,parts", [(5, 8193, 1028, 1), (32, 8256, 1156, 1), (17, 16384, 1100, 1), (31, 4100, 2056, 2), (24, 1100, 8300, 8),
+                                         (17, 16385, 1100, 1), (17, 8193, 1024, 1), (33, 8256, 1156, 1), (17, 8192, 1100, 1)])
+def test_gemm_f32_of_few_rows_over_a_long_walk(M, N, K, parts):
+    """Ordinary rows, rows of zeros, very small ones beside a very large one of W, infinities at both ends, in all tiles."""
+    from serve_amd import ops
+    a, w = rnd((M, K), torch.float32, 60), rnd((N, K), torch.float32, 61, 0.1)
+    a[1], a[3], a[M - 1] = 0, a[3] * 2.0 ** -127, a[M - 1] * 2.0 ** -110
+    w[5] *= 2.0 ** 100
+    w[N - 1] = 0
+    out = torch.full((parts, M, N), float("nan"), dtype=torch.float32, device=DEV)
+    ops.gemm_f32_mid_parts(a, w, out)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    got = out.double().sum(0)
+    # the terms left out are below 2^-23 of theirs; six instructions for every 16 columns round a running sum (at most `size`)
+    # by at most 2^-24 of it each, and so do the sums that are joined at the end; below 2^-126 parts are multiples of 2^-149
+    assert ((got - want).abs() <= size * (2.0 ** -23 + (6 * (K // 16 + 1) + 16) * 2.0 ** -24) + parts * 2.0 ** -149).all()
+    assert (got[1] == 0).all() and (got[:, N - 1] == 0).all()
+    a[0, 1], a[M - 1, K - 1], w[N - 1] = float("inf"), -float("inf"), 1
+    ops.gemm_f32_mid_parts(a, w, out)
+    want, got = a.double() @ w.double().T, out.double().sum(0)
+    assert torch.equal(torch.isinf(got), torch.isinf(want)) and not torch.isnan(got).any()
+    assert torch.equal(got[0].sign(), want[0].sign()) and torch.equal(got[M - 1].sign(), want[M - 1].sign())
+
+
 @pytest.mark.parametrize("M,N,K,parts", [(129, 70, 36, 1), (161, 64, 260, 2), (257, 200, 132, 3), (319, 129, 68, 1), (383, 4100, 64, 1)])
 def test_gemm_f32_by_split_operands_with_the_end_cut_off(monkeypatch, M, N, K, parts):
     """The rows behind the last whole tile through the kernel of few rows: the same sums as of those rows alone, in every
