@@ -454,52 +454,43 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(const u32x4_t* _
 
 // ---------------------------------------------------------------------------------------------
 // Up to 128 rows (decode steps of the 32-bit path): the work is reading W, once.  A workgroup of eight waves owns 32 NT
-// rows of W and MT tiles of 32 rows of A (gridDim.y runs of them; which, see few_rows).  A stage is 128 WT / NT columns of both
-// (a row of it is 512 WT / NT bytes), loaded straight into LDS, a kilobyte an instruction, in a ring of NB stages: no registers
-// hold what is on its way.  Wave = (tiles of W wt .. wt + WT - 1, run of 16 columns kc): it reads its fragments (lane l: row
-// l % 32, eight columns from 8 (l / 32)), splits them and multiplies; the sums of a tile's waves are added through LDS at the
-// end, in order.  Segment s (16 bytes) of row r lies at slot s ^ (r & 15): a 16-byte LDS read serves 16 lanes a cycle, in the
-// groups 0-3, 12-15, 20-23, 24-27 and 4-7, 8-11, 16-19, 28-31, and rows of 256 bytes and more then touch every bank once.
+// rows of W and MT tiles of 32 rows of A (gridDim.y runs of them; which, see few_rows).  A stage is 128 / NT columns of both (a row of it is 512 / NT bytes),
+// loaded straight into LDS, a kilobyte an instruction, in a ring of NB stages: no registers hold what is on its way.
+// Wave = (tile of W wt, run of 16 columns kc): it reads its fragments (lane l: row l % 32, eight columns from 8 (l / 32)),
+// splits them and multiplies; the sums of a tile's waves are added through LDS at the end, in order.  Segment s (16 bytes)
+// of row r lies at slot s ^ (r & 15): a 16-byte LDS read serves 16 lanes a cycle, in the groups 0-3, 12-15, 20-23, 24-27
+// and 4-7, 8-11, 16-19, 28-31, and rows of 256 bytes and more then touch every bank once.
 // gridDim.z parts of K, each with sums [M, N] of its own.
 //
-// Measured, the float32 matrix instruction / this kernel in us (weights not in a cache): K 2048, 16,384 rows of W 43 / 32 at
+// Measured, the float32 matrix instruction / this kernel in us (weights not in a cache): K 2048, 16,384 rows of W 43 / 33 at
 // 24 rows of A, 65 / 41 at 64, 121 / 67 at 128; 3,072 rows of W in four parts 20 / 10, 2,048 in eight 8.7 / 8.3; K 8192, 2,048
 // rows in eight parts 24 / 19; 128,256 rows 315 / 219 at 24, 489 / 332 at 64, 965 / 550 at 128.  A step at 24 rows reads
-// its 134 MB at 4.2 TB/s; from 64 rows on the splits of A, which every workgroup makes again, weigh as much.  Distance to
+// its 134 MB at 4.1 TB/s; from 64 rows on the splits of A, which every workgroup makes again, weigh as much.  Distance to
 // 64 bits (rms, of the result's size), normal operands: K 2048 2.9e-7 / 1.1e-7 at 24 rows and 1.35e-7 at 100, K 8192 3.9e-7 /
 // 1.4e-7 at 64 and 100; operands in 1 .. 2: 0.97e-7 / 0.48e-7 and 0.68e-7, 0.88e-7 / 0.56e-7.
-// Two tiles of W a wave (WT): the fragments of A are read and split once for both, eight waves to a row of 512 bytes.  With up to
-// 32 rows, one tile a wave / two, us: K 2048, 10,240 rows of W 27.3 / 24.8, 16,384 34.7 / 31.7 (31.2 / 30.6 at 8 rows); K 4096,
-// 14,336 rows 55.9 / 52.6; K 14336 in four parts, 4,096 rows 54.0 / 48.0; level at a walk of 1,024 columns (2,048 rows at K 8192 in
-// eight parts 17.8 / 18.0) and behind at 512 (3,072 rows 11.1 / 11.6: a ring of three such stages is hardly filled), and behind
-// where there are more workgroups than compute units (128,256 rows 221 / 240), as two of those of 73 KB run on one.  Distance to
-// 64 bits at K 2048 1.3e-7 / 1.1e-7, K 4096 and more 1.4e-7 / 1.4e-7; four steps of 24 rows of the 1B shape 7.17 / 7.08 ms.
+// Up to 32 rows of A a workgroup of 64 rows of W stays below half of a compute unit's LDS.  One whose waves take both tiles of W
+// (a fragment of A split once for the two, 147 KB of stages) needs a compute unit for itself: 256 of them over 16,384 rows of W
+// at K 2048, in decode steps, us a launch: 27.6 on one device, and 27, 34 or 38 by turns (32.2 on the average) on another, as if some had to
+// wait there for others to end; this one 29.8 and one mode.
 // From five rows, with K in parts: level with the kernel of few rows of csrc/gemm.hip over 3,072 and 2,048 rows of W at K 2048
 // (9.3 and 8.2 us there, 9.9 and 8.1 here), 21.3 / 18.6 over 2,048 at K 8192.  Up to 128 rows, which is what a stage has room
 // for: at 128 the tiles above take 20, 87 (16,384 rows of W) and 51 us where this takes 15, 64 and 37, and only over
 // 128,256 rows of W 366 for 550.
 // ---------------------------------------------------------------------------------------------
-template <int MT, int WT, int ROWB>
-__device__ __forceinline__ void read_rows(Frag8 (&w)[WT][2], Frag8 (&a)[MT][2], uint32_t w0, uint32_t w1, uint32_t a0, uint32_t a1) {
-  constexpr int TILE = 32 * ROWB;                            // bytes from tile to tile
-  static_assert(WT == 1 || (WT == 2 && MT == 1), "");
+template <int MT, int NT>
+__device__ __forceinline__ void read_rows(Frag8 (&w)[2], Frag8 (&a)[MT][2], uint32_t w0, uint32_t w1, uint32_t a0, uint32_t a1) {
+  constexpr int TILE = 32 * 512 / NT;                        // bytes from tile to tile
   // (blocks with their own wait: the compiler does not know that loads into LDS are stores there)
-  if constexpr (MT == 1 && WT == 1) {
+  if constexpr (MT == 1) {
     asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\t"
                  "s_waitcnt lgkmcnt(0)"
-                 : "=&v"(w[0][0].u), "=&v"(w[0][1].u), "=&v"(a[0][0].u), "=&v"(a[0][1].u)
+                 : "=&v"(w[0].u), "=&v"(w[1].u), "=&v"(a[0][0].u), "=&v"(a[0][1].u)
                  : "v"(w0), "v"(w1), "v"(a0), "v"(a1)
-                 : "memory");
-  } else if constexpr (MT == 1) {
-    asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %7\n\tds_read_b128 %2, %8\n\tds_read_b128 %3, %9\n\t"
-                 "ds_read_b128 %4, %6 offset:%10\n\tds_read_b128 %5, %7 offset:%10\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(w[0][0].u), "=&v"(w[0][1].u), "=&v"(a[0][0].u), "=&v"(a[0][1].u), "=&v"(w[1][0].u), "=&v"(w[1][1].u)
-                 : "v"(w0), "v"(w1), "v"(a0), "v"(a1), "n"(TILE)
                  : "memory");
   } else {
     asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %7\n\tds_read_b128 %2, %8\n\tds_read_b128 %3, %9\n\t"
                  "ds_read_b128 %4, %8 offset:%10\n\tds_read_b128 %5, %9 offset:%10\n\ts_waitcnt lgkmcnt(0)"
-                 : "=&v"(w[0][0].u), "=&v"(w[0][1].u), "=&v"(a[0][0].u), "=&v"(a[0][1].u), "=&v"(a[1][0].u), "=&v"(a[1][1].u)
+                 : "=&v"(w[0].u), "=&v"(w[1].u), "=&v"(a[0][0].u), "=&v"(a[0][1].u), "=&v"(a[1][0].u), "=&v"(a[1][1].u)
                  : "v"(w0), "v"(w1), "v"(a0), "v"(a1), "n"(TILE)
                  : "memory");
     if constexpr (MT == 3)
@@ -516,21 +507,21 @@ __device__ __forceinline__ void read_rows(Frag8 (&w)[WT][2], Frag8 (&a)[MT][2], 
   }
 }
 
-template <int MT, int NT, int NB, int WT>
+template <int MT, int NT, int NB>
 __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restrict__ A, const float* __restrict__ W,
                                                            float* __restrict__ C, int M, int N, int K, size_t part_stride) {
-  constexpr int COLS = 128 * WT / NT;                        // of a stage
+  constexpr int COLS = 128 / NT;                             // of a stage
   constexpr int ROWB = COLS * 4, SEGS = ROWB / 16;           // bytes and 16-byte segments of a row
   constexpr int ROWS = 32 * (NT + MT);                       // W's, then A's
   constexpr int STAGE = ROWS * ROWB;
   constexpr int RPI = 64 / SEGS;                             // rows an instruction loads
   constexpr int ND = ROWS / RPI / 8;                         // instructions a wave and stage
   static_assert(ROWS % (RPI * 8) == 0, "every wave issues the same number of loads");
-  constexpr int KH = 8 * WT / NT;                            // waves a tile of W
+  constexpr int KH = 8 / NT;                                 // waves a tile of W
   extern __shared__ __attribute__((aligned(16))) unsigned char ring[];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wt = wave % (NT / WT) * WT, kc = wave / (NT / WT);
+  const int wt = wave % NT, kc = wave / NT;
   const int r = lane & 31, h = lane >> 5;
   const int n0 = blockIdx.x * 32 * NT, m0 = blockIdx.y * 32 * MT;
   const int all = (K + COLS - 1) / COLS;
@@ -578,18 +569,15 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   // the large products x0 w0 and the small ones in sums of their own: a rounding of the large sum an instruction, not six
   // (the large ones in two levels; with four tiles of A there are no registers for it, and the launch keeps K short)
   constexpr int TOTALS = MT <= 3 ? MT : 0;
-  floatx16_t acc[WT][MT], low[WT][MT], total[WT][TOTALS ? TOTALS : 1];
+  floatx16_t acc[MT], low[MT], total[TOTALS ? TOTALS : 1];
 #pragma unroll
-  for (int wi = 0; wi < WT; ++wi) {
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int e = 0; e < 16; ++e) acc[mt][e] = low[mt][e] = 0.f;
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[wi][mt][e] = low[wi][mt][e] = 0.f;
+  for (int mt = 0; mt < TOTALS; ++mt)
 #pragma unroll
-    for (int mt = 0; mt < TOTALS; ++mt)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) total[wi][mt][e] = 0.f;
-  }
+    for (int e = 0; e < 16; ++e) total[mt][e] = 0.f;
 
   if (n > 0) {
 #pragma unroll
@@ -601,8 +589,8 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
         SP_STAGE_END(ND * (NB - 2));
         fetch(s + NB - 1);
         const uint32_t off = (uint32_t)((s % NB) * STAGE);
-        Frag8 wf[WT][2], af[MT][2];
-        read_rows<MT, WT, ROWB>(wf, af, w0 + off, w1 + off, a0 + off, a1 + off);
+        Frag8 wf[2], af[MT][2];
+        read_rows<MT, NT>(wf, af, w0 + off, w1 + off, a0 + off, a1 + off);
         const int at = stage_of(s), k = at * COLS + kc * 16 + h * 8;
         if ((at + 1) * COLS > K) {                             // the last columns: beyond K the operand of A is zero
           const u32x4_t zero4 = {0u, 0u, 0u, 0u};
@@ -614,45 +602,34 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
         }
         constexpr int PA[5] = {2, 1, 0, 1, 0}, PW[5] = {0, 1, 2, 0, 1};
         u32x4_t q[3];
-        Frag8 w[WT][3], a[MT][3];
+        Frag8 w[3], a[MT][3];
+        split8(wf[0].f, wf[1].f, q);
+        max8(most_w, wf[0].f, wf[1].f);
 #pragma unroll
-        for (int wi = 0; wi < WT; ++wi) {
-          split8(wf[wi][0].f, wf[wi][1].f, q);
-          max8(most_w, wf[wi][0].f, wf[wi][1].f);
-#pragma unroll
-          for (int p = 0; p < 3; ++p) w[wi][p].u = q[p];
-        }
+        for (int p = 0; p < 3; ++p) w[p].u = q[p];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
           split8(af[mt][0].f, af[mt][1].f, q);
           max8(most_a, af[mt][0].f, af[mt][1].f);
 #pragma unroll
           for (int p = 0; p < 3; ++p) a[mt][p].u = q[p];
+          acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[0].v, a[mt][0].v, acc[mt], 0, 0, 0);
 #pragma unroll
-          for (int wi = 0; wi < WT; ++wi) {
-            acc[wi][mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[wi][0].v, a[mt][0].v, acc[wi][mt], 0, 0, 0);
-#pragma unroll
-            for (int p = 0; p < 5; ++p)
-              low[wi][mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[wi][PW[p]].v, a[mt][PA[p]].v, low[wi][mt], 0, 0, 0);
-          }
+          for (int p = 0; p < 5; ++p)
+            low[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[PW[p]].v, a[mt][PA[p]].v, low[mt], 0, 0, 0);
         }
       }
 #pragma unroll
-      for (int wi = 0; wi < WT; ++wi)
+      for (int mt = 0; mt < TOTALS; ++mt) {
+        total[mt] += acc[mt];
 #pragma unroll
-        for (int mt = 0; mt < TOTALS; ++mt) {
-          total[wi][mt] += acc[wi][mt];
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[wi][mt][e] = 0.f;
-        }
+        for (int e = 0; e < 16; ++e) acc[mt][e] = 0.f;
+      }
     }
 #pragma unroll
-    for (int wi = 0; wi < WT; ++wi) {
+    for (int mt = 0; mt < TOTALS; ++mt) acc[mt] = total[mt];
 #pragma unroll
-      for (int mt = 0; mt < TOTALS; ++mt) acc[wi][mt] = total[wi][mt];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) acc[wi][mt] += low[wi][mt];
-    }
+    for (int mt = 0; mt < MT; ++mt) acc[mt] += low[mt];
     SP_STAGE_END(0);                                         // (loads beyond the last stage; everybody has read it)
   }
 
@@ -668,13 +645,11 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   // 3,072 rows of W 11.7 / 11.1 so; 100 rows, 16,384 of W 75.5 / 70.6; 128 rows, 128,256 of W 575 / 544.)
   f32x4_t* sums = reinterpret_cast<f32x4_t*>(ring);          // [KH][NT][MT][4][64]
 #pragma unroll
-  for (int wi = 0; wi < WT; ++wi)
+  for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        sums[(((kc * NT + wt + wi) * MT + mt) * 4 + q) * 64 + lane] =
-            (f32x4_t){acc[wi][mt][4 * q], acc[wi][mt][4 * q + 1], acc[wi][mt][4 * q + 2], acc[wi][mt][4 * q + 3]};
+    for (int q = 0; q < 4; ++q)
+      sums[((wave * MT + mt) * 4 + q) * 64 + lane] =
+          (f32x4_t){acc[mt][4 * q], acc[mt][4 * q + 1], acc[mt][4 * q + 2], acc[mt][4 * q + 3]};
   __syncthreads();
   if (wave >= 4 * NT) return;
 #pragma unroll
@@ -730,22 +705,23 @@ __global__ __launch_bounds__(512) void gemm_f32_wide_kernel(const float* __restr
   }
 }
 
-template <int MT, int NT, int NB, int WT = 1>
+template <int MT, int NT, int NB>
 static int launch_f32_wide(const void* A, const void* W, void* C, int M, int N, int K, int parts, size_t part_stride,
                            hipStream_t stream) {
-  constexpr int ring = NB * 32 * (NT + MT) * 512 * WT / NT, sums = 8 * WT * MT * 4096;
+  constexpr int ring = NB * 32 * (NT + MT) * 512 / NT, sums = 8 * MT * 4096;
   constexpr int lds = ring > sums ? ring : sums;
+  static_assert(MT > 1 || NT < 2 || 2 * lds < 160 * 1024, "two workgroups a compute unit");
   static bool sized[64] = {};                      // (per device: more than 64 KB of LDS has to be asked for)
   int dev = 0;
   hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return (int)e;
   if (dev < 0 || dev >= 64 || !sized[dev]) {
-    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_wide_kernel<MT, NT, NB, WT>),
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_f32_wide_kernel<MT, NT, NB>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (e != hipSuccess) return (int)e;
     if (dev >= 0 && dev < 64) sized[dev] = true;
   }
-  hipLaunchKernelGGL((gemm_f32_wide_kernel<MT, NT, NB, WT>), dim3((N + 32 * NT - 1) / (32 * NT), (M + 32 * MT - 1) / (32 * MT), parts), dim3(512), lds,
+  hipLaunchKernelGGL((gemm_f32_wide_kernel<MT, NT, NB>), dim3((N + 32 * NT - 1) / (32 * NT), (M + 32 * MT - 1) / (32 * MT), parts), dim3(512), lds,
                      stream, (const float*)A, (const float*)W, (float*)C, M, N, K, part_stride);
   SA_LAUNCH_CHECK();
   return 0;
@@ -764,8 +740,6 @@ static int few_rows(const void* A, const void* W, void* C, int M, int N, int K, 
   if (w32 * a32 <= cus) return launch_f32_wide<1, 1, 3>(A, W, C, M, N, K, parts, part_stride, stream);
   if (w64 * a32 <= cus && K / parts <= 1024) return launch_f32_wide<1, 2, 3>(A, W, C, M, N, K, parts, part_stride, stream);
   if (w32 * a64 <= cus) return launch_f32_wide<2, 1, 3>(A, W, C, M, N, K, parts, part_stride, stream);
-  // (one workgroup a compute unit, a long walk: both tiles of W a wave)
-  if (M <= 32 && w64 <= cus) return launch_f32_wide<1, 2, 3, 2>(A, W, C, M, N, K, parts, part_stride, stream);
   if (M <= 32) return launch_f32_wide<1, 2, 3>(A, W, C, M, N, K, parts, part_stride, stream);
   // (four tiles of A have no registers for sums in two levels: not over a long inner size)
   if (M <= 64 || w64 * a64 <= cus || (M > 96 && K / parts > 4096))

@@ -212,8 +212,8 @@ def test_gemm_f32_of_short_rows(monkeypatch, M, N, K):
     assert torch.equal(torch.isnan(out), torch.isnan(want)) and torch.equal(torch.isinf(out), torch.isinf(want))
 
 
-# (256 compute units)  more than 256 workgroups of 32 rows of W, at most 256 of 64, slices of more than 1,024 columns: two tiles
-# of W a wave; past each of these lines one
+# (256 compute units)  more than 256 workgroups of 32 rows of W, at most 256 of 64, slices of more than 1,024 columns; and past
+# each of these lines
 @pytest.mark.parametrize("M,N,K,parts", [(5, 8193, 1028, 1), (32, 8256, 1156, 1), (17, 16384, 1100, 1), (31, 4100, 2056, 2), (24, 1100, 8300, 8),
                                          (17, 16385, 1100, 1), (17, 8193, 1024, 1), (33, 8256, 1156, 1), (17, 8192, 1100, 1)])
 def test_gemm_f32_of_few_rows_over_a_long_walk(M, N, K, parts):
@@ -371,7 +371,7 @@ def test_gemm_f32_by_split_operands_is_as_close_as_sums_in_two_levels(M, N, K, s
     assert rms(out) <= rms(total), (rms(out), rms(total))
 
 
-@pytest.mark.parametrize("M,N,K", [(24, 2048, 2048), (100, 1024, 8192), (300, 2048, 2048), (300, 512, 8192)])
+@pytest.mark.parametrize("M,N,K", [(24, 2048, 2048), (24, 10240, 2048), (100, 1024, 8192), (300, 2048, 2048), (300, 512, 8192)])
 def test_gemm_f32_by_split_operands_is_as_close_as_float32(M, N, K):
     """The distance to 64 bits is no larger than that of one float32 sum a result in steps of two columns (what the matrix
     cores' float32 instruction does)."""
