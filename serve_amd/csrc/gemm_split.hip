@@ -190,8 +190,10 @@ __device__ __forceinline__ void redo(const float* A, const float* W, float* C, i
 // A wave's small results, a bit each in `small`, one at a time by the two rows they come from: sums of ordinary operands that
 // cancel to zero, of which large products have one here and there (2,048 x 16,384 of 2,048 columns: one or two in all), and
 // those of rows of zeros, which go together.  (512 x 8,192 results, K 2048, one of them zero: 134 us with the wave's rows
-// searched as a whole for it, 105 so and without it; 24 rows, one of zeros, over 16,384: 61 and 32, 28 without it.)  True
-// where some are left after SP_FEW: the wave's rows are then searched as a whole, 30 us at K 2048.  `row_of` and `col_of`
+// searched as a whole for it, 105 so and without it.  24 rows over 16,384, K 2048, us, with W's row searched too for a row of A of
+// zeros / so: none 31.7 / 31.9, one 39.7 / 35.7, twelve 82.9 / 73.3; 100 rows, fifty of zeros 169 / 158.)  True where some are
+// left after SP_FEW: the wave's rows are then searched as a whole.  (With twice as many, twelve 49 and fifty 167, but where all
+// numbers are small 1,900 us for 1,265 at 24 rows and 3,709 for 3,109 at 100.)  `row_of` and `col_of`
 // give a bit's place, `in_row` and `in_col` this lane's bits of a row of A and of one of W.  For a whole wave.
 #define SP_FEW 8
 template <typename RowOf, typename ColOf, typename InRow, typename InCol>
@@ -204,10 +206,14 @@ __device__ __forceinline__ bool settle(const float* A, const float* W, float* C,
     const int l = __builtin_ctzll(lanes);
     const int x = small ? __builtin_ctzll(small) : 0;
     const int m = __builtin_amdgcn_readlane(row_of(x), l), n = __builtin_amdgcn_readlane(col_of(x), l);
-    const uint32_t ka = least_key(A + (size_t)m * K, k_begin, k_end), kw = least_key(W + (size_t)n * K, k_begin, k_end);
-    if (small_operands(ka, kw) && lane == l) redo(A, W, C, m, n, N, K, k_begin, k_end, limit);
     if (lane == l) small &= small - 1;
-    if (ka == 0xffffffffu) small &= ~in_row(m);
+    const uint32_t ka = least_key(A + (size_t)m * K, k_begin, k_end);
+    if (ka == 0xffffffffu) {                                           // (then W's row is of no account)
+      small &= ~in_row(m);
+      continue;
+    }
+    const uint32_t kw = least_key(W + (size_t)n * K, k_begin, k_end);
+    if (small_operands(ka, kw) && lane == l) redo(A, W, C, m, n, N, K, k_begin, k_end, limit);
     if (kw == 0xffffffffu) small &= ~in_col(n);
   }
   return __any(small != 0);

@@ -238,6 +238,24 @@ def test_gemm_f32_of_few_rows_over_a_long_walk(M, N, K, parts):
     assert torch.equal(got[0].sign(), want[0].sign()) and torch.equal(got[M - 1].sign(), want[M - 1].sign())
 
 
+@pytest.mark.parametrize("M,N,K,parts", [(24, 70, 516, 1), (32, 520, 260, 8), (100, 8200, 132, 1), (128, 200, 1028, 3), (300, 129, 516, 1)])
+@pytest.mark.parametrize("every", [2, 9])                  # rows of zeros: more than a wave looks at one by one, and fewer
+def test_gemm_f32_of_rows_of_zeros_beside_very_small_ones(M, N, K, parts, every):
+    """Zeros stay zeros, and rows whose smallest parts lie below the normal numbers keep their digits beside them."""
+    from serve_amd import ops
+    a, w = rnd((M, K), torch.float32, 62), rnd((N, K), torch.float32, 63, 0.1)
+    a[::every] = 0
+    a[1], a[3 + every], w[2] = a[1] * 2.0 ** -110, a[3 + every] * 2.0 ** -120, w[2] * 2.0 ** -100
+    w[::8] = 0
+    out = torch.full((parts, M, N), float("nan"), dtype=torch.float32, device=DEV)
+    (ops.gemm_f32_mid_parts if M <= ops.F32_MID_MAX_ROWS else ops.gemm_f32_split)(a, w, out)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    got = out.double().sum(0)
+    assert (got[::every] == 0).all() and (got[:, ::8] == 0).all()
+    # (as above: the terms left out, the sums' roundings, and results below 2^-126 in multiples of 2^-149)
+    assert ((got - want).abs() <= size * (2.0 ** -23 + (6 * (K // 16 + 1) + 16) * 2.0 ** -24) + parts * 2.0 ** -149).all()
+
+
 @pytest.mark.parametrize("M,N,K,parts", [(129, 70, 36, 1), (161, 64, 260, 2), (257, 200, 132, 3), (319, 129, 68, 1), (383, 4100, 64, 1)])
 def test_gemm_f32_by_split_operands_with_the_end_cut_off(monkeypatch, M, N, K, parts):
     """The rows behind the last whole tile through the kernel of few rows: the same sums as of those rows alone, in every
