@@ -33,7 +33,7 @@ typedef const __attribute__((address_space(1))) void* gptr_t;
 
 // FIRST: act[r] = gate(Wg_e x, Wu_e x) with x = A[perm[r] / top], W [2, E, N, K] (gates, then ups, `up_offset` rows apart).
 // else:  C[perm[r]] = W_e A[r], W [E, N, K].  r: grouped rows of this tile.
-// perm null (the shared expert): every row in its place, and C in bf16 either way.
+// SHARED (a template argument): every row in its place; perm, top, the tiles' lists and in_wts are not read.
 struct ExpertArgs {
   const bf16_t* A;
   const bf16_t* W;
@@ -180,7 +180,7 @@ __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, i
       const int m = (rg * RT + mt) * 16 + c;
       if (m >= M) continue;
       const int r = row0 + m;
-      const int at = SHARED || (FIRST && !p.in_wts) ? 0 : p.perm[r];
+      const int at = SHARED ? r : FIRST && !p.in_wts ? 0 : p.perm[r];
       const float in_w = FIRST && !SHARED && p.in_wts ? p.in_wts[at] : 1.f;   // (a weight on the input: gate and up are linear in it)
 #pragma unroll
       for (int nt = 0; nt < (FIRST ? CT / 2 : CT); ++nt) {
@@ -196,7 +196,7 @@ __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, i
           }
         }
         if (n < N) {                                 // (N is a multiple of 64)
-          if constexpr (FIRST || SHARED) {
+          if constexpr (FIRST) {
             uint2 q;
             q.x = floats_to_bf16_bits(o[0], o[1]);
             q.y = floats_to_bf16_bits(o[2], o[3]);
@@ -355,7 +355,7 @@ extern "C" int sa_expert_tile_rows(int rows, int E, int F) {
 //            (in_wts, fp32 [T top] or null: both sums times the row's weight first, for weights on the experts' inputs)
 //   down:    act [rows, F], Wd [E, d, F] -> yk [T top, d] fp32 at row perm[r]
 // Sgu not null: in the same two launches a shared expert for all T rows, its gates and ups Sgu [2 S, d], Sd [d, S], the same kind of
-// gate with its own limit: s_act [T, S], s_out [T, d], both bf16 (S a multiple of 64).
+// gate with its own limit: s_act [T, S] bf16, s_out [T, d] fp32 (S a multiple of 64).
 extern "C" int sa_expert_products(const void* h, const void* Wgu, const void* Wd, void* act, float* yk, int E, int d, int F,
                                   int max_tiles, const int* perm, const int* tile_expert, const int* tile_row0,
                                   const int* num_tiles, int top, int gate_kind, float gate_limit, const float* in_wts,

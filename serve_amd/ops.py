@@ -1534,7 +1534,7 @@ def moe_wide_available(h: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor
 
 
 class SharedExpert:
-    """A shared expert's matrices for `moe_experts`, which leaves its rows [T, d] in `out`."""
+    """A shared expert's matrices for `moe_experts`, which leaves its rows, fp32 [T, d], in `out`."""
 
     def __init__(self, w_gate_up: torch.Tensor, w_down: torch.Tensor, limit: float = 0.0):
         self.w_gate_up, self.w_down, self.limit = w_gate_up, w_down, float(limit)
@@ -1620,7 +1620,7 @@ def moe_experts(h: torch.Tensor, ids: torch.Tensor, w_gate: torch.Tensor, w_up: 
             _check(moe_shared_available(h, sgu, sd) and sgu.shape == (2 * S, d), "the shared expert's matrices must be bf16 [2 S, d], [d, S]")
             _check(gate != "clamped_swish" or s_limit > 0.0, "the clamped gate needs a positive limit")
             s_act = torch.empty((T, S), dtype=h.dtype, device=h.device)
-            s_out = shared.out = torch.empty((T, d), dtype=h.dtype, device=h.device)
+            s_out = shared.out = torch.empty((T, d), dtype=torch.float32, device=h.device)
         _ret(wide.sa_expert_products(_ptr(h), _ptr(w_gate), _ptr(w_down), _ptr(act), _ptr(yk), c_int(E), c_int(d), c_int(F),
                               c_int(-(-n // rows) + E), c_void_p(perm), c_void_p(tile_expert),
                               c_void_p(tile_row0), c_void_p(num_tiles), c_int(top), c_int(GATES[gate]), c_float(limit),

@@ -839,6 +839,72 @@ def test_a_shared_expert_in_the_experts_launches(T, d, S, gate, limit, shared_li
     assert shared.out.shape == (T, d) and ((shared.out.double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("T,d,S", [(65, 64, 64), (100, 320, 128), (129, 128, 64), (700, 64, 192)])
+def test_a_shared_expert_in_the_experts_launches_stays_in_32_bits_behind_its_gate(T, d, S):
+    """One column of the last matrix: a result is one product of two bf16 numbers, which has more bits than bf16."""
+    from serve_amd import ops
+    E, F, top = 64, 128, 2
+    g = torch.Generator("cuda").manual_seed(T + d + S)
+    h = torch.randn((T, d), device="cuda", generator=g).bfloat16()
+    wgu, wd = torch.zeros((2, E, F, d), device="cuda").bfloat16(), torch.zeros((E, d, F), device="cuda").bfloat16()
+    sgu = (torch.randn((2 * S, d), device="cuda", generator=g) * d ** -0.5).bfloat16()
+    sd = torch.zeros((d, S), device="cuda").bfloat16()
+    sd[:, S - 3] = torch.randn((d,), device="cuda", generator=g).bfloat16()
+    sd[0, S - 3] = 1.0
+    ids = torch.stack([torch.randperm(E, device="cuda", generator=g)[:top] for _ in range(T)]).int().contiguous()
+    shared = ops.SharedExpert(sgu, sd)
+    ops.moe_experts(h, ids, wgu[0], wgu[1], wd, torch.empty((T * top, d), device="cuda"), shared=shared)
+    act = shared.out[:, 0].float()
+    assert torch.equal(act, act.bfloat16().float()) and (act != 0).float().mean() > 0.9
+    assert torch.equal(shared.out.float(), act[:, None] * sd[:, S - 3].float())
+
+
+def _gated(z, u, gate, limit):
+    if gate == "silu":
+        return z * torch.sigmoid(z) * u
+    if gate == "gelu_tanh":
+        return 0.5 * z * (1.0 + torch.tanh(math.sqrt(2.0 / math.pi) * (z + 0.044715 * z ** 3))) * u
+    z, u = z.clamp(max=limit), u.clamp(-limit, limit)
+    return z * torch.sigmoid(1.702 * z) * (u + 1.0)
+
+
+# (256 compute units) 256 weight rows a workgroup in both products of the experts, the last ones ragged; ahead and behind
+@pytest.mark.parametrize("gate", ["silu", "gelu_tanh", "clamped_swish"])
+@pytest.mark.parametrize("weight_inputs", [False, True])
+@pytest.mark.parametrize("T,S", [(129, 64), (200, 448), (640, 192), (641, 192), (1030, 320)])
+def test_a_shared_expert_beside_experts_of_wide_columns(T, S, weight_inputs, gate):
+    """... which takes no part in the weights on the experts' inputs and has a limit of its own."""
+    from serve_amd import ops
+    E, F, d, top, limit, shared_limit = 64, 320, 704, 2, 0.8, 1.7
+    g = torch.Generator("cuda").manual_seed(T + S)
+    h = torch.randn((T, d), device="cuda", generator=g).bfloat16()
+    wgu = (torch.randn((2, E, F, d), device="cuda", generator=g) * d ** -0.5).bfloat16()
+    wd = (torch.randn((E, d, F), device="cuda", generator=g) * F ** -0.5).bfloat16()
+    sgu = (torch.randn((2 * S, d), device="cuda", generator=g) * d ** -0.5).bfloat16()
+    sd = (torch.randn((d, S), device="cuda", generator=g) * S ** -0.5).bfloat16()
+    ids = torch.rand((T, E), device="cuda", generator=g).topk(top, dim=1).indices.int().contiguous()
+    weights = 0.25 + torch.rand((T, top), device="cuda", generator=g)
+    assert ops.moe_wide_pays(T * top, E, F) and 4 * E * -(-F // 128) >= 3 * ops.compute_units() and 4 * E * -(-d // 256) >= 3 * ops.compute_units()
+    alone, both = (torch.full((T * top, d), float("nan"), device="cuda") for _ in range(2))
+    more = dict(weights=weights, gate=gate, limit=limit, weight_inputs=weight_inputs)
+    ops.moe_experts(h, ids, wgu[0], wgu[1], wd, alone, **more)
+    shared = ops.SharedExpert(sgu, sd, shared_limit)
+    ops.moe_experts(h, ids, wgu[0], wgu[1], wd, both, shared=shared, **more)
+    assert torch.equal(alone, both), "the experts' own rows have changed"
+    x = h.double()
+    act = _gated(x @ sgu[:S].double().T, x @ sgu[S:].double().T, gate, shared_limit)
+    want = act @ sd.double().T
+    # the gated values are rounded to eight bits, by at most 2^-8 of each; the rest is float32
+    assert ((shared.out.double() - want).abs() <= 1.1 * 2.0 ** -8 * (act.abs() @ sd.double().abs().T)).all()
+    w_in = weights.double() if weight_inputs else torch.ones_like(weights, dtype=torch.float64)
+    rows = both.view(T, top, d).double()
+    for e in (0, 31, E - 1):
+        t, k = (ids == e).nonzero(as_tuple=True)
+        xe = x[t] * w_in[t, k][:, None]
+        act = _gated(xe @ wgu[0, e].double().T, xe @ wgu[1, e].double().T, gate, limit)
+        assert ((rows[t, k] - act @ wd[e].double().T).abs() <= 1.1 * 2.0 ** -8 * (act.abs() @ wd[e].double().abs().T)).all(), e
+
+
 @pytest.mark.parametrize("gate,limit", [("silu", 0.0), ("clamped_swish", 0.8)])
 @pytest.mark.parametrize("T,d,F,E,top", [(700, 128, 192, 5, 2), (300, 64, 64, 9, 4), (2048, 256, 128, 6, 1)])
 def test_experts_of_many_rows_with_both_operands_through_lds(T, d, F, E, top, gate, limit):
