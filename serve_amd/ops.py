@@ -1553,12 +1553,24 @@ def moe_shared_inside(h: torch.Tensor, top: int, w_gate: torch.Tensor, w_up: tor
     """Whether `moe_experts` computes the shared expert of these in its own launches, whose tiles of it fill what the experts leave of
     the chip.  Up to 128 tokens the products of few rows are as fast by themselves where the experts have workgroups for half of the
     chip (32 x 2048 x 1024 with a shared one of 2,048 at 24, 64 and 128 tokens 104, 114 and 124 us, in the experts' launches 103, 119
-    and 125; 8 of them with one of 1,024 at 64 53 / 41).  Large ones run faster in the library (16 x 4096 x 1024 with a shared one of
-    4,096 at 300, 512, 700 and 1,000 tokens 170 / 155, 193 / 184, 216 / 226, 244 / 252; the first shape at 2,048 and 4,096 259 / 258
-    and 443 / 452)."""
+    and 125; 8 of them with one of 1,024 at 64 53 / 41).  Large ones run faster in the library, from about 9e9 multiplications a
+    matrix on (16 x 4096 x 1024 with a shared one of 4,096 at 300, 512, 700 and 1,000 tokens, 4.9 to 17e9, 170 / 155, 193 / 184,
+    216 / 226, 244 / 252; the first shape at 2,048, 8.6e9, and 4,096 259 / 258 and 443 / 452).
+
+    A tile of the second product walks the whole inner width, in a chain that nothing shortens, where products of its own cut it in
+    parts: up to 2,048 always; up to 4,096 beside fewer tokens than tiles come behind for, in a model at least half as wide (as wide,
+    where the products are those of few rows).  By themselves / inside, us, experts x model width x expert width + shared: 8 x 2048 x 512 +
+    8,192 at 24, 129 and 400 tokens 67 / 87, 88 / 129, 126 / 157; 64 x 1024 x 1024 + 8,192 at 256 155 / 186; 8 x 1024 x 768 + 6,144 at 160
+    81 / 105; 16 x 1536 x 1024 + 4,096 at 64 79 / 91; 64 x 1024 x 512 + 4,096 at 320, 800 and 2,048 95 / 101, 115 / 129, 143 / 166; 64 x 3072
+    x 256 + 4,096 at 640 and 641 163 / 160, 171 / 193; 32 x 2048 x 256 + 3,072 at 96 and 256 77 / 82, 98 / 87; 8 x 5120 x 2048 + 4,096 at 256
+    243 / 186.  Over 866 drawn sizes the whole takes 0.895 of the time so, and 0.910 without these lines, over 626 others 0.920 and 0.949;
+    at the worst 13 and 84 % more than with products of its own."""
     E, F, _ = w_gate.shape
     T, d = h.shape
-    if T <= MOE_ROUTE_INSIDE or T * d * shared_down.shape[-1] > 9e9:
+    S = shared_down.shape[-1]
+    if T <= MOE_ROUTE_INSIDE or T * d * S > 9e9:
+        return False
+    if S > 2048 and (S > 4096 or T > 640 or S > (d if T <= SKINNY_MAX_ROWS else 2 * d)):
         return False
     if T <= SKINNY_MAX_ROWS and 2 * E * -(-F // 128) > compute_units():
         return False

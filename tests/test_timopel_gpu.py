@@ -905,6 +905,61 @@ def test_a_shared_expert_beside_experts_of_wide_columns(T, S, weight_inputs, gat
         assert ((rows[t, k] - act @ wd[e].double().T).abs() <= 1.1 * 2.0 ** -8 * (act.abs() @ wd[e].double().abs().T)).all(), e
 
 
+# T, d, E, F, top, S: both sides of each line of the rule
+@pytest.mark.parametrize("T,d,E,F,top,S,inside", [
+    (16, 128, 64, 128, 8, 64, False), (17, 128, 64, 128, 8, 64, True),                  # the routing in a call of its own
+    (128, 128, 64, 256, 4, 128, True), (128, 128, 64, 320, 4, 128, False), (129, 128, 64, 320, 4, 128, True),
+    (300, 64, 64, 128, 4, 2048, True), (300, 64, 64, 128, 4, 2112, False),
+    (300, 1088, 64, 128, 4, 2176, True), (300, 1088, 64, 128, 4, 2240, False), (128, 1088, 64, 128, 4, 2176, False),
+    (640, 1088, 64, 128, 2, 2176, True), (641, 1088, 64, 128, 2, 2176, False), (128, 2112, 64, 64, 4, 2112, True),
+    (2145, 2048, 8, 64, 1, 2048, True), (2146, 2048, 8, 64, 1, 2048, False)])
+@pytest.mark.parametrize("gate,limit,shared_limit", [("silu", 0.0, None), ("clamped_swish", 0.8, 1.7)])
+def test_when_the_shared_expert_goes_with_the_experts(monkeypatch, T, d, E, F, top, S, inside, gate, limit, shared_limit):
+    """The whole feed-forward with its shared expert's gate: which way it takes, its result, and no further from 64 bits than with the
+    shared expert in products of its own."""
+    from serve_amd import ops
+    from serve_amd.parts.base import Runtime
+    from serve_amd.registry import get_part
+    part = get_part("feed_forward", "routed_experts")(hidden_size=d, experts=E, top=top, expert_size=F, shared_size=S, activation=gate,
+                                                      limit=limit, shared_limit=shared_limit)
+    g = torch.Generator("cuda").manual_seed(T + d + S)
+    tensors = {r.name: (torch.randn(tuple(r.shape), device="cuda", generator=g) * r.shape[1] ** -0.5).bfloat16() for r in part.param_requests()}
+    part.load(tensors, Runtime(torch.device("cuda:0"), torch.bfloat16, max_context=64))
+    h = torch.randn((T, d), device="cuda", generator=g).bfloat16()
+    calls, experts = [], ops.moe_experts
+
+    def spy(h, ids, *args, **more):
+        out = experts(h, ids, *args, **more)
+        calls.append((more.get("shared"), ids, more.get("weights", args[5] if len(args) > 5 else None)))
+        return out
+    monkeypatch.setattr(ops, "moe_experts", spy)
+    y = part.forward(h, None)
+    shared, ids, weights = calls[0]
+    assert (shared is not None) == inside
+    w = {n: t.double() for n, t in tensors.items()}
+    x = h.double()
+    act = _gated(x @ w["shared.gate"].T, x @ w["shared.up"].T, gate, limit if shared_limit is None else shared_limit)
+    share = torch.sigmoid(x @ w["shared.sg"].T)
+    want, size = share * (act @ w["shared.down"].T), share * (act.abs() @ w["shared.down"].abs().T)
+    for e in range(E):
+        t, k = (ids == e).nonzero(as_tuple=True)
+        act = _gated(x[t] @ w[f"e{e}.gate"].T, x[t] @ w[f"e{e}.up"].T, gate, limit)
+        want.index_add_(0, t, weights[t, k].double()[:, None] * (act @ w[f"e{e}.down"].T))
+        size.index_add_(0, t, weights[t, k].double()[:, None] * (act.abs() @ w[f"e{e}.down"].abs().T))
+    off = (y.double() - want).abs()
+    # inside, the gated values are rounded to eight bits, by at most 2^-8 of each, and the rest is float32; in products of its own the
+    # shared expert's gates, ups and rows may be rounded too (0.003 of the result, and four times that)
+    if inside:
+        assert (off <= 1.1 * 2.0 ** -8 * size + 1e-5).all()
+    assert off.norm() <= 0.012 * want.norm()
+    monkeypatch.setattr(ops, "moe_shared_inside", lambda *a: False)
+    alone = part.forward(h, None)
+    if inside:
+        assert off.norm() <= 1.02 * (alone.double() - want).norm()
+    else:
+        assert torch.equal(alone, y)
+
+
 @pytest.mark.parametrize("gate,limit", [("silu", 0.0), ("clamped_swish", 0.8)])
 @pytest.mark.parametrize("T,d,F,E,top", [(700, 128, 192, 5, 2), (300, 64, 64, 9, 4), (2048, 256, 128, 6, 1)])
 def test_experts_of_many_rows_with_both_operands_through_lds(T, d, F, E, top, gate, limit):
