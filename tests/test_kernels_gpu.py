@@ -1064,6 +1064,15 @@ def test_prompt_attention_on_both_sides_of_the_largest_page_of_a_load(Hq, Hk, D,
     attention_case("bfloat16", Hq, Hk, D, ps, [(0, 200), (33, 65)], seed=573 + D, kernel="dispatch", poison=True)
 
 
+@pytest.mark.parametrize("Hq,Hk,D,ps", [(8, 2, 64, 8), (8, 2, 64, 32), (8, 2, 64, 64), (8, 2, 64, 128), (4, 1, 128, 8), (4, 1, 128, 32),
+                                        (4, 1, 128, 64)])
+def test_prompt_attention_of_few_rows_on_both_sides_of_the_largest_page_of_a_load(Hq, Hk, D, ps):
+    """The same for segments of at most 64 rows a key head, whose workgroups have four waves along the keys."""
+    attention_case("bfloat16", Hq, Hk, D, ps, [(0, 16), (100, 7), (255, 16), (511, 1), (1300, 13)], seed=574 + D, kernel="mfma", poison=True)
+    attention_case("bfloat16", Hq, Hk, D, ps, [(700, 16), (64, 5), (333, 11)], seed=575 + D, kernel="mfma", window=290, poison=True)
+    attention_case("bfloat16", Hq, Hk, D, ps, [(2000, 16), (900, 9)], seed=576 + D, kernel="mfma", splits=3, poison=True)
+
+
 @pytest.mark.parametrize("Hq,Hk,D,ps", [(8, 2, 64, 16), (4, 1, 128, 32), (3, 3, 80, 20)])
 def test_prompt_attention_long_prompts_windows_and_split_keys(Hq, Hk, D, ps):
     """Many row groups per segment (a workgroup takes group w and group last - w; an odd count leaves
