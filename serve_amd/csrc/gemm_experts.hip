@@ -214,11 +214,12 @@ __device__ __forceinline__ void expert_tile(const ExpertArgs& p, u32x4_t* lds, i
 }
 
 // The shared expert's part of a product, in the same launch: of all M rows, tiles of `rows` by 128 weight rows (SHARED_CT), which
-// fill what the experts leave of the chip.  Up to SHARED_AHEAD rows they stand before the experts' workgroups in the grid, whose
+// fill what the experts leave of the chip, and save two launches and a pass of the gate where they leave nothing.  Up to SHARED_AHEAD rows they stand before the experts' workgroups in the grid, whose
 // stream of weights then begins beside them; of more rows each takes so long that they come behind.  The whole feed-forward, us, the
 // shared expert as two products of its own / ahead / behind: 32 experts of 2,048 x 1,024 and a shared one of 2,048 at 129, 256, 400,
 // 512, 700, 1,000 and 2,048 tokens 127 / 116 / 132, 142 / 125 / 137, 139 / 125 / 140, 156 / 151 / 153, 168 / 159 / 159, 177 / 170 / 166,
-// 259 / 263 / 258; 8 of them and a shared one of 1,024 at 40, 128, 256 and 1,000 53 / 42 / 42, 64 / 52 / 51, 87 / 55 / 54, 122 / 95 / 95.
+// 259 / 263 / 258; 8 of them and a shared one of 1,024 at 40, 128, 256 and 1,000 53 / 42 / 42, 64 / 52 / 51, 87 / 55 / 54, 122 / 95 / 95.  (Its
+// rows in bf16 then; in fp32, as its own products leave them up to 128 rows, up to 1 us more, 2 at the last.)
 // What bounds them is the way into a compute unit (a tile reads 1 MB); tiles of 256 weight rows, or of 256 rows, leave half of the chip
 // idle: 198 and 228 us at 1,000 tokens.
 struct SharedArgs {
